@@ -104,6 +104,11 @@ int bcstruct_get_counts(const bc_struct *bc, int *num_ob_gz_pts, int *num_ib_gz_
                         int *nterms_total);
 int bcstruct_get_layer(const bc_struct *bc, int which_gz, outer_bc *outer_out, inner_bc *inner_out);
 int bcstruct_get_composed(const bc_struct *bc, int *gdest, int *rowptr, int *src, double *coeff, int *negmask);
+/* The ghost fill's rows (stage != 0: only the ghosts that the step's stencils read), 4 ints each:
+ * dest, base, code, negmask; rows that are not products of one-dimensional extrapolations have
+ * code 1 << 30, and their negmask entries start at base in coeff, src, negmask. NULL skips an output. */
+int bcstruct_get_fill(const bc_struct *bc, int stage, int *nrows, int *nterms, int *rows, double *coeff, int *src,
+                      int *negmask);
 
 /* Replaces apply_bcs_curvilinear() of apply_bcs_curvilinear.h:7-64: for every
  * gridfunction, layer by layer, quadratic extrapolation at outer points then

@@ -26,7 +26,7 @@ def batched_kernel(name, kid):
     """(kernel source, launcher source, range) for the batched variant of kernel ``name``."""
     spec = lp.BATCH_SPECS[name]
     o = lp.parse_loopopts(spec["loopopts"])
-    rng = "NRPY_RANGE_INTERIOR" if o["range"] == "interior" else "NRPY_RANGE_ALL"
+    rng = {"interior": "NRPY_RANGE_INTERIOR", "all": "NRPY_RANGE_ALL", "stage": "NRPY_RANGE_STAGE"}[o["range"]]
     kbody = lp.simple_loop(spec["loopopts"], spec["body"], batched=True)
     unpack = "".join("  const %s %s = params.%s;\n" % (lp._ctype(t), n, n) for n, t in lp._used_cparams(kbody))
     for n in ("Nxx0", "Nxx1", "Nxx2", "Nxx_plus_2NGHOSTS0", "Nxx_plus_2NGHOSTS1", "Nxx_plus_2NGHOSTS2"):

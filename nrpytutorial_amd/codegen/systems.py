@@ -49,21 +49,23 @@ BUNDLES = ("scalarwave_cartesian", "bssn_cartesian", "bssn_spherical_sym2", "max
     tuple(CURVI_SCALARWAVE) + ("bssn_etk",) + tuple(CURVI_MAXWELL)
 
 
-def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args):
+def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
     """MoL_step_forward_in_time + hipGraph replay for the diagonal RK4 schedule."""
     ricci = ("  if ((rc = Ricci_eval(rfmstruct, params, IN, auxevol_gfs, stream))) return rc;\n" if has_ricci else "")
-    detg = ("  if ((rc = enforce_detgammabar_constraint(rfmstruct, params, OUT, stream))) return rc;\n"
+    detg = ("  if ((rc = DETG(rfmstruct, params, OUT, stream))) return rc;\n"
             if has_detg else "")
     sub = ("  /* substep S: IN -> OUT */\n" + ricci +
            "  if ((rc = rhs_eval_rk4_substep(S, " + rhs_call_args + ", y_n_gfs, y_nplus1_running_total_gfs, OUT, dt, "
            "stream))) return rc;\n"
-           "  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, OUT, stream))) "
-           "return rc;\n" + detg)
+           "  if ((rc = FILL(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, OUT, stream))) return rc;\n" + detg)
     steps = ""
+    # The stage states (substeps 0-2) are read by the next right-hand side only: they get the
+    # ghosts its stencils reach. The new state gets every ghost.
     for s, (i, o) in enumerate((("y_n_gfs", "k_odd_gfs"), ("k_odd_gfs", "k_even_gfs"),
                                 ("k_even_gfs", "k_odd_gfs"), ("k_odd_gfs", "y_n_gfs"))):
         steps += sub.replace("IN", i).replace("OUT", o).replace("substep S", "substep %d" % s) \
-            .replace("(S,", "(%d," % s)
+            .replace("(S,", "(%d," % s).replace("FILL", "nrpy_stage_fill" if s < 3 else "apply_bcs_curvilinear_composed") \
+            .replace("DETG", "enforce_detgammabar_constraint" + (detg_stage if s < 3 else ""))
     sig = ("const rfm_struct *rfmstruct, const paramstruct *params, const bc_struct *bcstruct, double *y_n_gfs, "
            "double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, double *auxevol_gfs, "
            "const double dt")
@@ -193,7 +195,7 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
             meta)
 
 
-def _mol_batch_glue(n_ricci, n_rhs):
+def _mol_batch_glue(n_ricci, n_rhs, detg_stage):
     """MoL_batch_step / MoL_batch_graph_create: one RK4 step of every instance of a batch,
     the diagonal schedule with one launch per kernel per substep for all instances."""
     sub = ""
@@ -208,8 +210,10 @@ def _mol_batch_glue(n_ricci, n_rhs):
         for k in range(n_rhs):
             sub += ("  if ((rc = rhs_eval_rk4_substep_g%d_batched(%d, b, NRPY_BATCH_ROLE_AUXEVOL, %s, NRPY_BATCH_ROLE_YN, "
                     "NRPY_BATCH_ROLE_RT, %s, stream))) return rc;\n" % (k, s, i, o))
-        sub += ("  if ((rc = nrpy_batch_apply_bcs(b, %s, NUM_EVOL_GFS, evol_gf_parity, stream))) return rc;\n"
-                "  if ((rc = enforce_detgammabar_constraint_batched(b, %s, stream))) return rc;\n" % (o, o))
+        # ghosts as in MoL_step_forward_in_time: a stage gets those its stencils reach
+        sub += ("  if ((rc = nrpy_batch_fill(b, %s, %s, NUM_EVOL_GFS, evol_gf_parity, stream))) return rc;\n"
+                "  if ((rc = enforce_detgammabar_constraint%s_batched(b, %s, stream))) return rc;\n"
+                % ("&b->fill_stage" if s < 3 else "&b->fill_all", o, detg_stage if s < 3 else "", o))
     return (
         "// One RK4 step of every instance of the batch (their own dt), as MoL_step_forward_in_time does\n"
         "// for one grid.\n"
@@ -256,22 +260,19 @@ def _mol_adjoint_glue(has_rfm_vjp, state_dependent, writes_all):
     vjp = (("" if writes_all else "  if ((rc = nrpy_fill(n, w, 0.0, stream))) return rc;\n") +
            "  if ((rc = rhs_eval_vjp(" + rfm_arg + "params, auxevol_gfs, STATE, kbar, vjp_G, w, nullptr, stream))) "
            "return rc;\n"
-           "  if ((rc = bc_apply_T(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, w, stream))) return rc;\n")
+           "  if ((rc = nrpy_stage_apply_T(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, w, stream))) return rc;\n")
     if state_dependent:
         recompute = (
             "  double *yn = (double *)y_n_gfs;  // substeps 0-2 read y_n only\n"
             "  if ((rc = rhs_eval_rk4_substep(0, rfmstruct, params, auxevol_gfs, yn, yn, rt, U1, dt, stream))) "
             "return rc;\n"
-            "  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U1, stream))) "
-            "return rc;\n"
+            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U1, stream))) return rc;\n"
             "  if ((rc = rhs_eval_rk4_substep(1, rfmstruct, params, auxevol_gfs, U1, yn, rt, U2, dt, stream))) "
             "return rc;\n"
-            "  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U2, stream))) "
-            "return rc;\n"
+            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U2, stream))) return rc;\n"
             "  if ((rc = rhs_eval_rk4_substep(2, rfmstruct, params, auxevol_gfs, U2, yn, rt, U3, dt, stream))) "
             "return rc;\n"
-            "  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U3, stream))) "
-            "return rc;\n")
+            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U3, stream))) return rc;\n")
         states = ("U3", "U2", "U1", "y_n_gfs")
     else:
         recompute = "  (void)U1; (void)U2; (void)U3; (void)rt;  // linear right-hand side: the adjoint ignores the state\n"
@@ -464,13 +465,32 @@ def ricci_groups(names):
     return groups
 
 
-def _header(NGHOSTS):
+_OFFSET = re.compile(r"\[IDX4\(\w+GF, i0([+-]\d+)?,i1([+-]\d+)?,i2([+-]\d+)?\)\]")
+
+
+def stage_offsets(bodies):
+    """The point offsets that the stencils of the step kernels' bodies read, other than (0, 0, 0)."""
+    found = {tuple(int(v or 0) for v in m) for b in bodies for m in _OFFSET.findall(b)}
+    return sorted(found - {(0, 0, 0)}) or [(0, 0, 0)]
+
+
+def stage_axes(offsets):
+    """Per axis, whether a stencil reads neighbours along it."""
+    return [any(o[d] for o in offsets) for d in range(3)]
+
+
+def _header(NGHOSTS, offsets):
     ps, members = bd.paramstruct_decl()
     defines, lists = bd.gf_defines_and_meta()
     parity = [bd.parity_type(n) for n in lists["evol"]]
     pre = ('#include "../nrpy_runtime_pre.h"\n#define NGHOSTS %d\n' % NGHOSTS + defines + "\n" + ps + "\n"
            + "static const int8_t evol_gf_parity[%d] = {%s};\n" % (max(1, len(parity)),
                                                                    ", ".join(str(p) for p in parity) or "0")
+           + "// point offsets read by the stencils of the RK4 step's kernels\n"
+           + "static const int8_t nrpy_stage_offsets[%d][3] = {%s};\n"
+           % (len(offsets), ", ".join("{%d, %d, %d}" % o for o in offsets))
+           + "".join("#define NRPY_STAGE_LO%d %s\n" % (d, "0" if a else "NGHOSTS")
+                     for d, a in enumerate(stage_axes(offsets)))
            + bd.check_params_code())
     meta = {"NGHOSTS": NGHOSTS, "paramstruct": members, "gfs": lists, "evol_parity": parity,
             "aux_parity": [bd.parity_type(n) for n in lists["aux"]],
@@ -513,7 +533,7 @@ def scalarwave_cartesian():
     vjp_src, slots, vouts, vdep = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
     som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
                                          shell_call=SHELL_CALL)
-    pre, meta = _header(3)
+    pre, meta = _header(3, stage_offsets([body]))
     parts = [pre, bd.coord_host_functions("Cartesian"), '#include "../nrpy_runtime.h"', bd.rfm_struct_code(),
              rhs_src, fused, id_src, vjp_src,
              _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"),
@@ -567,7 +587,7 @@ def maxwell_cartesian():
     # the Start-to-Finish Maxwell run's choice: second-order radial derivative, falloff power 3
     som_src, som_meta = _sommerfeld_glue(2, "rhs_eval(params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
                                          shell_call=SHELL_CALL)
-    pre, meta = _header(3)
+    pre, meta = _header(3, stage_offsets([body]))
     vjp_src, slots, vouts, vdep = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
     parts = [pre, coords, '#include "../nrpy_runtime.h"', bd.rfm_struct_code(), rhs_src, con_src, fused, id_src,
              vjp_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"),
@@ -621,7 +641,7 @@ def scalarwave_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
     # the coordinate functions are generated before the paramstruct is declared.
     coords = bd.coord_host_functions(CoordSystem)
     som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)")
-    pre, meta = _header(NGHOSTS)
+    pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code,
              rhs_src, fused, id_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]
     meta["sommerfeld"] = som_meta
@@ -687,7 +707,7 @@ def maxwell_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
     id_src = _initial_data_kernel(id_rhss, id_names)
     coords = bd.coord_host_functions(CoordSystem)
     som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)")
-    pre, meta = _header(NGHOSTS)
+    pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code, rhs_src, con_src, fused, id_src,
              _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]
     meta["sommerfeld"] = som_meta
@@ -775,6 +795,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     args_decl = ("const paramstruct params, const rfm_struct rfmstruct, const double *__restrict__ auxevol_gfs, "
                  "const double *__restrict__ in_gfs")
     rhs_src, fused, group_costs, group_inputs = "", "", [], []
+    step_bodies = []
     # Large Cartesian grids: the RHS, Ricci and Hamiltonian kernels read their
     # mixed-derivative stencils from LDS tiles (codegen/lds.py). The small
     # curvilinear grids of the Brill-Lindquist runs (two points in phi) keep the
@@ -801,6 +822,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
         sel = [e for (n, _), e in zip(pairs, evol_rhss) if n in grp]
         body = fin.FD_outputC("returnstring", sel, params="outCverbose=False", upwindcontrolvec=betaU)
         group_costs.append(bd.count_body(body))
+        step_bodies.append(body)
         rhs_src += oc.outCfunction(outfile="returnstring", desc="BSSN RHSs of %s" % ", ".join(grp),
                                    name="rhs_eval_g%d" % k, params=rhs_params, body=body,
                                    loopopts="InteriorPoints,Enable_rfm_precompute")
@@ -835,6 +857,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
         body_k = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
                                                  for n in grp], params="outCverbose=False")
         ricci_costs.append(bd.count_body(body_k))
+        step_bodies.append(body_k)
         ricci_src += oc.outCfunction(outfile="returnstring", desc="Evaluate the Ricci tensor components %s"
                                      % ", ".join(grp), name="Ricci_eval_g%d" % k, params=ricci_params, body=body_k,
                                      loopopts="InteriorPoints,Enable_rfm_precompute")
@@ -870,6 +893,16 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                                params="const rfm_struct *restrict rfmstruct,const paramstruct *restrict params, "
                                       "REAL *restrict in_gfs",
                                body=detg_body, loopopts="AllPoints,Enable_rfm_precompute")
+    # The stage states need the enforcement only where a stencil reads: without the ghost planes
+    # of an axis along which there is none (i2 in the axisymmetric bundles).
+    offsets = stage_offsets(step_bodies)
+    detg_stage = "" if all(stage_axes(offsets)) else "_stage"
+    if detg_stage:
+        detg_src += oc.outCfunction(outfile="returnstring", desc="The same at the points a stage's stencils read.",
+                                    name="enforce_detgammabar_constraint_stage",
+                                    params="const rfm_struct *restrict rfmstruct,const paramstruct *restrict params, "
+                                           "REAL *restrict in_gfs",
+                                    body=detg_body, loopopts="StagePoints,Enable_rfm_precompute")
     # Precompute tables depend on which functions remain; build the struct now.
     rfm_code = bd.rfm_struct_code()
     tables = [(n, str(e), list(a)) for n, e, a in rfm.rfm_precompute_tables()]
@@ -921,15 +954,16 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     print("(BENCH) VJP codegen %.1fs (%d + %d + %d + %d slots)" % (time.time() - t0, len(vslots), len(rslots),
                                                                   len(dslots), len(hslots)), flush=True)
     batch_names = (["Ricci_eval_g%d" % k for k in range(len(ric_groups))] +
-                   ["rhs_eval_rk4_substep_g%d" % k for k in range(len(groups))] + ["enforce_detgammabar_constraint"])
+                   ["rhs_eval_rk4_substep_g%d" % k for k in range(len(groups))] + ["enforce_detgammabar_constraint"] +
+                   (["enforce_detgammabar_constraint_stage"] if detg_stage else []))
     batch_src, batch_table = bt.batched_kernels(batch_names)
-    pre, meta = _header(FD_order // 2 + 1)
+    pre, meta = _header(FD_order // 2 + 1, offsets)
     parts = [pre, bd.coord_host_functions(CoordSystem), '#include "../nrpy_runtime.h"', rfm_code,
              ricci_src, rhs_src, fused, h_src, mu_src, detg_src, id_src, id_dmass_src, vjp_src, rvjp_src, dvjp_src,
              hvjp_src,
-             _mol_glue(True, True, None, "rfmstruct, params, auxevol_gfs, IN"),
+             _mol_glue(True, True, None, "rfmstruct, params, auxevol_gfs, IN", detg_stage),
              bt.instance_struct(), batch_table, '#include "../nrpy_batch.h"', batch_src,
-             _mol_batch_glue(len(ric_groups), len(groups))]
+             _mol_batch_glue(len(ric_groups), len(groups), detg_stage)]
     meta["rhs_groups"] = groups
     # distinct gridfunctions each group's kernel reads (evolved and RbarDD): its algorithmic
     # traffic is 8 (inputs + 4 outputs) bytes per point

@@ -39,6 +39,11 @@ typedef struct __paramstruct__ {
 } paramstruct;
 
 static const int8_t evol_gf_parity[2] = {0, 0};
+// point offsets read by the stencils of the RK4 step's kernels
+static const int8_t nrpy_stage_offsets[12][3] = {{-2, 0, 0}, {-1, 0, 0}, {0, -2, 0}, {0, -1, 0}, {0, 0, -2}, {0, 0, -1}, {0, 0, 1}, {0, 0, 2}, {0, 1, 0}, {0, 2, 0}, {1, 0, 0}, {2, 0, 0}};
+#define NRPY_STAGE_LO0 0
+#define NRPY_STAGE_LO1 0
+#define NRPY_STAGE_LO2 0
 static int nrpy_check_params(const paramstruct *p) {
   if (p->Nxx0 < 1 || p->Nxx1 < 1 || p->Nxx2 < 1) return 1;
   if (p->Nxx_plus_2NGHOSTS0 != p->Nxx0 + 2*NGHOSTS || p->Nxx_plus_2NGHOSTS1 != p->Nxx1 + 2*NGHOSTS ||
@@ -502,13 +507,13 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
   int rc;
   /* substep 0: y_n_gfs -> k_odd_gfs */
   if ((rc = rhs_eval_rk4_substep(0, rfmstruct, params, auxevol_gfs, y_n_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
+  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
   /* substep 1: k_odd_gfs -> k_even_gfs */
   if ((rc = rhs_eval_rk4_substep(1, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
-  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_even_gfs, stream))) return rc;
+  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_even_gfs, stream))) return rc;
   /* substep 2: k_even_gfs -> k_odd_gfs */
   if ((rc = rhs_eval_rk4_substep(2, rfmstruct, params, auxevol_gfs, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
+  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
   /* substep 3: k_odd_gfs -> y_n_gfs */
   if ((rc = rhs_eval_rk4_substep(3, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
   if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, stream))) return rc;

@@ -38,6 +38,36 @@
     nrpy_bz = t_ / (nbx_ * nby_);                                                              \
   }
 
+// Fill rows of many instances: row r belongs to instance h_inst[r] (a generic row's base
+// counts from the start of the concatenated terms).
+struct nrpy_batch_fill_list {
+  int n = 0;
+  std::vector<nrpy_fill_row> h_rows;
+  std::vector<nrpy_fill_term> h_terms;
+  std::vector<int> h_inst;
+  nrpy_fill_row *d_rows = nullptr;
+  nrpy_fill_term *d_terms = nullptr;
+  int *d_inst = nullptr;
+  void append(const nrpy_fill_list &L, const int k) {
+    for (nrpy_fill_row R : L.h_rows) {
+      if (R.code == NRPY_FILL_GENERIC) R.base += (int)h_terms.size();
+      h_rows.push_back(R);
+      h_inst.push_back(k);
+    }
+    h_terms.insert(h_terms.end(), L.h_terms.begin(), L.h_terms.end());
+    n = (int)h_rows.size();
+  }
+  bool upload() {
+    return nrpy_upload(&d_rows, h_rows.data(), h_rows.size()) && nrpy_upload(&d_terms, h_terms.data(), h_terms.size()) &&
+           nrpy_upload(&d_inst, h_inst.data(), h_inst.size());
+  }
+  void free_device() {
+    (void)hipFree(d_rows);
+    (void)hipFree(d_terms);
+    (void)hipFree(d_inst);
+  }
+};
+
 struct nrpy_batch {
   int ninst = 0;
   std::vector<nrpy_batch_instance> h_inst;
@@ -45,17 +75,18 @@ struct nrpy_batch {
   // prefix tables: key (bx, by, bz, range) -> device array of ninst + 1 tile offsets
   std::map<std::vector<int>, int *> prefix;
   std::map<std::vector<int>, int> ntiles;
-  // concatenated composed ghost maps: row r belongs to instance row_inst[r]
-  int nrows = 0;
-  int *d_row_inst = nullptr, *d_row_dest = nullptr, *d_rowptr = nullptr, *d_src = nullptr, *d_negmask = nullptr;
-  double *d_coeff = nullptr;
+  // the instances' fill lists one after another, every ghost and those a stage's stencils reach
+  nrpy_batch_fill_list fill_all, fill_stage;
 };
 
 static void nrpy_batch_range(const nrpy_batch_instance &I, int range, int n[3]) {
   if (range == NRPY_RANGE_INTERIOR) {
     n[0] = I.params.Nxx0; n[1] = I.params.Nxx1; n[2] = I.params.Nxx2;
   } else {
-    n[0] = I.params.Nxx_plus_2NGHOSTS0; n[1] = I.params.Nxx_plus_2NGHOSTS1; n[2] = I.params.Nxx_plus_2NGHOSTS2;
+    const int s = range == NRPY_RANGE_STAGE ? 2 : 0;
+    n[0] = I.params.Nxx_plus_2NGHOSTS0 - s * NRPY_STAGE_LO0;
+    n[1] = I.params.Nxx_plus_2NGHOSTS1 - s * NRPY_STAGE_LO1;
+    n[2] = I.params.Nxx_plus_2NGHOSTS2 - s * NRPY_STAGE_LO2;
   }
 }
 
@@ -90,12 +121,8 @@ extern "C" void nrpy_batch_free(nrpy_batch *b) {
   if (!b) return;
   (void)hipFree(b->d_inst);
   for (auto &kv : b->prefix) (void)hipFree(kv.second);
-  (void)hipFree(b->d_row_inst);
-  (void)hipFree(b->d_row_dest);
-  (void)hipFree(b->d_rowptr);
-  (void)hipFree(b->d_src);
-  (void)hipFree(b->d_negmask);
-  (void)hipFree(b->d_coeff);
+  b->fill_all.free_device();
+  b->fill_stage.free_device();
   delete b;
 }
 
@@ -125,8 +152,6 @@ extern "C" int nrpy_batch_create(const int ninst, const paramstruct *params, con
   nrpy_batch *b = new nrpy_batch();
   b->ninst = ninst;
   b->h_inst.resize(ninst);
-  std::vector<int> row_inst, row_dest, rowptr(1, 0), src, negmask;
-  std::vector<double> coeff;
   for (int k = 0; k < ninst; k++) {
     if (!rfms[k] || !bcs[k] || nrpy_check_params(&params[k])) {
       nrpy_batch_free(b);
@@ -150,25 +175,11 @@ extern "C" int nrpy_batch_create(const int ninst, const paramstruct *params, con
       }
     I.dt = dts[k];
     I.Ntot = (long)bc->N[0] * bc->N[1] * bc->N[2];
-    for (int r = 0; r < bc->nghost; r++) {
-      row_inst.push_back(k);
-      row_dest.push_back(bc->h_gdest[r]);
-      for (int t = bc->h_rowptr[r]; t < bc->h_rowptr[r + 1]; t++) {
-        src.push_back(bc->h_src[t]);
-        coeff.push_back(bc->h_coeff[t]);
-        negmask.push_back(bc->h_negmask[t]);
-      }
-      rowptr.push_back((int)src.size());
-    }
+    b->fill_all.append(bc->fill_all, k);
+    b->fill_stage.append(bc->fill_stage, k);
   }
-  b->nrows = (int)row_inst.size();
-  bool ok = nrpy_upload(&b->d_inst, b->h_inst.data(), b->h_inst.size()) &&
-            nrpy_upload(&b->d_row_inst, row_inst.data(), row_inst.size()) &&
-            nrpy_upload(&b->d_row_dest, row_dest.data(), row_dest.size()) &&
-            nrpy_upload(&b->d_rowptr, rowptr.data(), rowptr.size()) &&
-            nrpy_upload(&b->d_src, src.data(), src.size()) &&
-            nrpy_upload(&b->d_coeff, coeff.data(), coeff.size()) &&
-            nrpy_upload(&b->d_negmask, negmask.data(), negmask.size());
+  const bool ok = nrpy_upload(&b->d_inst, b->h_inst.data(), b->h_inst.size()) && b->fill_all.upload() &&
+                  b->fill_stage.upload();
   if (!ok) {
     nrpy_batch_free(b);
     return NRPY_ERR_ALLOC;
@@ -182,52 +193,29 @@ extern "C" int nrpy_batch_create(const int ninst, const paramstruct *params, con
   return NRPY_OK;
 }
 
-// Composed ghost fill of the array in role 'role' of every instance, one launch. One thread
-// per ghost row fills NRPY_BATCH_BC_CHUNK gridfunctions per pass over the row's terms: the
-// concatenated maps of a sweep (~100 MB for 256 Brill-Lindquist instances) are then read
-// ceil(num_gfs / NRPY_BATCH_BC_CHUNK) times instead of once per gridfunction. Each
-// gridfunction's sum runs over the same terms in the same order as one thread per
-// (row, gridfunction) would, so the values are identical.
-#define NRPY_BATCH_BC_CHUNK 8
-__global__ void nrpy_batch_bc_kernel(int nrows, const nrpy_batch_instance *__restrict__ inst,
-                                     const int *__restrict__ row_inst, const int *__restrict__ row_dest,
-                                     const int *__restrict__ rowptr, const int *__restrict__ src,
-                                     const double *__restrict__ coeff, const int *__restrict__ negmask, int role,
-                                     int num_gfs, nrpy_gf_parity_args gfp) {
-  const int r = (int)((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+// Ghost fill of the array in role 'role' of every instance, one launch, from the list of every
+// ghost or of those a stage's stencils reach. A thread fills NRPY_BATCH_FILL_K gridfunctions of
+// one row, with the code of the single-grid fill, so the values are the same bits.
+#define NRPY_BATCH_FILL_K 8
+__global__ void __launch_bounds__(256)
+nrpy_batch_fill_kernel(const int nrows, const nrpy_batch_instance *__restrict__ inst,
+                       const int *__restrict__ row_inst, const nrpy_fill_row *__restrict__ rows,
+                       const nrpy_fill_term *__restrict__ terms, const int role, const int num_gfs,
+                       const nrpy_gf_parity_args gfp) {
+  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (r >= nrows) return;
-  const int k = row_inst[r];
-  double *base = inst[k].arr[role];
-  const size_t Ntot = inst[k].Ntot;
-  const int q0 = rowptr[r], q1 = rowptr[r + 1], dest = row_dest[r];
-  for (int gf0 = 0; gf0 < num_gfs; gf0 += NRPY_BATCH_BC_CHUNK) {
-    double acc[NRPY_BATCH_BC_CHUNK];
-#pragma unroll
-    for (int j = 0; j < NRPY_BATCH_BC_CHUNK; j++) acc[j] = 0.0;
-    for (int q = q0; q < q1; q++) {
-      const int s = src[q];
-      const double c = coeff[q];
-      const int m = negmask[q];
-#pragma unroll
-      for (int j = 0; j < NRPY_BATCH_BC_CHUNK; j++) {
-        const int gf = gf0 + j;
-        if (gf < num_gfs) {
-          const double cj = (m & (1 << gfp.p[gf])) ? -c : c;
-          acc[j] += cj * base[(size_t)gf * Ntot + s];
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NRPY_BATCH_BC_CHUNK; j++)
-      if (gf0 + j < num_gfs) base[(size_t)(gf0 + j) * Ntot + dest] = acc[j];
-  }
+  const nrpy_fill_row R = rows[r];
+  const nrpy_batch_instance *I = inst + row_inst[r];
+  const int N0 = I->params.Nxx_plus_2NGHOSTS0, N01 = N0 * I->params.Nxx_plus_2NGHOSTS1;
+  nrpy_fill_point<NRPY_BATCH_FILL_K>(R, terms, N0, N01, (size_t)I->Ntot, NRPY_BATCH_FILL_K * (int)blockIdx.y, num_gfs,
+                                     gfp, I->arr[role]);
 }
 
-extern "C" int nrpy_batch_apply_bcs(const nrpy_batch *b, const int role, const int NUM_GFS, const int8_t *gfs_parity,
-                                    hipStream_t stream) {
+static int nrpy_batch_fill(const nrpy_batch *b, const nrpy_batch_fill_list *L, const int role, const int NUM_GFS,
+                           const int8_t *gfs_parity, hipStream_t stream) {
   if (!b || !gfs_parity) return NRPY_ERR_NULL;
   if (role < 0 || role >= NRPY_BATCH_ROLES || NUM_GFS < 1 || NUM_GFS > 64) return NRPY_ERR_PARAM;
-  if (b->nrows == 0) return NRPY_OK;
+  if (L->n == 0) return NRPY_OK;
   nrpy_gf_parity_args gfp;
   memset(&gfp, 0, sizeof(gfp));
   for (int g = 0; g < NUM_GFS; g++) {
@@ -235,9 +223,15 @@ extern "C" int nrpy_batch_apply_bcs(const nrpy_batch *b, const int role, const i
     gfp.p[g] = gfs_parity[g];
   }
   const int B = 256;
-  const size_t work = (size_t)b->nrows;
-  hipLaunchKernelGGL(nrpy_batch_bc_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream, b->nrows,
-                     b->d_inst, b->d_row_inst, b->d_row_dest, b->d_rowptr, b->d_src, b->d_coeff, b->d_negmask, role,
-                     NUM_GFS, gfp);
+  hipLaunchKernelGGL(nrpy_batch_fill_kernel,
+                     dim3((unsigned)((L->n + B - 1) / B), (NUM_GFS + NRPY_BATCH_FILL_K - 1) / NRPY_BATCH_FILL_K), dim3(B),
+                     0, stream, L->n, b->d_inst, L->d_inst, L->d_rows, L->d_terms, role, NUM_GFS, gfp);
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+
+// Every ghost point of the array in role 'role' of every instance, one launch.
+extern "C" int nrpy_batch_apply_bcs(const nrpy_batch *b, const int role, const int NUM_GFS, const int8_t *gfs_parity,
+                                    hipStream_t stream) {
+  if (!b) return NRPY_ERR_NULL;
+  return nrpy_batch_fill(b, &b->fill_all, role, NUM_GFS, gfs_parity, stream);
 }

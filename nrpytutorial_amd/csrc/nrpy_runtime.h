@@ -21,7 +21,8 @@
 //     the host; apply_bcs_curvilinear_composed then fills every ghost of every
 //     gridfunction in a single launch that reads only interior points. The RK
 //     substep kernels write interior points only, so this fill runs right
-//     after them with no ordering between ghost points.
+//     after them with no ordering between ghost points. A stage of the RK4 step
+//     needs only the ghosts that the bundle's stencils reach (nrpy_stage_fill).
 //  4. Deterministic sum-of-squares reduction over interior points.
 //  5. RK4 update macro used by the fused RHS + method-of-lines kernels.
 #pragma once
@@ -55,6 +56,41 @@ static const int8_t MAXFACE = -1;
 static const int8_t NUL = +0;
 static const int8_t MINFACE = +1;
 
+// One ghost point of the composed map in the form the fill kernel reads (16 bytes). Almost
+// every row is a product of one-dimensional quadratic extrapolations (or a parity copy of
+// such a point, or of an interior point): its value is
+//   sign * sum_{c,b,a} w_c w_b w_a f[base + a s0 + b s1 + c s2],
+// where along axis d the factor is one term (no extrapolation) or three, w the weights of
+// layer l = 1, 2, 3 outside the interior and s_d the index stride inwards. code holds 3 bits per
+// axis: 0, the layer (1..3) outside the low edge, or 3 + the layer outside the high edge; sign
+// is negative where negmask has the gridfunction's parity bit. Rows of any other form have
+// code NRPY_FILL_GENERIC, base = their first entry in the list's terms and negmask = the number
+// of entries.
+struct nrpy_fill_row {
+  int dest, base, code, negmask;
+};
+struct nrpy_fill_term {
+  double coeff;
+  int src, negmask;
+};
+#define NRPY_FILL_GENERIC (1 << 30)
+// Rows sorted by the number of extrapolated axes (0 or 1, then 2, 3, then generic ones).
+struct nrpy_fill_list {
+  int n = 0;
+  std::vector<nrpy_fill_row> h_rows;
+  std::vector<nrpy_fill_term> h_terms;
+  nrpy_fill_row *d_rows = nullptr;
+  nrpy_fill_term *d_terms = nullptr;
+};
+// Transpose of a set of ghost rows (CSR over the interior points they read).
+struct nrpy_transpose_list {
+  int n = 0;
+  std::vector<int> h_src, h_rowptr, h_ghost, h_negmask;
+  std::vector<double> h_coeff;
+  int *d_src = nullptr, *d_rowptr = nullptr, *d_ghost = nullptr, *d_negmask = nullptr;
+  double *d_coeff = nullptr;
+};
+
 // Device + host boundary-condition descriptor (opaque to callers).
 struct bc_struct {
   int N[3];                        // Nxx_plus_2NGHOSTS of the grid it was built for
@@ -77,24 +113,16 @@ struct bc_struct {
   int *d_ob_xedge_dest = nullptr;
   int8_t *d_ob_xedge_face = nullptr;
   int ob_xedge_off[NGHOSTS + 1];
-  // composed ghost map (CSR over ghost points)
+  // composed ghost map (CSR over ghost points); negmask bit t set: parity type t contributes
+  // with a minus sign
   int nghost = 0, nterms = 0;
   int *d_gdest = nullptr;
-  int *d_rowptr = nullptr;
-  int *d_src = nullptr;
-  double *d_coeff = nullptr;
-  int *d_negmask = nullptr;        // bit t set: parity type t contributes with a minus sign
   std::vector<int> h_gdest, h_rowptr, h_src, h_negmask;
   std::vector<double> h_coeff;
-  // transpose of the composed map (CSR over interior source points), for bc_apply_T
-  int ntsrc = 0;
-  int *d_tsrc = nullptr;
-  int *d_trowptr = nullptr;
-  int *d_tghost = nullptr;
-  double *d_tcoeff = nullptr;
-  int *d_tnegmask = nullptr;
-  std::vector<int> h_tsrc, h_trowptr, h_tghost, h_tnegmask;
-  std::vector<double> h_tcoeff;
+  // the map as the fill kernel reads it: every ghost point, and those a stencil reaches
+  nrpy_fill_list fill_all, fill_stage;
+  // its transpose, for bc_apply_T, and that of the reached ghosts, for the step adjoint
+  nrpy_transpose_list trans_all, trans_stage;
   // right-hand-side scratch of the fused Sommerfeld RK4 step (nrpy_sommerfeld_scratch)
   double *d_som_rhs = nullptr;
   size_t som_rhs_n = 0;
@@ -227,6 +255,124 @@ struct nrpy_term {
   double coeff;
 };
 
+// Whether a stencil of the bundle, centred at some interior point, reads ghost point idx.
+// nrpy_stage_offsets lists the offsets its step kernels read; the test takes the point's
+// distance outside the interior along each axis and asks for an offset that reaches at least
+// that far on each of them, whatever it does along the axes where the point is inside.
+static bool nrpy_stage_reads(const paramstruct *params, int idx) {
+  const int N0 = params->Nxx_plus_2NGHOSTS0, N1 = params->Nxx_plus_2NGHOSTS1, N2 = params->Nxx_plus_2NGHOSTS2;
+  const int N[3] = {N0, N1, N2}, i[3] = {idx % N0, (idx / N0) % N1, idx / (N0 * N1)};
+  int out[3];
+  for (int d = 0; d < 3; d++)
+    out[d] = i[d] < NGHOSTS ? i[d] - NGHOSTS : i[d] >= N[d] - NGHOSTS ? i[d] - (N[d] - NGHOSTS - 1) : 0;
+  const int n = (int)(sizeof(nrpy_stage_offsets) / sizeof(nrpy_stage_offsets[0]));
+  for (int k = 0; k < n; k++) {
+    bool reaches = true;
+    for (int d = 0; d < 3; d++) {
+      const int o = nrpy_stage_offsets[k][d];
+      if (out[d] < 0) reaches = reaches && o <= out[d];
+      if (out[d] > 0) reaches = reaches && o >= out[d];
+    }
+    if (reaches) return true;
+  }
+  return false;
+}
+
+static void nrpy_build_transpose(const bc_struct *bc, const int Ntot, const std::vector<char> &take,
+                                 nrpy_transpose_list *T) {
+  // counting sort of the entries by the interior point they read
+  std::vector<int> first(Ntot + 1, 0);
+  for (int r = 0; r < bc->nghost; r++)
+    if (take[r])
+      for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) first[bc->h_src[k] + 1]++;
+  T->h_rowptr.assign(1, 0);
+  for (int i = 0; i < Ntot; i++) {
+    if (first[i + 1]) {
+      T->h_src.push_back(i);
+      T->h_rowptr.push_back(first[i] + first[i + 1]);
+    }
+    first[i + 1] += first[i];
+  }
+  const size_t n = (size_t)first[Ntot];
+  T->h_ghost.resize(n);
+  T->h_coeff.resize(n);
+  T->h_negmask.resize(n);
+  for (int r = 0; r < bc->nghost; r++)
+    if (take[r])
+      for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) {
+        const int at = first[bc->h_src[k]]++;
+        T->h_ghost[at] = bc->h_gdest[r];
+        T->h_coeff[at] = bc->h_coeff[k];
+        T->h_negmask[at] = bc->h_negmask[k];
+      }
+  T->n = (int)T->h_src.size();
+}
+
+// Weights of the quadratic extrapolation to layer l outside the interior, from the three
+// points next to the edge (l = 1: 3, -3, 1).
+__host__ __device__ static inline double nrpy_extrap_weight(const int l, const int a) {
+  return a == 0 ? 0.5 * (l + 1) * (l + 2) : a == 1 ? -(double)l * (l + 2) : 0.5 * l * (l + 1);
+}
+
+// The rows of ``take`` in the fill kernel's form. anchor[r]: the point row r copies (its own
+// point if it is an extrapolated one, else the point its parity copy reads). The product form
+// built from the anchor is used only if it is the composed row, entry by entry.
+static void nrpy_build_fill(const paramstruct *params, const bc_struct *bc, const std::vector<int> &anchor,
+                            const std::vector<char> &take, nrpy_fill_list *L) {
+  const int N0 = params->Nxx_plus_2NGHOSTS0, N1 = params->Nxx_plus_2NGHOSTS1, N2 = params->Nxx_plus_2NGHOSTS2;
+  const int N[3] = {N0, N1, N2}, stride[3] = {1, N0, N0 * N1};
+  std::vector<nrpy_fill_row> kind[4];
+  for (int r = 0; r < bc->nghost; r++) {
+    if (!take[r]) continue;
+    const int b = bc->h_rowptr[r], n = bc->h_rowptr[r + 1] - b;
+    const int i[3] = {anchor[r] % N0, (anchor[r] / N0) % N1, anchor[r] / (N0 * N1)};
+    int base = 0, code = 0, axes = 0, layer[3], s[3];
+    bool product = n > 0;
+    for (int d = 0; d < 3; d++) {
+      layer[d] = 0;
+      s[d] = stride[d];
+      int at = i[d];
+      if (i[d] < NGHOSTS) {
+        layer[d] = NGHOSTS - i[d];
+        at = NGHOSTS;
+        code |= layer[d] << (3 * d);
+      } else if (i[d] >= N[d] - NGHOSTS) {
+        layer[d] = i[d] - (N[d] - NGHOSTS - 1);
+        at = N[d] - NGHOSTS - 1;
+        s[d] = -stride[d];
+        code |= (3 + layer[d]) << (3 * d);
+      }
+      axes += layer[d] > 0;
+      product = product && layer[d] <= 3;
+      base += at * stride[d];
+    }
+    product = product && n == (axes == 0 ? 1 : axes == 1 ? 3 : axes == 2 ? 9 : 27);
+    const int neg = n > 0 ? bc->h_negmask[b] : 0;
+    for (int k = 0; product && k < n; k++) {
+      const int e[3] = {layer[0] ? k % 3 : 0, layer[1] ? (k / (layer[0] ? 3 : 1)) % 3 : 0,
+                        layer[2] ? (k / ((layer[0] ? 3 : 1) * (layer[1] ? 3 : 1))) % 3 : 0};
+      int src = base;
+      double w = 1.0;
+      for (int d = 0; d < 3; d++) {
+        src += e[d] * s[d];
+        if (layer[d]) w *= nrpy_extrap_weight(layer[d], e[d]);
+      }
+      bool found = false;
+      for (int q = b; q < b + n; q++)
+        found = found || (bc->h_src[q] == src && bc->h_coeff[q] == w && bc->h_negmask[q] == neg);
+      product = found;
+    }
+    if (product) {
+      kind[axes < 1 ? 0 : axes - 1].push_back({bc->h_gdest[r], base, code, neg});
+    } else {
+      kind[3].push_back({bc->h_gdest[r], (int)L->h_terms.size(), NRPY_FILL_GENERIC, n});
+      for (int q = b; q < b + n; q++) L->h_terms.push_back({bc->h_coeff[q], bc->h_src[q], bc->h_negmask[q]});
+    }
+  }
+  for (const auto &rows : kind) L->h_rows.insert(L->h_rows.end(), rows.begin(), rows.end());
+  L->n = (int)L->h_rows.size();
+}
+
 static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
   const int Nxx_plus_2NGHOSTS0 = params->Nxx_plus_2NGHOSTS0;
   const int Nxx_plus_2NGHOSTS1 = params->Nxx_plus_2NGHOSTS1;
@@ -239,42 +385,51 @@ static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
     return i0 >= NGHOSTS && i0 < Nxx_plus_2NGHOSTS0 - NGHOSTS && i1 >= NGHOSTS &&
            i1 < Nxx_plus_2NGHOSTS1 - NGHOSTS && i2 >= NGHOSTS && i2 < Nxx_plus_2NGHOSTS2 - NGHOSTS;
   };
-  std::vector<int> slot(Ntot, -1);            // ghost idx3 -> row in 'rows'
-  std::vector<std::vector<nrpy_term>> rows;
-  std::vector<int> dests;
-  auto expand = [&](int idx, double c, int neg, std::vector<nrpy_term> &acc) -> bool {
+  std::vector<int> slot(Ntot, -1);            // ghost idx3 -> its row: terms [begin, end) of 'terms'
+  std::vector<nrpy_term> terms, acc;
+  std::vector<int> begin, end, anchors;       // anchor: the point a row copies
+  auto expand = [&](int idx, double c, int neg) -> bool {
     if (idx < 0 || idx >= Ntot) return false;
     if (interior(idx)) {
       acc.push_back({idx, neg, c});
       return true;
     }
     if (slot[idx] < 0) return false;          // ghost read before it was set
-    for (const nrpy_term &t : rows[slot[idx]]) acc.push_back({t.src, t.negmask ^ neg, t.coeff * c});
+    for (int k = begin[slot[idx]]; k < end[slot[idx]]; k++)
+      acc.push_back({terms[k].src, terms[k].negmask ^ neg, terms[k].coeff * c});
     return true;
   };
-  auto finish = [&](int dest, std::vector<nrpy_term> &acc) {
-    std::map<std::pair<int, int>, double> merged;
-    for (const nrpy_term &t : acc) merged[{t.src, t.negmask}] += t.coeff;
-    std::vector<nrpy_term> row;
-    for (auto &kv : merged)
-      if (kv.second != 0.0) row.push_back({kv.first.first, kv.first.second, kv.second});
-    if (slot[dest] < 0) {
-      slot[dest] = (int)rows.size();
-      rows.push_back(row);
-      dests.push_back(dest);
-    } else {
-      rows[slot[dest]] = row;
+  // the row of dest: acc sorted by (source, negmask), equal ones added up in their order
+  auto finish = [&](int dest, int from) {
+    const int anchor = from != dest && slot[from] >= 0 ? anchors[slot[from]] : from;
+    std::stable_sort(acc.begin(), acc.end(), [](const nrpy_term &x, const nrpy_term &y) {
+      return x.src != y.src ? x.src < y.src : x.negmask < y.negmask;
+    });
+    const int b = (int)terms.size();
+    for (size_t k = 0; k < acc.size();) {
+      nrpy_term t = acc[k++];
+      t.coeff = 0.0 + t.coeff;
+      for (; k < acc.size() && acc[k].src == t.src && acc[k].negmask == t.negmask; k++) t.coeff += acc[k].coeff;
+      if (t.coeff != 0.0) terms.push_back(t);
     }
+    if (slot[dest] < 0) {
+      slot[dest] = (int)begin.size();
+      begin.push_back(0);
+      end.push_back(0);
+      anchors.push_back(0);
+    }
+    begin[slot[dest]] = b;
+    end[slot[dest]] = (int)terms.size();
+    anchors[slot[dest]] = anchor;
+    acc.clear();
   };
   for (int gz = 0; gz < NGHOSTS; gz++) {
     for (const outer_bc &o : bc->outer[gz]) {
       const int dest = IDX3S(o.outer_bc_dest_pt.i0, o.outer_bc_dest_pt.i1, o.outer_bc_dest_pt.i2);
       const int stride = o.FACEi0 + Nxx_plus_2NGHOSTS0 * (o.FACEi1 + Nxx_plus_2NGHOSTS1 * o.FACEi2);
-      std::vector<nrpy_term> acc;
-      if (!expand(dest + stride, 3.0, 0, acc) || !expand(dest + 2 * stride, -3.0, 0, acc) ||
-          !expand(dest + 3 * stride, 1.0, 0, acc))
+      if (!expand(dest + stride, 3.0, 0) || !expand(dest + 2 * stride, -3.0, 0) || !expand(dest + 3 * stride, 1.0, 0))
         return NRPY_ERR_BCMAP;
-      finish(dest, acc);
+      finish(dest, dest);
     }
     for (const inner_bc &n : bc->inner[gz]) {
       const int dest = IDX3S(n.inner_bc_dest_pt.i0, n.inner_bc_dest_pt.i1, n.inner_bc_dest_pt.i2);
@@ -282,9 +437,8 @@ static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
       int neg = 0;
       for (int p = 0; p < 10; p++)
         if (n.parity[p] < 0) neg |= (1 << p);
-      std::vector<nrpy_term> acc;
-      if (!expand(src, 1.0, neg, acc)) return NRPY_ERR_BCMAP;
-      finish(dest, acc);
+      if (!expand(src, 1.0, neg)) return NRPY_ERR_BCMAP;
+      finish(dest, src);
     }
   }
   bc->h_gdest.clear();
@@ -292,46 +446,31 @@ static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
   bc->h_src.clear();
   bc->h_coeff.clear();
   bc->h_negmask.clear();
-  // Order rows by destination so consecutive lanes write nearby addresses.
-  std::vector<int> order(rows.size());
-  for (size_t r = 0; r < rows.size(); r++) order[r] = (int)r;
-  std::sort(order.begin(), order.end(), [&](int a, int b) { return dests[a] < dests[b]; });
-  for (int r : order) {
-    bc->h_gdest.push_back(dests[r]);
-    for (const nrpy_term &t : rows[r]) {
-      bc->h_src.push_back(t.src);
-      bc->h_coeff.push_back(t.coeff);
-      bc->h_negmask.push_back(t.negmask);
+  // Rows in the order of their points, so that consecutive lanes write nearby addresses.
+  std::vector<int> anchor;
+  bc->h_gdest.reserve(begin.size());
+  bc->h_rowptr.reserve(begin.size() + 1);
+  anchor.reserve(begin.size());
+  for (int idx = 0; idx < Ntot; idx++) {
+    const int r = slot[idx];
+    if (r < 0) continue;
+    bc->h_gdest.push_back(idx);
+    anchor.push_back(anchors[r]);
+    for (int k = begin[r]; k < end[r]; k++) {
+      bc->h_src.push_back(terms[k].src);
+      bc->h_coeff.push_back(terms[k].coeff);
+      bc->h_negmask.push_back(terms[k].negmask);
     }
     bc->h_rowptr.push_back((int)bc->h_src.size());
   }
   bc->nghost = (int)bc->h_gdest.size();
   bc->nterms = (int)bc->h_src.size();
-  // Transpose: for every interior source point, the ghost points whose value it enters.
-  {
-    std::vector<int> perm(bc->h_src.size()), termrow(bc->h_src.size());
-    for (int r = 0; r < bc->nghost; r++)
-      for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) termrow[k] = r;
-    for (size_t k = 0; k < perm.size(); k++) perm[k] = (int)k;
-    std::stable_sort(perm.begin(), perm.end(), [&](int a, int b) { return bc->h_src[a] < bc->h_src[b]; });
-    bc->h_tsrc.clear();
-    bc->h_trowptr.assign(1, 0);
-    bc->h_tghost.clear();
-    bc->h_tcoeff.clear();
-    bc->h_tnegmask.clear();
-    for (size_t q = 0; q < perm.size(); q++) {
-      const int k = perm[q];
-      if (bc->h_tsrc.empty() || bc->h_tsrc.back() != bc->h_src[k]) {
-        if (!bc->h_tsrc.empty()) bc->h_trowptr.push_back((int)bc->h_tghost.size());
-        bc->h_tsrc.push_back(bc->h_src[k]);
-      }
-      bc->h_tghost.push_back(bc->h_gdest[termrow[k]]);
-      bc->h_tcoeff.push_back(bc->h_coeff[k]);
-      bc->h_tnegmask.push_back(bc->h_negmask[k]);
-    }
-    if (!bc->h_tsrc.empty()) bc->h_trowptr.push_back((int)bc->h_tghost.size());
-    bc->ntsrc = (int)bc->h_tsrc.size();
-  }
+  std::vector<char> all(bc->nghost, 1), reached(bc->nghost);
+  for (int r = 0; r < bc->nghost; r++) reached[r] = nrpy_stage_reads(params, bc->h_gdest[r]);
+  nrpy_build_transpose(bc, Ntot, all, &bc->trans_all);
+  nrpy_build_transpose(bc, Ntot, reached, &bc->trans_stage);
+  nrpy_build_fill(params, bc, anchor, all, &bc->fill_all);
+  nrpy_build_fill(params, bc, anchor, reached, &bc->fill_stage);
   return NRPY_OK;
 }
 
@@ -354,15 +493,17 @@ extern "C" void bcstruct_free(bc_struct *bc) {
   (void)hipFree(bc->d_ib_src);
   (void)hipFree(bc->d_ib_parity);
   (void)hipFree(bc->d_gdest);
-  (void)hipFree(bc->d_rowptr);
-  (void)hipFree(bc->d_src);
-  (void)hipFree(bc->d_coeff);
-  (void)hipFree(bc->d_negmask);
-  (void)hipFree(bc->d_tsrc);
-  (void)hipFree(bc->d_trowptr);
-  (void)hipFree(bc->d_tghost);
-  (void)hipFree(bc->d_tcoeff);
-  (void)hipFree(bc->d_tnegmask);
+  for (nrpy_fill_list *L : {&bc->fill_all, &bc->fill_stage}) {
+    (void)hipFree(L->d_rows);
+    (void)hipFree(L->d_terms);
+  }
+  for (nrpy_transpose_list *T : {&bc->trans_all, &bc->trans_stage}) {
+    (void)hipFree(T->d_src);
+    (void)hipFree(T->d_rowptr);
+    (void)hipFree(T->d_ghost);
+    (void)hipFree(T->d_coeff);
+    (void)hipFree(T->d_negmask);
+  }
   (void)hipFree(bc->d_som_rhs);
   delete bc;
 }
@@ -462,16 +603,16 @@ extern "C" int bcstruct_create(const paramstruct *params, double *xx[3], bc_stru
             nrpy_upload(&bc->d_ib_dest, ibd.data(), ibd.size()) &&
             nrpy_upload(&bc->d_ib_src, ibs.data(), ibs.size()) &&
             nrpy_upload(&bc->d_ib_parity, ibp.data(), ibp.size()) &&
-            nrpy_upload(&bc->d_gdest, bc->h_gdest.data(), bc->h_gdest.size()) &&
-            nrpy_upload(&bc->d_rowptr, bc->h_rowptr.data(), bc->h_rowptr.size()) &&
-            nrpy_upload(&bc->d_src, bc->h_src.data(), bc->h_src.size()) &&
-            nrpy_upload(&bc->d_coeff, bc->h_coeff.data(), bc->h_coeff.size()) &&
-            nrpy_upload(&bc->d_negmask, bc->h_negmask.data(), bc->h_negmask.size()) &&
-            nrpy_upload(&bc->d_tsrc, bc->h_tsrc.data(), bc->h_tsrc.size()) &&
-            nrpy_upload(&bc->d_trowptr, bc->h_trowptr.data(), bc->h_trowptr.size()) &&
-            nrpy_upload(&bc->d_tghost, bc->h_tghost.data(), bc->h_tghost.size()) &&
-            nrpy_upload(&bc->d_tcoeff, bc->h_tcoeff.data(), bc->h_tcoeff.size()) &&
-            nrpy_upload(&bc->d_tnegmask, bc->h_tnegmask.data(), bc->h_tnegmask.size());
+            nrpy_upload(&bc->d_gdest, bc->h_gdest.data(), bc->h_gdest.size());
+  for (nrpy_fill_list *L : {&bc->fill_all, &bc->fill_stage})
+    ok = ok && nrpy_upload(&L->d_rows, L->h_rows.data(), L->h_rows.size()) &&
+         nrpy_upload(&L->d_terms, L->h_terms.data(), L->h_terms.size());
+  for (nrpy_transpose_list *T : {&bc->trans_all, &bc->trans_stage})
+    ok = ok && nrpy_upload(&T->d_src, T->h_src.data(), T->h_src.size()) &&
+         nrpy_upload(&T->d_rowptr, T->h_rowptr.data(), T->h_rowptr.size()) &&
+         nrpy_upload(&T->d_ghost, T->h_ghost.data(), T->h_ghost.size()) &&
+         nrpy_upload(&T->d_coeff, T->h_coeff.data(), T->h_coeff.size()) &&
+         nrpy_upload(&T->d_negmask, T->h_negmask.data(), T->h_negmask.size());
   if (!ok) {
     bcstruct_free(bc);
     return NRPY_ERR_ALLOC;
@@ -511,6 +652,23 @@ extern "C" int bcstruct_get_composed(const bc_struct *bc, int *gdest, int *rowpt
   if (src) memcpy(src, bc->h_src.data(), sizeof(int) * bc->h_src.size());
   if (coeff) memcpy(coeff, bc->h_coeff.data(), sizeof(double) * bc->h_coeff.size());
   if (negmask) memcpy(negmask, bc->h_negmask.data(), sizeof(int) * bc->h_negmask.size());
+  return NRPY_OK;
+}
+
+// The rows of the fill lists (every ghost, or with stage != 0 those a stage's stencils reach):
+// rows 4 ints each (dest, base, code, negmask), terms as coefficients, sources and masks.
+extern "C" int bcstruct_get_fill(const bc_struct *bc, int stage, int *nrows, int *nterms, int *rows, double *coeff,
+                                 int *src, int *negmask) {
+  if (!bc) return NRPY_ERR_NULL;
+  const nrpy_fill_list &L = stage ? bc->fill_stage : bc->fill_all;
+  if (nrows) *nrows = L.n;
+  if (nterms) *nterms = (int)L.h_terms.size();
+  if (rows) memcpy(rows, L.h_rows.data(), sizeof(nrpy_fill_row) * L.h_rows.size());
+  for (size_t k = 0; k < L.h_terms.size(); k++) {
+    if (coeff) coeff[k] = L.h_terms[k].coeff;
+    if (src) src[k] = L.h_terms[k].src;
+    if (negmask) negmask[k] = L.h_terms[k].negmask;
+  }
   return NRPY_OK;
 }
 
@@ -621,33 +779,114 @@ __device__ __forceinline__ double nrpy_map_row_sum(const int b, const int e, con
   return acc;
 }
 
-__global__ void nrpy_bc_composed_kernel(int nghost, const int *__restrict__ gdest, const int *__restrict__ rowptr,
-                                        const int *__restrict__ src, const double *__restrict__ coeff,
-                                        const int *__restrict__ negmask, int num_gfs, nrpy_gf_parity_args gfp,
-                                        size_t Ntot, double *__restrict__ gfs) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)nghost * num_gfs) return;
-  const int gf = (int)(t / nghost);
-  const int r = (int)(t % nghost);
-  double *g = gfs + (size_t)gf * Ntot;
-  const int bit = 1 << gfp.p[gf];
-  g[gdest[r]] = nrpy_map_row_sum(rowptr[r], rowptr[r + 1], src, coeff, negmask, bit, g);
+// Ghost value(s) of row R for the K gridfunctions gf0 .. of the array gfs (num_gfs in all),
+// with plane strides of the grid the row belongs to. The loads of a row with up to one
+// extrapolated axis, and of nine terms of the others, are issued together for all K.
+template <int K>
+__device__ __forceinline__ void nrpy_fill_point(const nrpy_fill_row R, const nrpy_fill_term *__restrict__ terms,
+                                                const int N0, const int N01, const size_t Ntot, const int gf0,
+                                                const int num_gfs, const nrpy_gf_parity_args &gfp,
+                                                double *__restrict__ gfs) {
+  const double *g[K];
+  double acc[K];
+#pragma unroll
+  for (int j = 0; j < K; j++) g[j] = gfs + (size_t)min(gf0 + j, num_gfs - 1) * Ntot;
+  if (R.code == NRPY_FILL_GENERIC) {
+#pragma unroll
+    for (int j = 0; j < K; j++) acc[j] = 0.0;
+    for (int k = 0; k < R.negmask; k++) {
+      const nrpy_fill_term t = terms[R.base + k];
+#pragma unroll
+      for (int j = 0; j < K; j++) {
+        const int bit = 1 << gfp.p[min(gf0 + j, num_gfs - 1)];
+        acc[j] += ((t.negmask & bit) ? -t.coeff : t.coeff) * g[j][t.src];
+      }
+    }
+  } else {
+    const int c0 = R.code & 7, c1 = (R.code >> 3) & 7, c2 = (R.code >> 6) & 7;
+    const int l0 = c0 > 3 ? c0 - 3 : c0, l1 = c1 > 3 ? c1 - 3 : c1, l2 = c2 > 3 ? c2 - 3 : c2;
+    const int s0 = c0 > 3 ? -1 : 1, s1 = c1 > 3 ? -N0 : N0, s2 = c2 > 3 ? -N01 : N01;
+    // the first extrapolated axis is the inner one; a row without one has a single term
+    const int li = l0 ? l0 : l1 ? l1 : l2, si = l0 ? s0 : l1 ? s1 : s2;
+    const int lm = l0 ? (l1 ? l1 : l2) : l1 ? l2 : 0, sm = l0 ? (l1 ? s1 : s2) : s2;
+    const int lo = l0 && l1 ? l2 : 0, so = s2;
+    if (lm == 0) {
+      double v[K][3];
+#pragma unroll
+      for (int j = 0; j < K; j++) {
+        v[j][0] = g[j][R.base];
+        v[j][1] = g[j][li ? R.base + si : R.base];
+        v[j][2] = g[j][li ? R.base + 2 * si : R.base];
+      }
+#pragma unroll
+      for (int j = 0; j < K; j++)
+        acc[j] = li ? fma(nrpy_extrap_weight(li, 2), v[j][2],
+                          fma(nrpy_extrap_weight(li, 1), v[j][1], nrpy_extrap_weight(li, 0) * v[j][0]))
+                    : v[j][0];
+    } else {
+#pragma unroll
+      for (int j = 0; j < K; j++) acc[j] = 0.0;
+      for (int c = 0; c < (lo ? 3 : 1); c++) {
+        const double wc = lo ? nrpy_extrap_weight(lo, c) : 1.0;
+        double v[K][9];
+#pragma unroll
+        for (int j = 0; j < K; j++)
+#pragma unroll
+          for (int q = 0; q < 9; q++) v[j][q] = g[j][R.base + c * so + (q / 3) * sm + (q % 3) * si];
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+          const double w = wc * nrpy_extrap_weight(lm, q / 3) * nrpy_extrap_weight(li, q % 3);
+#pragma unroll
+          for (int j = 0; j < K; j++) acc[j] = fma(w, v[j][q], acc[j]);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < K; j++) acc[j] = (R.negmask & (1 << gfp.p[min(gf0 + j, num_gfs - 1)])) ? -acc[j] : acc[j];
+  }
+#pragma unroll
+  for (int j = 0; j < K; j++)
+    if (gf0 + j < num_gfs) gfs[(size_t)(gf0 + j) * Ntot + R.dest] = acc[j];
 }
 
-extern "C" int apply_bcs_curvilinear_composed(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
-                                              const int8_t *gfs_parity, double *gfs, hipStream_t stream) {
+#define NRPY_FILL_K 2
+__global__ void __launch_bounds__(256)
+nrpy_bc_fill_kernel(const int nrows, const nrpy_fill_row *__restrict__ rows,
+                    const nrpy_fill_term *__restrict__ terms, const int N0, const int N01, const int num_gfs,
+                    const nrpy_gf_parity_args gfp, const size_t Ntot, double *__restrict__ gfs) {
+  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (r >= nrows) return;
+  nrpy_fill_point<NRPY_FILL_K>(rows[r], terms, N0, N01, Ntot, NRPY_FILL_K * (int)blockIdx.y, num_gfs, gfp, gfs);
+}
+
+static int nrpy_fill_launch(const paramstruct *params, const bc_struct *bc, const nrpy_fill_list &L, const int NUM_GFS,
+                            const int8_t *gfs_parity, double *gfs, hipStream_t stream) {
   nrpy_gf_parity_args gfp;
   memset(&gfp, 0, sizeof(gfp));
   int rc = nrpy_bc_check(params, bc, NUM_GFS, gfs_parity, gfs, &gfp);
   if (rc) return rc;
-  if (bc->nghost == 0) return NRPY_OK;
+  if (L.n == 0) return NRPY_OK;
   const size_t Ntot = (size_t)bc->N[0] * bc->N[1] * bc->N[2];
   const int B = 256;
-  const size_t work = (size_t)bc->nghost * NUM_GFS;
-  hipLaunchKernelGGL(nrpy_bc_composed_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream,
-                     bc->nghost, bc->d_gdest, bc->d_rowptr, bc->d_src, bc->d_coeff, bc->d_negmask, NUM_GFS, gfp,
-                     Ntot, gfs);
+  hipLaunchKernelGGL(nrpy_bc_fill_kernel, dim3((unsigned)((L.n + B - 1) / B), (NUM_GFS + NRPY_FILL_K - 1) / NRPY_FILL_K),
+                     dim3(B), 0, stream, L.n, L.d_rows, L.d_terms, bc->N[0], bc->N[0] * bc->N[1], NUM_GFS, gfp, Ntot,
+                     gfs);
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+
+extern "C" int apply_bcs_curvilinear_composed(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
+                                              const int8_t *gfs_parity, double *gfs, hipStream_t stream) {
+  if (!bc) return NRPY_ERR_NULL;
+  return nrpy_fill_launch(params, bc, bc->fill_all, NUM_GFS, gfs_parity, gfs, stream);
+}
+
+// The fill of a stage of the RK4 step, whose state is only read by the next right-hand side:
+// the ghost points that its stencils reach. Corner ghosts (27 terms each) are never among
+// them, and in the axisymmetric bundles, which read no neighbours in i2, nor is any i2 ghost.
+static int nrpy_stage_fill(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
+                           const int8_t *gfs_parity, double *gfs, hipStream_t stream) {
+  if (!bc) return NRPY_ERR_NULL;
+  return nrpy_fill_launch(params, bc, bc->fill_stage, NUM_GFS, gfs_parity, gfs, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -677,11 +916,8 @@ __global__ void nrpy_clear_ghosts_kernel(int nghost, const int *__restrict__ gde
   gfs[(size_t)(t / nghost) * Ntot + gdest[t % nghost]] = 0.0;
 }
 
-// Transpose of apply_bcs_curvilinear(_composed): folds the cotangents held at ghost
-// points onto the interior points the ghost values were computed from, then zeroes
-// the ghost cotangents. No counterpart in the reference (it has no adjoint).
-extern "C" int bc_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
-                          const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
+static int nrpy_transpose_launch(const paramstruct *params, const bc_struct *bc, const nrpy_transpose_list &T,
+                                 const int NUM_GFS, const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
   nrpy_gf_parity_args gfp;
   memset(&gfp, 0, sizeof(gfp));
   int rc = nrpy_bc_check(params, bc, NUM_GFS, gfs_parity, cot_gfs, &gfp);
@@ -689,16 +925,32 @@ extern "C" int bc_apply_T(const paramstruct *params, const bc_struct *bc, const 
   if (bc->nghost == 0) return NRPY_OK;
   const size_t Ntot = (size_t)bc->N[0] * bc->N[1] * bc->N[2];
   const int B = 256;
-  if (bc->ntsrc > 0) {
-    const size_t work = (size_t)bc->ntsrc * NUM_GFS;
-    hipLaunchKernelGGL(nrpy_bc_transpose_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream,
-                       bc->ntsrc, bc->d_tsrc, bc->d_trowptr, bc->d_tghost, bc->d_tcoeff, bc->d_tnegmask, NUM_GFS,
-                       gfp, Ntot, cot_gfs);
+  if (T.n > 0) {
+    const size_t work = (size_t)T.n * NUM_GFS;
+    hipLaunchKernelGGL(nrpy_bc_transpose_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream, T.n,
+                       T.d_src, T.d_rowptr, T.d_ghost, T.d_coeff, T.d_negmask, NUM_GFS, gfp, Ntot, cot_gfs);
   }
   const size_t work = (size_t)bc->nghost * NUM_GFS;
   hipLaunchKernelGGL(nrpy_clear_ghosts_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream,
                      bc->nghost, bc->d_gdest, NUM_GFS, Ntot, cot_gfs);
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+
+// Transpose of apply_bcs_curvilinear(_composed): folds the cotangents held at ghost
+// points onto the interior points the ghost values were computed from, then zeroes
+// the ghost cotangents. No counterpart in the reference (it has no adjoint).
+extern "C" int bc_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
+                          const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
+  if (!bc) return NRPY_ERR_NULL;
+  return nrpy_transpose_launch(params, bc, bc->trans_all, NUM_GFS, gfs_parity, cot_gfs, stream);
+}
+
+// The same for a cotangent that a right-hand side's transposed stencils wrote: it is zero at
+// the ghost points they do not reach, so only the others are folded.
+static int nrpy_stage_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
+                              const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
+  if (!bc) return NRPY_ERR_NULL;
+  return nrpy_transpose_launch(params, bc, bc->trans_stage, NUM_GFS, gfs_parity, cot_gfs, stream);
 }
 
 __global__ void nrpy_lincomb_kernel(size_t n, double *__restrict__ out, double a, const double *__restrict__ x,

@@ -165,6 +165,7 @@ static __device__ double nrpy_discard[64];
 #define NRPY_BATCH_ROLE_AUX 5
 #define NRPY_RANGE_INTERIOR 0
 #define NRPY_RANGE_ALL 1
+#define NRPY_RANGE_STAGE 2  // without the ghosts of the axes along which no stencil reads
 
 // Per-kernel block shapes, settable at run time (nrpy_set_block_shape) so an
 // autotuner can pick them; index by NRPY_KERNEL_* ids defined per bundle.

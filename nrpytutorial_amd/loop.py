@@ -2,7 +2,8 @@
 
 ``simple_loop(options, interior)`` keeps the option vocabulary of loop.py
 (loop.py:129-194): ``AllPoints`` / ``InteriorPoints`` choose the index range
-([0, N+2G) or [G, N+G) in each direction), ``Read_xxs`` makes the coordinates
+([0, N+2G) or [G, N+G) in each direction; ``StagePoints``, not in the reference, the whole range
+along the axes on which the bundle's stencils read neighbours and the interior along the others), ``Read_xxs`` makes the coordinates
 xx0, xx1, xx2 available, ``Enable_rfm_precompute`` reads the precomputed
 reference-metric tables, and ``EnableSIMD`` / ``DisableOpenMP`` /
 ``OMP_custom_pragma`` are accepted and have no effect.
@@ -127,6 +128,8 @@ def parse_loopopts(options):
             opts["range"] = "all"
         elif o == "InteriorPoints":
             opts["range"] = "interior"
+        elif o == "StagePoints":
+            opts["range"] = "stage"
         elif o == "Read_xxs":
             opts["Read_xxs"] = True
         elif o == "Enable_rfm_precompute":
@@ -137,7 +140,7 @@ def parse_loopopts(options):
         else:
             raise ValueError("unknown loop option '" + o + "'")
     if opts["range"] is None:
-        raise ValueError("loop options must contain AllPoints or InteriorPoints")
+        raise ValueError("loop options must contain AllPoints, InteriorPoints or StagePoints")
     if opts["Read_xxs"] and opts["rfm"]:
         raise ValueError("Read_xxs and Enable_rfm_precompute are mutually exclusive")
     return opts
@@ -165,19 +168,26 @@ def simple_loop(options, interior, batched=False):
     batched=True: the block's tile comes from the instance table of a batched launch
     (NRPY_BATCH_TILE, defined by the batched kernel prologue) instead of the XCD remap."""
     o = parse_loopopts(options)
-    lo = "NGHOSTS" if o["range"] == "interior" else "0"
-    n = ("Nxx%d" if o["range"] == "interior" else "Nxx_plus_2NGHOSTS%d")
+    lo = {"interior": "NGHOSTS", "all": "0", "stage": "NRPY_STAGE_LO%d"}[o["range"]]
+    n = {"interior": "Nxx%d", "all": "Nxx_plus_2NGHOSTS%d",
+         "stage": "(Nxx_plus_2NGHOSTS%d - 2*NRPY_STAGE_LO%d)"}[o["range"]]
+
+    def at(t, d):
+        return t.replace("%d", str(d))
     # One-dimensional grid of blocks; NRPY_BLOCK_COORDS remaps the hardware's
     # round-robin block-to-XCD assignment to contiguous tiles per XCD and
     # decodes the (bx, by, bz) tile of this block.
     if batched:
-        s = "NRPY_BATCH_TILE(%s, %s, %s);\n" % (n % 0, n % 1, n % 2)
+        s = "NRPY_BATCH_TILE(%s, %s, %s);\n" % (at(n, 0), at(n, 1), at(n, 2))
     else:
-        s = "NRPY_BLOCK_COORDS(%s, %s, %s);\n" % (n % 0, n % 1, n % 2)
+        s = "NRPY_BLOCK_COORDS(%s, %s, %s);\n" % (at(n, 0), at(n, 1), at(n, 2))
     for d, t in ((0, "x"), (1, "y"), (2, "z")):
-        s += "const int i%d = %s + nrpy_b%s*(int)blockDim.%s + (int)threadIdx.%s;\n" % (d, lo, t, t, t)
+        s += "const int i%d = %s + nrpy_b%s*(int)blockDim.%s + (int)threadIdx.%s;\n" % (d, at(lo, d), t, t, t)
     if o["range"] == "interior":
         s += "if (i0 >= Nxx0 + NGHOSTS || i1 >= Nxx1 + NGHOSTS || i2 >= Nxx2 + NGHOSTS) return;\n"
+    elif o["range"] == "stage":
+        s += "if (%s) return;\n" % " || ".join("i%d >= Nxx_plus_2NGHOSTS%d - NRPY_STAGE_LO%d" % (d, d, d)
+                                               for d in range(3))
     else:
         s += ("if (i0 >= Nxx_plus_2NGHOSTS0 || i1 >= Nxx_plus_2NGHOSTS1 || i2 >= Nxx_plus_2NGHOSTS2) return;\n")
     if o["Read_xxs"]:
@@ -260,7 +270,7 @@ def kernel_and_launcher(name, desc, args, preloop, body, loopopts, postloop):
     kernel = ("/* %s */\n__global__ void __launch_bounds__(%s) %s(%s) {\n%s%s}\n" %
               (desc, launch_bounds(name), kname, ", ".join(kargs), unpack,
                "".join("  " + l + "\n" for l in full.splitlines())))
-    rng = "interior" if o["range"] == "interior" else "all"
+    rng = o["range"]
     block = None
     if rng == "interior":
         kernel, block = stage_lds(name, kernel)
@@ -274,6 +284,8 @@ def kernel_and_launcher(name, desc, args, preloop, body, loopopts, postloop):
             block = "dim3(%d, %d, %d)" % tile
     if rng == "interior":
         n0, n1, n2 = "params->Nxx0", "params->Nxx1", "params->Nxx2"
+    elif rng == "stage":
+        n0, n1, n2 = ("params->Nxx_plus_2NGHOSTS%d - 2*NRPY_STAGE_LO%d" % (d, d) for d in range(3))
     else:
         n0, n1, n2 = "params->Nxx_plus_2NGHOSTS0", "params->Nxx_plus_2NGHOSTS1", "params->Nxx_plus_2NGHOSTS2"
     ptr_checks = " || ".join("!" + c for c in call if not c.startswith("*") and "xx[" not in c) or "0"
