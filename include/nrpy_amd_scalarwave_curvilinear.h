@@ -47,7 +47,10 @@ int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *params, const
 
 
 /* The Sommerfeld step above captured into a hipGraph (no counterpart in the reference; pointers, xx
- * and dt fixed at capture), replayed nsteps times per MoL_graph_launch, freed with MoL_graph_free. */
+ * and dt fixed at capture), replayed nsteps times per MoL_graph_launch, freed with MoL_graph_free.
+ * The captured step takes two launches per substep instead of one per layer and face group, with
+ * the same values. It allocates device memory that the graph owns until MoL_graph_free
+ * (2 NUM_EVOL_GFS + 5 gridfunctions); without that memory it captures the step above. */
 int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3],
                                 const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs,
                                 double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out);

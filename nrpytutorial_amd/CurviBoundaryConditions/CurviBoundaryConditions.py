@@ -194,13 +194,7 @@ class sommerfeld_boundary_condition_class():
             body = "double J00, J01, J02, J10, J11, J12, J20, J21, J22;\n" + body
             body += ("const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;\n"
                      "*dfdr_out = (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/(J00*cof0 + J01*cof1 + J02*cof2);\n")
-        coef = ""
-        if fd_order == 4:
-            coef = ("  const double u0 = -25./12., u1 = 4., u2 = -3., u3 = 4./3., u4 = -1./4.;\n"
-                    "  const double c1 = 2./3., c2 = 1./12.;\n")
-        elif fd_order == 6:
-            coef = ("  const double u0 = -49./20., u1 = 6., u2 = -15./2., u3 = 20./3., u4 = -15./4., u5 = 6./5., "
-                    "u6 = -1./6.;\n  const double c1 = 3./4., c2 = 3./20., c3 = 1./60;\n")
+        coef = self._stencil_constants(fd_order)
         dirs = "".join(self._direction_code(d, fd_order) for d in range(3))
         text = coef + dirs + "".join("  " + line + "\n" for line in body.splitlines())
         unpack = bd._unpack_for(text).replace("params->", "params.")
@@ -219,12 +213,79 @@ class sommerfeld_boundary_condition_class():
                 "  double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;\n"
                 "  (void)fdD0; (void)fdD1; (void)fdD2;\n" + text + "}\n")
 
-    def hip_source(self):
-        """Parameters, r/dfdr device function, kernels and the apply_bcs_sommerfeld launcher."""
+    def geometry_functions(self):
+        """dfdr_function in two parts, for bundles with a kernel that keeps the geometry in a table:
+        nrpy_sommerfeld_geometry gives r and what the derivative needs of the Jacobian at a point
+        (the three cofactors and the determinant, or the simplified contraction's three
+        coefficients over 1), nrpy_sommerfeld_dfdr_from contracts the stencils with them, and
+        nrpy_sommerfeld_r_dfdr is one after the other. The geometry is opaque to the compiler in
+        between, so that no multiply-add is contracted across and both uses round alike."""
+        from .. import outputC as oc
+        from ..codegen import bundle as bd
+        if self._simplified():
+            r, contraction = self.radial_contraction()
+            fdD = ixp.declarerank1("fdD")
+            unit = [contraction.subs({fdD[j]: 1 if i == j else 0 for j in range(3)}) for i in range(3)]
+            body = oc.outputC([r] + unit + [sp.Integer(1)], ["geo[%d]" % k for k in range(5)], "returnstring",
+                              params="includebraces=False,outCverbose=False")
+        else:
+            r, J = self.jacobian()
+            body = "double J00, J01, J02, J10, J11, J12, J20, J21, J22;\n" + oc.outputC(
+                [r] + [J[i][j] for i in range(3) for j in range(3)],
+                ["geo[0]"] + ["J%d%d" % (i, j) for i in range(3) for j in range(3)], "returnstring",
+                params="includebraces=False,outCverbose=False")
+            body += ("const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;\n"
+                     "geo[1] = cof0; geo[2] = cof1; geo[3] = cof2;\n"
+                     "geo[4] = J00*cof0 + J01*cof1 + J02*cof2;\n")
+        unpack = bd._unpack_for(body).replace("params->", "params.")
+        dirs = "".join(self._direction_code(d, self.fd_order) for d in range(3))
+        coef = self._stencil_constants(self.fd_order)
+        dunpack = bd._unpack_for(coef + dirs).replace("params->", "params.")
+        for n in ("Nxx_plus_2NGHOSTS0", "Nxx_plus_2NGHOSTS1", "Nxx_plus_2NGHOSTS2", "invdx0", "invdx1", "invdx2"):
+            if "const int %s =" % n not in dunpack and "const double %s =" % n not in dunpack:
+                dunpack += "  const %s %s = params.%s;\n" % ("int" if n.startswith("Nxx") else "double", n, n)
+        return ("// r and the radial derivative's geometry at a point: geo = r, then a_i and b of\n"
+                "// d f/d r = sum_i fdD_i a_i / b.\n"
+                "static __device__ void nrpy_sommerfeld_geometry(const paramstruct &params, const double xx0, "
+                "const double xx1, const double xx2, double *geo) {\n" + unpack +
+                "  (void)xx0; (void)xx1; (void)xx2;\n" + "".join("  " + line + "\n" for line in body.splitlines()) + "}\n"
+                "template <typename FA>\n"
+                "static __device__ double nrpy_sommerfeld_dfdr_from(const paramstruct &params, const double *geo, FA fa, "
+                "const int F0, const int F1, const int F2, const int i0, const int i1, const int i2) {\n" + dunpack +
+                "  double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;\n" + coef + dirs +
+                "  const double cof0 = geo[1], cof1 = geo[2], cof2 = geo[3];\n"
+                "  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];\n}\n"
+                "// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's\n"
+                "// FACE (CurviBoundaryConditions.py:329-516).\n"
+                "template <typename FA>\n"
+                "static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ "
+                "xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, "
+                "const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, "
+                "double *dfdr_out) {\n"
+                "  double geo[5];\n  nrpy_sommerfeld_geometry(params, xx0_arr[i0], xx1_arr[i1], xx2_arr[i2], geo);\n"
+                "#pragma unroll\n  for (int k = 0; k < 5; k++) asm(\"\" : \"+v\"(geo[k]));\n"
+                "  *r_out = geo[0];\n"
+                "  *dfdr_out = nrpy_sommerfeld_dfdr_from(params, geo, fa, F0, F1, F2, i0, i1, i2);\n}\n")
+
+    @staticmethod
+    def _stencil_constants(fd_order):
+        if fd_order == 4:
+            return ("  const double u0 = -25./12., u1 = 4., u2 = -3., u3 = 4./3., u4 = -1./4.;\n"
+                    "  const double c1 = 2./3., c2 = 1./12.;\n")
+        if fd_order == 6:
+            return ("  const double u0 = -49./20., u1 = 6., u2 = -15./2., u3 = 20./3., u4 = -15./4., u5 = 6./5., "
+                    "u6 = -1./6.;\n  const double c1 = 3./4., c2 = 3./20., c3 = 1./60;\n")
+        return ""
+
+    def hip_source(self, chain=False):
+        """Parameters, r/dfdr device function, kernels and the apply_bcs_sommerfeld launcher; with
+        ``chain`` also the one-launch form for grids with inner boundary points."""
         # the one-sided stencils reach fd_order points inward from a point within NGHOSTS of an edge
         minn = ("#define NRPY_SOMMERFELD_MIN_N (NGHOSTS + %d + 1)\n#define NRPY_SOMMERFELD_FD %d\n"
                 % (self.fd_order, self.fd_order))
-        return self.sommerfeld_params() + minn + self.dfdr_function() + _SOMMERFELD_KERNELS
+        return (self.sommerfeld_params() + minn + (self.geometry_functions() if chain else self.dfdr_function()) +
+                _SOMMERFELD_KERNELS +
+                (_SOMMERFELD_CHAIN if chain else ""))
 
     def write_sommerfeld_main_Ccode(self, Ccodesdir):
         os.makedirs(os.path.join(Ccodesdir, "boundary_conditions"), exist_ok=True)
@@ -621,6 +682,240 @@ extern "C" int apply_bcs_sommerfeld(const paramstruct *params, double *xx[3], co
                          bc->d_ib_dest + bc->ib_off[gz], bc->d_ib_src + bc->ib_off[gz],
                          bc->d_ib_parity + 10 * (size_t)bc->ib_off[gz], NUM_GFS, gfp, Ntot, rhs_gfs);
     }
+  }
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+'''
+
+_SOMMERFELD_CHAIN = r'''
+// The whole condition in two launches per substep, for grids with inner boundary points. The
+// reference's order (layer by layer, face group by face group, then the parity copies) makes a
+// chain of each outer point: its RHS is
+//   rhs_p = A_p + (rhs_q + B_p) (r_q / r_p)^n,   q its inward neighbour (an interior point, or an
+// outer point one step further in), A_p = -v X_p, B_p = v X_q, X = d f/d r + (f - f_inf)/r with
+// the stencils of p's FACE. A and B need only the state the substep starts from, so they are
+// evaluated for every outer point at once, in extra blocks of the interior RHS launch
+// (nrpy_sommerfeld_eval); the second launch (nrpy_sommerfeld_chain_kernel) walks each ghost
+// point's chain from the interior out, at most 3 NGHOSTS multiply-adds, an inner point that of
+// the point it copies, and does the RK4 update there. Every point's FACE follows from its
+// indices: the axis with the largest distance outside the interior, the last of equals
+// (nrpy_sommerfeld_chainable checks it against the lists). The arithmetic is that of
+// nrpy_sommerfeld_rhs.
+// Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
+// launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
+// chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table
+// (geo, 5 values per point, written once per captured step) instead of the Jacobian.
+// Scratch of a captured step: R, NUM_EVOL_GFS gridfunctions: the RHS at the interior points a
+// chain or copy ends at (rhs_eval_rk4_substep_rim), A at the outer points; then B, as many; then geo.
+#define NRPY_SOM_NSCRATCH (2 * NUM_EVOL_GFS + 5)
+
+// Step k of n (k = 0 the innermost) of the chain with layers l: its axis.
+__device__ __forceinline__ int nrpy_som_chain_axis(const int l0, const int l1, const int l2, const int k) {
+  int m0 = l0, m1 = l1, m2 = l2, a = 0;
+  for (int j = l0 + l1 + l2 - 1; j >= k; j--) {
+    const int far = max(m0, max(m1, m2));
+    a = m2 == far ? 2 : m1 == far ? 1 : 0;
+    m0 -= a == 0;
+    m1 -= a == 1;
+    m2 -= a == 2;
+  }
+  return a;
+}
+
+// A and B at outer point number t % n of the lists (all layers) of gridfunction t / n.
+__device__ __forceinline__ void nrpy_sommerfeld_eval(const paramstruct &params, const size_t t, const int n,
+                                                     const int *__restrict__ dest, const int8_t *__restrict__ face,
+                                                     const double *__restrict__ gfs, double *__restrict__ R) {
+  if (t >= (size_t)n * NUM_EVOL_GFS) return;
+  const int gf = (int)(t / n), p = (int)(t % n);
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1;
+  const size_t Ntot = (size_t)N0 * N1 * params.Nxx_plus_2NGHOSTS2;
+  const double *__restrict__ geo = R + (size_t)(2 * NUM_EVOL_GFS) * Ntot;
+  const double *__restrict__ f = gfs + (size_t)gf * Ntot;
+  const int d = dest[p], F0 = face[3 * p], F1 = face[3 * p + 1], F2 = face[3 * p + 2];
+  const int i0 = d % N0, i1 = (d / N0) % N1, i2 = d / (N0 * N1);
+  const auto fa = [f, N0, N1](const int a, const int b, const int c) { return f[a + N0 * (b + N1 * c)]; };
+  const double char_speed = evolgf_speed[gf], var_at_infinity = evolgf_at_inf[gf];
+  double X[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const int j0 = i0 + q * F0, j1 = i1 + q * F1, j2 = i2 + q * F2;
+    const size_t at = (size_t)j0 + N0 * ((size_t)j1 + N1 * (size_t)j2);
+    const double g[5] = {geo[at], geo[Ntot + at], geo[2 * Ntot + at], geo[3 * Ntot + at], geo[4 * Ntot + at]};
+    const double invr = 1. / g[0];
+    X[q] = nrpy_sommerfeld_dfdr_from(params, g, fa, F0, F1, F2, j0, j1, j2) + invr * (fa(j0, j1, j2) - var_at_infinity);
+  }
+  R[(size_t)gf * Ntot + d] = -char_speed * X[0];
+  R[(size_t)(NUM_EVOL_GFS + gf) * Ntot + d] = char_speed * X[1];
+}
+
+// The chain of at most MAX steps: every operand is loaded before the first multiply-add.
+template <int MAX>
+__device__ __forceinline__ double nrpy_som_walk(const nrpy_fill_row row, const int *l, const int *F, const int n,
+                                                const int N0, const int N1, const size_t Ntot, const int gf,
+                                                const double *__restrict__ R) {
+  const double *__restrict__ A = R + (size_t)gf * Ntot;
+  const double *__restrict__ B = A + (size_t)NUM_EVOL_GFS * Ntot;
+  const double *__restrict__ r = R + (size_t)(2 * NUM_EVOL_GFS) * Ntot;
+  const double power = evolgf_radial_falloff_power[gf];
+  double a[MAX], b[MAX], rp[MAX + 1];
+  double ki = A[row.base];
+  rp[0] = r[row.base];
+  int at = row.base;
+#pragma unroll
+  for (int k = 0; k < MAX; k++) {
+    if (k < n) {
+      const int ax = nrpy_som_chain_axis(l[0], l[1], l[2], k);
+      at -= ax == 0 ? F[0] : ax == 1 ? F[1] * N0 : F[2] * N0 * N1;
+    }
+    a[k] = A[at];
+    b[k] = B[at];
+    rp[k + 1] = r[at];
+  }
+#pragma unroll
+  for (int k = 0; k < MAX; k++) {
+    const double invr = 1. / rp[k + 1];
+    const double next = power > 0 ? a[k] + (ki + b[k]) * nrpy_som_falloff(rp[k] * invr, power) : a[k];
+    ki = k < n ? next : ki;
+  }
+  return ki;
+}
+
+template <int S>
+__global__ void __launch_bounds__(256)
+nrpy_sommerfeld_chain_kernel(const paramstruct params, const int nrows, const nrpy_fill_row *__restrict__ rows,
+                             const nrpy_gf_parity_args gfp, const double *__restrict__ R, double *y_n, double *rt,
+                             double *out, const double dt) {
+  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x), gf = (int)blockIdx.y;
+  if (p >= nrows) return;
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1, N2 = params.Nxx_plus_2NGHOSTS2;
+  const size_t Ntot = (size_t)N0 * N1 * N2;
+  const nrpy_fill_row row = rows[p];
+  const size_t i = (size_t)gf * Ntot + row.dest;
+  const double yv = S < 3 ? y_n[i] : 0.0;
+  const double rv = S == 0 ? 0.0 : S < 3 ? rt[i] : y_n[i] + rt[i];
+  int l[3], F[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int c = (row.code >> (3 * d)) & 7;
+    l[d] = c > 3 ? c - 3 : c;
+    F[d] = c > 3 ? -1 : 1;
+  }
+  const int n = l[0] + l[1] + l[2];
+  double ki;
+  if (n == 0)
+    ki = R[(size_t)gf * Ntot + row.base];
+  else if (n <= NGHOSTS)
+    ki = nrpy_som_walk<NGHOSTS>(row, l, F, n, N0, N1, Ntot, gf, R);
+  else
+    ki = nrpy_som_walk<3 * NGHOSTS>(row, l, F, n, N0, N1, Ntot, gf, R);
+  if (row.negmask & (1 << gfp.p[gf])) ki = -ki;
+  if (S == 0) {
+    rt[i] = ki * dt * (1.0 / 6.0);
+    out[i] = yv + ki * dt * (1.0 / 2.0);
+  } else if (S == 1) {
+    rt[i] = rv + ki * dt * (1.0 / 3.0);
+    out[i] = yv + ki * dt * (1.0 / 2.0);
+  } else if (S == 2) {
+    rt[i] = rv + ki * dt * (1.0 / 3.0);
+    out[i] = yv + ki * dt;
+  } else {
+    out[i] = rv + ki * dt * (1.0 / 6.0);
+  }
+}
+
+// The geometry table, at the ghost points and the interior points next to them.
+__global__ void __launch_bounds__(256)
+nrpy_sommerfeld_geometry_kernel(const paramstruct params, const double *__restrict__ xx0,
+                                const double *__restrict__ xx1, const double *__restrict__ xx2,
+                                double *__restrict__ geo) {
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1, N2 = params.Nxx_plus_2NGHOSTS2;
+  const size_t Ntot = (size_t)N0 * N1 * N2, at = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (at >= Ntot) return;
+  const int i0 = (int)(at % N0), i1 = (int)((at / N0) % N1), i2 = (int)(at / ((size_t)N0 * N1));
+  if (i0 > NGHOSTS && i0 < N0 - 1 - NGHOSTS && i1 > NGHOSTS && i1 < N1 - 1 - NGHOSTS && i2 > NGHOSTS &&
+      i2 < N2 - 1 - NGHOSTS)
+    return;
+  double g[5];
+  nrpy_sommerfeld_geometry(params, xx0[i0], xx1[i1], xx2[i2], g);
+#pragma unroll
+  for (int k = 0; k < 5; k++) geo[k * Ntot + at] = g[k];
+}
+
+// Whether the two launches cover the grid's ghost points: each is an outer point or a copy of
+// an outer or interior point (no generic row), each outer point's FACE is the one its indices
+// give, and every interior point a chain or copy ends at lies within NGHOSTS of an edge.
+static bool nrpy_sommerfeld_chainable(const bc_struct *bc) {
+  const int *N = bc->N;
+  for (int gz = 0; gz < NGHOSTS; gz++)
+    for (const outer_bc &o : bc->outer[gz]) {
+      const int i[3] = {o.outer_bc_dest_pt.i0, o.outer_bc_dest_pt.i1, o.outer_bc_dest_pt.i2};
+      const int F[3] = {o.FACEi0, o.FACEi1, o.FACEi2};
+      int far = 0, axis = -1, sign = 0;
+      for (int d = 0; d < 3; d++) {
+        const int m = i[d] < NGHOSTS ? NGHOSTS - i[d] : i[d] >= N[d] - NGHOSTS ? i[d] - (N[d] - NGHOSTS - 1) : 0;
+        if (m > 0 && m >= far) {
+          far = m;
+          axis = d;
+          sign = i[d] < NGHOSTS ? 1 : -1;
+        }
+      }
+      for (int d = 0; d < 3; d++)
+        if (F[d] != (d == axis ? sign : 0)) return false;
+    }
+  for (const nrpy_fill_row &R : bc->fill_all.h_rows) {
+    if (R.code == NRPY_FILL_GENERIC) return false;
+    const int i[3] = {R.base % N[0], (R.base / N[0]) % N[1], R.base / (N[0] * N[1])};
+    bool rim = false;
+    for (int d = 0; d < 3; d++) rim = rim || i[d] < 2 * NGHOSTS || i[d] >= N[d] - 2 * NGHOSTS;
+    if (!rim) return false;
+  }
+  return true;
+}
+
+// Device memory of a captured step on the grid, its geometry table filled before this returns.
+// nullptr where the two launches do not cover the grid, or without memory: the caller takes
+// the unfused step.
+static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc,
+                                             hipStream_t stream) {
+  if (!params || !bc || !xx || !xx[0] || !xx[1] || !xx[2] || nrpy_check_params(params)) return nullptr;
+  if (bc->N[0] != params->Nxx_plus_2NGHOSTS0 || bc->N[1] != params->Nxx_plus_2NGHOSTS1 ||
+      bc->N[2] != params->Nxx_plus_2NGHOSTS2 || bc->N[0] < NRPY_SOMMERFELD_MIN_N || bc->N[1] < NRPY_SOMMERFELD_MIN_N ||
+      bc->N[2] < NRPY_SOMMERFELD_MIN_N || bc->fill_all.n == 0 || !nrpy_sommerfeld_chainable(bc))
+    return nullptr;
+  const size_t Ntot = (size_t)bc->N[0] * bc->N[1] * bc->N[2];
+  double *p = nullptr;
+  if (hipMalloc((void **)&p, sizeof(double) * NRPY_SOM_NSCRATCH * Ntot) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
+                     xx[0], xx[1], xx[2], p + 2 * NUM_EVOL_GFS * Ntot);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
+    (void)hipFree(p);
+    return nullptr;
+  }
+  return p;
+}
+
+static int nrpy_sommerfeld_chain(const int S, const paramstruct *params, const bc_struct *bc, const int8_t *gfs_parity,
+                                 double *R, double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
+  nrpy_gf_parity_args gfp;
+  memset(&gfp, 0, sizeof(gfp));
+  const int rc = nrpy_bc_check(params, bc, NUM_EVOL_GFS, gfs_parity, R, &gfp);
+  if (rc) return rc;
+  const nrpy_fill_list &L = bc->fill_all;
+  const int B = 64;
+  const dim3 grid((unsigned)((L.n + B - 1) / B), NUM_EVOL_GFS);
+  switch (S) {
+    case 0: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<0>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    case 1: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<1>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    case 2: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<2>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    default: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<3>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp,
+                                R, y_n, rt, out, dt); break;
   }
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
 }

@@ -77,7 +77,8 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
         "      !y_nplus1_running_total_gfs) return NRPY_ERR_NULL;\n"
         + ("  if (!auxevol_gfs) return NRPY_ERR_NULL;\n" if has_ricci else "") +
         "  int rc;\n" + steps + "  return NRPY_OK;\n}\n\n"
-        "struct MoL_graph {\n  hipGraph_t graph;\n  hipGraphExec_t exec;\n};\n"
+        "struct MoL_graph {\n  hipGraph_t graph;\n  hipGraphExec_t exec;\n"
+        "  double *scratch = nullptr;  // device memory of the captured step, owned by the graph\n};\n"
         "// Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed\n"
         "// at capture time.\n"
         'extern "C" int MoL_graph_create(' + sig + ", MoL_graph **out) {\n"
@@ -107,10 +108,11 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
         "    if (hipGraphLaunch(g->exec, stream) != hipSuccess) return NRPY_ERR_LAUNCH;\n"
         "  return NRPY_OK;\n}\n"
         'extern "C" void MoL_graph_free(MoL_graph *g) {\n'
-        "  if (!g) return;\n  (void)hipGraphExecDestroy(g->exec);\n  (void)hipGraphDestroy(g->graph);\n  delete g;\n}\n")
+        "  if (!g) return;\n  (void)hipGraphExecDestroy(g->exec);\n  (void)hipGraphDestroy(g->graph);\n"
+        "  (void)hipFree(g->scratch);\n  delete g;\n}\n")
 
 
-def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
+def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
     """Sommerfeld radiation condition (CurviBoundaryConditions.py:259-658) and the RK4 step of
     the Start-to-Finish drivers' BoundaryCondition = "Sommerfeld" branch
     (Tutorial-Start_to_Finish-Solving_Maxwells_Equations_in_Vacuum-Cartesian.ipynb:240-246):
@@ -124,8 +126,12 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
     points fused with their update, layer by layer (apply_bcs_sommerfeld_rk4). The values are
     those of the unfused step: the same RHS and update arithmetic at every point, only the
     separate all-points update pass is gone. Grids with inner boundary points, and a step
-    recorded into a graph before R exists, take the unfused step. Returns (HIP source,
-    per-gridfunction parameters for the meta)."""
+    recorded into a graph before R exists, take the unfused step.
+
+    With ``rim`` (the source of <fused kernel>_rim, curvilinear bundles) a captured step is two
+    launches per substep: the fused interior RHS + update, which leaves the RHS of the points
+    near the grid's edges in scratch memory that the graph owns and evaluates the radiation
+    condition's own terms at the outer points, and the chain kernel for every ghost point. Returns (HIP source, per-gridfunction parameters for the meta)."""
     from ..CurviBoundaryConditions import CurviBoundaryConditions as cbcs
     from ..MoLtimestepping import C_Code_Generation as MoL
     bcs = cbcs.sommerfeld_boundary_condition_class(fd_order=fd_order, **defaults)
@@ -157,6 +163,19 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
              'extern "C" int MoL_step_forward_in_time_sommerfeld(const paramstruct *params, %s, double *y_n_gfs, '
              "double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, "
              "hipStream_t stream) {\n%s}\n" % (sig, fused_body))
+    chain_body = ""
+    if rim is not None:
+        for S, (i, o) in enumerate((("y_n_gfs", "k_odd_gfs"), ("k_odd_gfs", "k_even_gfs"),
+                                    ("k_even_gfs", "k_odd_gfs"), ("k_odd_gfs", "y_n_gfs"))):
+            chain_body += ("  if ((rc = %s)) return rc;\n" % RIM_CALL.replace("IN", i).replace("OUT", o)
+                           .replace("SUBSTEP", str(S)) +
+                           "  if ((rc = nrpy_sommerfeld_chain(%d, params, bcstruct, evol_gf_parity, R, y_n_gfs, "
+                           "y_nplus1_running_total_gfs, %s, dt, stream))) return rc;\n" % (S, o))
+        step += ("// The same step as two launches per substep (values those of the unfused step); R:\n"
+                 "// the scratch of nrpy_sommerfeld_chain_scratch, not shared with a step on another stream.\n"
+                 "static int nrpy_sommerfeld_chain_step(const paramstruct *params, %s, double *y_n_gfs, double *k_odd_gfs, "
+                 "double *k_even_gfs, double *y_nplus1_running_total_gfs, double *R, const double dt, "
+                 "hipStream_t stream) {\n  int rc;\n%s  return NRPY_OK;\n}\n" % (sig, chain_body))
     meta = {"fd_order": fd_order, "at_inf": list(bcs.vars_at_infinity.values()),
             "radial_falloff_power": list(bcs.vars_radial_falloff_power.values()),
             "speed": list(bcs.vars_speed.values())}
@@ -175,11 +194,19 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
          "    if (!inner) (void)nrpy_sommerfeld_scratch(bcstruct, NUM_EVOL_GFS, s);\n"
          "  }\n" if shell_call is not None else "") +
         "  MoL_graph *g = new MoL_graph();\n"
-        "  int rc = NRPY_OK;\n"
+        "  int rc = NRPY_OK;\n" +
+        ("  // without scratch memory, or on a grid the chain kernel does not cover: the unfused step\n"
+         "  if (rfmstruct && y_n_gfs && k_odd_gfs && k_even_gfs && y_nplus1_running_total_gfs)\n"
+         "    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct, s);\n" if rim is not None else "") +
         "  if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = NRPY_ERR_LAUNCH;\n"
         "  if (!rc) {\n"
-        "    rc = MoL_step_forward_in_time_sommerfeld(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs, "
-        "k_even_gfs,\n                                             y_nplus1_running_total_gfs, dt, s);\n"
+        + ("    rc = g->scratch ? nrpy_sommerfeld_chain_step(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,\n"
+           "                                                 k_even_gfs, y_nplus1_running_total_gfs, g->scratch, dt, s)\n"
+           "                    : MoL_step_forward_in_time_sommerfeld(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,\n"
+           "                                                          k_even_gfs, y_nplus1_running_total_gfs, dt, s);\n"
+           if rim is not None else
+           "    rc = MoL_step_forward_in_time_sommerfeld(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs, "
+           "k_even_gfs,\n                                             y_nplus1_running_total_gfs, dt, s);\n") +
         "    hipGraph_t gr;\n"
         "    const hipError_t e = hipStreamEndCapture(s, &gr);\n"
         "    if (!rc && e != hipSuccess) rc = NRPY_ERR_LAUNCH;\n"
@@ -189,9 +216,9 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, **defaults):
         "    }\n"
         "  }\n"
         "  (void)hipStreamDestroy(s);\n"
-        "  if (rc) { delete g; return rc; }\n"
+        "  if (rc) { (void)hipFree(g->scratch); delete g; return rc; }\n"
         "  *out = g;\n  return NRPY_OK;\n}\n")
-    return ("// One RK4 step with the Sommerfeld radiation condition on the RHS.\n" + bcs.hip_source() + step + graph,
+    return ("// One RK4 step with the Sommerfeld radiation condition on the RHS.\n" + bcs.hip_source(chain=rim is not None) + (rim or "") + step + graph,
             meta)
 
 
@@ -361,6 +388,54 @@ def _fused_shell_kernel(fused_kernel, name):
              "".join("    xb[(size_t)%sGF * 2 * Nxx_plus_2NGHOSTS1 * Nxx_plus_2NGHOSTS2] = __rhs_%s;\n" % (g, g)
                      for g in stores) + "  }")
     return k[:last] + block + k[last:]
+
+
+# the two-launch Sommerfeld step's interior substep in the curvilinear bundles
+RIM_CALL = ("rhs_eval_rk4_substep_rim(SUBSTEP, rfmstruct, params, bcstruct, nullptr, IN, y_n_gfs, "
+            "y_nplus1_running_total_gfs, OUT, R, dt, stream)")
+
+
+def _fused_rim(fused_kernel, name, args_sig, call_args):
+    """The fused RHS + RK4 kernel ``name`` as ``<name>_rim`` with its launcher: the same computation,
+    and at the interior points within NGHOSTS of an edge of the grid (those that the ghost points'
+    chains and parity copies end at) it also stores each RHS into rim_rhs. Blocks after the
+    first rim_blocks evaluate the radiation condition's terms at the outer points."""
+    i = fused_kernel.index("%s__gpu(" % name)
+    start = fused_kernel.rindex("template <int S>", 0, i)
+    end = fused_kernel.index("\n}\n", i) + 3
+    k = fused_kernel[start:end].replace("%s__gpu(" % name, "%s_rim__gpu(" % name, 1)
+    k = k.replace("const double dt) {", "const double dt, double *rim_rhs, const int rim_blocks, const int rim_n, "
+                  "const int *__restrict__ rim_dest, const int8_t *__restrict__ rim_face) {\n"
+                  "  if ((int)blockIdx.x >= rim_blocks) {\n"
+                  "    const int nrpy_t = (int)threadIdx.x + (int)blockDim.x * ((int)threadIdx.y + "
+                  "(int)blockDim.y * (int)threadIdx.z);\n"
+                  "    nrpy_sommerfeld_eval(params, (size_t)((int)blockIdx.x - rim_blocks) * (blockDim.x * blockDim.y * "
+                  "blockDim.z) + nrpy_t, rim_n, rim_dest, rim_face, in_gfs, rim_rhs);\n"
+                  "    return;\n  }", 1)
+    if k.count("NRPY_BLOCK_COORDS(") != 1:
+        raise ValueError("%s: one NRPY_BLOCK_COORDS expected" % name)
+    k = k.replace("NRPY_BLOCK_COORDS(", "NRPY_BLOCK_COORDS_OF(rim_blocks, ", 1)
+    found = list(re.finditer(r"NRPY_RK4_STORE\(S, \d+, __rhs_(\w+)\);", k))
+    block = ("\n  if (i0 < 2*NGHOSTS || i0 >= Nxx0 || i1 < 2*NGHOSTS || i1 >= Nxx1 || i2 < 2*NGHOSTS || i2 >= Nxx2) {\n" +
+             "".join("    rim_rhs[IDX4(%sGF, i0, i1, i2)] = __rhs_%s;\n" % (m.group(1), m.group(1)) for m in found) + "  }")
+    k = k[:found[-1].end()] + block + k[found[-1].end():]
+    kid = bd.lp.kernel_id(name)
+    cases = "".join(
+        "    case %d: hipLaunchKernelGGL(%s_rim__gpu<%d>, grid, block, 0, stream, %s, y_n, rt, out, dt, rim_rhs, "
+        "(int)nb, n, bc->d_ob_dest, bc->d_ob_face); break;\n" % (s, name, s, call_args) for s in range(4))
+    return k + ('static int %s_rim(const int S, %s, double *y_n, double *rt, double *out, double *rim_rhs, '
+                "const double dt, hipStream_t stream) {\n"
+                "  if (!params || !bc || !y_n || !rt || !out || !rim_rhs) return NRPY_ERR_NULL;\n"
+                "  if (S < 0 || S > 3) return NRPY_ERR_PARAM;\n"
+                "  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;\n"
+                "  const dim3 block = nrpy_block(%d, %d, %d, %d);\n"
+                "  const unsigned nb = nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2);\n"
+                "  const int n = bc->ob_off[NGHOSTS];\n"
+                "  const size_t threads = (size_t)block.x * block.y * block.z;\n"
+                "  const dim3 grid(nb + (unsigned)(((size_t)n * NUM_EVOL_GFS + threads - 1) / threads));\n"
+                "  switch (S) {\n%s  }\n"
+                "  return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;\n}\n"
+                % (name, args_sig, kid, bd.lp.BLOCK_X, bd.lp.BLOCK_Y, bd.lp.BLOCK_Z, cases))
 
 
 def _fused_shell_launcher(name, args_sig, call_args):
@@ -632,6 +707,9 @@ def scalarwave_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
     fused += _fused_launcher("rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
                              "const double *auxevol_gfs, const double *in_gfs",
                              "*params, *rfmstruct, auxevol_gfs, in_gfs", "InteriorPoints")
+    rim = _fused_rim(fused, "rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
+                     "const bc_struct *bc, const double *auxevol_gfs, const double *in_gfs",
+                     "*params, *rfmstruct, auxevol_gfs, in_gfs")
     rfm_code = bd.rfm_struct_code()
     tables = [(n, str(e), list(a)) for n, e, a in rfm.rfm_precompute_tables()]
     par.set_parval_from_str("reference_metric::enable_rfm_precompute", "False")
@@ -640,7 +718,8 @@ def scalarwave_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
     # The EigenCoord's reference metric registers its own C parameters (e.g. RMAX), so
     # the coordinate functions are generated before the paramstruct is declared.
     coords = bd.coord_host_functions(CoordSystem)
-    som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)")
+    som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
+                                         rim=rim)
     pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code,
              rhs_src, fused, id_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]
@@ -700,13 +779,17 @@ def maxwell_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
     fused += _fused_launcher("rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
                              "const double *auxevol_gfs, const double *in_gfs",
                              "*params, *rfmstruct, auxevol_gfs, in_gfs", "InteriorPoints")
+    rim = _fused_rim(fused, "rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
+                     "const bc_struct *bc, const double *auxevol_gfs, const double *in_gfs",
+                     "*params, *rfmstruct, auxevol_gfs, in_gfs")
     rfm_code = bd.rfm_struct_code()
     tables = [(n, str(e), list(a)) for n, e, a in rfm.rfm_precompute_tables()]
     par.set_parval_from_str("reference_metric::enable_rfm_precompute", "False")
     rfm.ref_metric__hatted_quantities()
     id_src = _initial_data_kernel(id_rhss, id_names)
     coords = bd.coord_host_functions(CoordSystem)
-    som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)")
+    som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(rfmstruct, params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
+                                         rim=rim)
     pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code, rhs_src, con_src, fused, id_src,
              _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]

@@ -1066,6 +1066,7 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
 struct MoL_graph {
   hipGraph_t graph;
   hipGraphExec_t exec;
+  double *scratch = nullptr;  // device memory of the captured step, owned by the graph
 };
 // Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed
 // at capture time.
@@ -1104,6 +1105,7 @@ extern "C" void MoL_graph_free(MoL_graph *g) {
   if (!g) return;
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
+  (void)hipFree(g->scratch);
   delete g;
 }
 
@@ -1653,7 +1655,7 @@ extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_
     }
   }
   (void)hipStreamDestroy(s);
-  if (rc) { delete g; return rc; }
+  if (rc) { (void)hipFree(g->scratch); delete g; return rc; }
   *out = g;
   return NRPY_OK;
 }

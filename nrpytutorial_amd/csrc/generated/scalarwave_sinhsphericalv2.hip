@@ -509,6 +509,7 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
 struct MoL_graph {
   hipGraph_t graph;
   hipGraphExec_t exec;
+  double *scratch = nullptr;  // device memory of the captured step, owned by the graph
 };
 // Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed
 // at capture time.
@@ -547,6 +548,7 @@ extern "C" void MoL_graph_free(MoL_graph *g) {
   if (!g) return;
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
+  (void)hipFree(g->scratch);
   delete g;
 }
 
@@ -557,23 +559,42 @@ static __constant__ double evolgf_radial_falloff_power[NUM_EVOL_GFS] = {3.0, 3.0
 static __constant__ double evolgf_speed[NUM_EVOL_GFS] = {1.0, 1.0};
 #define NRPY_SOMMERFELD_MIN_N (NGHOSTS + 4 + 1)
 #define NRPY_SOMMERFELD_FD 4
-// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's
-// FACE (CurviBoundaryConditions.py:329-516).
-template <typename FA>
-static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, double *dfdr_out) {
+// r and the radial derivative's geometry at a point: geo = r, then a_i and b of
+// d f/d r = sum_i fdD_i a_i / b.
+static __device__ void nrpy_sommerfeld_geometry(const paramstruct &params, const double xx0, const double xx1, const double xx2, double *geo) {
   const double AMPL = params.AMPL;
+  const double SINHW = params.SINHW;
+  const double const_dr = params.const_dr;
+  (void)xx0; (void)xx1; (void)xx2;
+  double J00, J01, J02, J10, J11, J12, J20, J21, J22;
+  const double tmp_0 = (1.0/((SINHW)));
+  const double tmp_1 = (1.0/((exp(tmp_0) - exp(-tmp_0))));
+  const double tmp_2 = tmp_0*xx0;
+  const double tmp_3 = exp(tmp_2);
+  const double tmp_4 = exp(-tmp_2);
+  geo[0] = AMPL*(const_dr*xx0 + tmp_1*(tmp_3 - tmp_4));
+  J00 = AMPL*(const_dr + tmp_1*(tmp_0*tmp_3 + tmp_0*tmp_4));
+  J01 = 0;
+  J02 = 0;
+  J10 = 0;
+  J11 = 1;
+  J12 = 0;
+  J20 = 0;
+  J21 = 0;
+  J22 = 1;
+  const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;
+  geo[1] = cof0; geo[2] = cof1; geo[3] = cof2;
+  geo[4] = J00*cof0 + J01*cof1 + J02*cof2;
+}
+template <typename FA>
+static __device__ double nrpy_sommerfeld_dfdr_from(const paramstruct &params, const double *geo, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2) {
   const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
   const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
   const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
-  const double SINHW = params.SINHW;
-  const double const_dr = params.const_dr;
   const double invdx0 = params.invdx0;
   const double invdx1 = params.invdx1;
   const double invdx2 = params.invdx2;
-  const double xx0 = xx0_arr[i0], xx1 = xx1_arr[i1], xx2 = xx2_arr[i2];
-  (void)xx0; (void)xx1; (void)xx2; (void)F0; (void)F1; (void)F2;
   double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;
-  (void)fdD0; (void)fdD1; (void)fdD2;
   const double u0 = -25./12., u1 = 4., u2 = -3., u3 = 4./3., u4 = -1./4.;
   const double c1 = 2./3., c2 = 1./12.;
   {
@@ -606,24 +627,19 @@ static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const d
     const double cen = (-c2*fa(i0,i1,nrpy_ic2+2) + c1*fa(i0,i1,nrpy_ic2+1) - c1*fa(i0,i1,nrpy_ic2+-1) + c2*fa(i0,i1,nrpy_ic2+-2))*invdx2;
     fdD2 = one_sided ? one : cen;
   }
-  double J00, J01, J02, J10, J11, J12, J20, J21, J22;
-  const double tmp_0 = (1.0/((SINHW)));
-  const double tmp_1 = (1.0/((exp(tmp_0) - exp(-tmp_0))));
-  const double tmp_2 = tmp_0*xx0;
-  const double tmp_3 = exp(tmp_2);
-  const double tmp_4 = exp(-tmp_2);
-  *r_out = AMPL*(const_dr*xx0 + tmp_1*(tmp_3 - tmp_4));
-  J00 = AMPL*(const_dr + tmp_1*(tmp_0*tmp_3 + tmp_0*tmp_4));
-  J01 = 0;
-  J02 = 0;
-  J10 = 0;
-  J11 = 1;
-  J12 = 0;
-  J20 = 0;
-  J21 = 0;
-  J22 = 1;
-  const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;
-  *dfdr_out = (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/(J00*cof0 + J01*cof1 + J02*cof2);
+  const double cof0 = geo[1], cof1 = geo[2], cof2 = geo[3];
+  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];
+}
+// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's
+// FACE (CurviBoundaryConditions.py:329-516).
+template <typename FA>
+static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, double *dfdr_out) {
+  double geo[5];
+  nrpy_sommerfeld_geometry(params, xx0_arr[i0], xx1_arr[i1], xx2_arr[i2], geo);
+#pragma unroll
+  for (int k = 0; k < 5; k++) asm("" : "+v"(geo[k]));
+  *r_out = geo[0];
+  *dfdr_out = nrpy_sommerfeld_dfdr_from(params, geo, fa, F0, F1, F2, i0, i1, i2);
 }
 
 // The radiation condition's right-hand side at outer point (i0,i1,i2) of gridfunction gf
@@ -1010,6 +1026,327 @@ extern "C" int apply_bcs_sommerfeld(const paramstruct *params, double *xx[3], co
   }
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
 }
+
+// The whole condition in two launches per substep, for grids with inner boundary points. The
+// reference's order (layer by layer, face group by face group, then the parity copies) makes a
+// chain of each outer point: its RHS is
+//   rhs_p = A_p + (rhs_q + B_p) (r_q / r_p)^n,   q its inward neighbour (an interior point, or an
+// outer point one step further in), A_p = -v X_p, B_p = v X_q, X = d f/d r + (f - f_inf)/r with
+// the stencils of p's FACE. A and B need only the state the substep starts from, so they are
+// evaluated for every outer point at once, in extra blocks of the interior RHS launch
+// (nrpy_sommerfeld_eval); the second launch (nrpy_sommerfeld_chain_kernel) walks each ghost
+// point's chain from the interior out, at most 3 NGHOSTS multiply-adds, an inner point that of
+// the point it copies, and does the RK4 update there. Every point's FACE follows from its
+// indices: the axis with the largest distance outside the interior, the last of equals
+// (nrpy_sommerfeld_chainable checks it against the lists). The arithmetic is that of
+// nrpy_sommerfeld_rhs.
+// Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
+// launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
+// chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table
+// (geo, 5 values per point, written once per captured step) instead of the Jacobian.
+// Scratch of a captured step: R, NUM_EVOL_GFS gridfunctions: the RHS at the interior points a
+// chain or copy ends at (rhs_eval_rk4_substep_rim), A at the outer points; then B, as many; then geo.
+#define NRPY_SOM_NSCRATCH (2 * NUM_EVOL_GFS + 5)
+
+// Step k of n (k = 0 the innermost) of the chain with layers l: its axis.
+__device__ __forceinline__ int nrpy_som_chain_axis(const int l0, const int l1, const int l2, const int k) {
+  int m0 = l0, m1 = l1, m2 = l2, a = 0;
+  for (int j = l0 + l1 + l2 - 1; j >= k; j--) {
+    const int far = max(m0, max(m1, m2));
+    a = m2 == far ? 2 : m1 == far ? 1 : 0;
+    m0 -= a == 0;
+    m1 -= a == 1;
+    m2 -= a == 2;
+  }
+  return a;
+}
+
+// A and B at outer point number t % n of the lists (all layers) of gridfunction t / n.
+__device__ __forceinline__ void nrpy_sommerfeld_eval(const paramstruct &params, const size_t t, const int n,
+                                                     const int *__restrict__ dest, const int8_t *__restrict__ face,
+                                                     const double *__restrict__ gfs, double *__restrict__ R) {
+  if (t >= (size_t)n * NUM_EVOL_GFS) return;
+  const int gf = (int)(t / n), p = (int)(t % n);
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1;
+  const size_t Ntot = (size_t)N0 * N1 * params.Nxx_plus_2NGHOSTS2;
+  const double *__restrict__ geo = R + (size_t)(2 * NUM_EVOL_GFS) * Ntot;
+  const double *__restrict__ f = gfs + (size_t)gf * Ntot;
+  const int d = dest[p], F0 = face[3 * p], F1 = face[3 * p + 1], F2 = face[3 * p + 2];
+  const int i0 = d % N0, i1 = (d / N0) % N1, i2 = d / (N0 * N1);
+  const auto fa = [f, N0, N1](const int a, const int b, const int c) { return f[a + N0 * (b + N1 * c)]; };
+  const double char_speed = evolgf_speed[gf], var_at_infinity = evolgf_at_inf[gf];
+  double X[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const int j0 = i0 + q * F0, j1 = i1 + q * F1, j2 = i2 + q * F2;
+    const size_t at = (size_t)j0 + N0 * ((size_t)j1 + N1 * (size_t)j2);
+    const double g[5] = {geo[at], geo[Ntot + at], geo[2 * Ntot + at], geo[3 * Ntot + at], geo[4 * Ntot + at]};
+    const double invr = 1. / g[0];
+    X[q] = nrpy_sommerfeld_dfdr_from(params, g, fa, F0, F1, F2, j0, j1, j2) + invr * (fa(j0, j1, j2) - var_at_infinity);
+  }
+  R[(size_t)gf * Ntot + d] = -char_speed * X[0];
+  R[(size_t)(NUM_EVOL_GFS + gf) * Ntot + d] = char_speed * X[1];
+}
+
+// The chain of at most MAX steps: every operand is loaded before the first multiply-add.
+template <int MAX>
+__device__ __forceinline__ double nrpy_som_walk(const nrpy_fill_row row, const int *l, const int *F, const int n,
+                                                const int N0, const int N1, const size_t Ntot, const int gf,
+                                                const double *__restrict__ R) {
+  const double *__restrict__ A = R + (size_t)gf * Ntot;
+  const double *__restrict__ B = A + (size_t)NUM_EVOL_GFS * Ntot;
+  const double *__restrict__ r = R + (size_t)(2 * NUM_EVOL_GFS) * Ntot;
+  const double power = evolgf_radial_falloff_power[gf];
+  double a[MAX], b[MAX], rp[MAX + 1];
+  double ki = A[row.base];
+  rp[0] = r[row.base];
+  int at = row.base;
+#pragma unroll
+  for (int k = 0; k < MAX; k++) {
+    if (k < n) {
+      const int ax = nrpy_som_chain_axis(l[0], l[1], l[2], k);
+      at -= ax == 0 ? F[0] : ax == 1 ? F[1] * N0 : F[2] * N0 * N1;
+    }
+    a[k] = A[at];
+    b[k] = B[at];
+    rp[k + 1] = r[at];
+  }
+#pragma unroll
+  for (int k = 0; k < MAX; k++) {
+    const double invr = 1. / rp[k + 1];
+    const double next = power > 0 ? a[k] + (ki + b[k]) * nrpy_som_falloff(rp[k] * invr, power) : a[k];
+    ki = k < n ? next : ki;
+  }
+  return ki;
+}
+
+template <int S>
+__global__ void __launch_bounds__(256)
+nrpy_sommerfeld_chain_kernel(const paramstruct params, const int nrows, const nrpy_fill_row *__restrict__ rows,
+                             const nrpy_gf_parity_args gfp, const double *__restrict__ R, double *y_n, double *rt,
+                             double *out, const double dt) {
+  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x), gf = (int)blockIdx.y;
+  if (p >= nrows) return;
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1, N2 = params.Nxx_plus_2NGHOSTS2;
+  const size_t Ntot = (size_t)N0 * N1 * N2;
+  const nrpy_fill_row row = rows[p];
+  const size_t i = (size_t)gf * Ntot + row.dest;
+  const double yv = S < 3 ? y_n[i] : 0.0;
+  const double rv = S == 0 ? 0.0 : S < 3 ? rt[i] : y_n[i] + rt[i];
+  int l[3], F[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int c = (row.code >> (3 * d)) & 7;
+    l[d] = c > 3 ? c - 3 : c;
+    F[d] = c > 3 ? -1 : 1;
+  }
+  const int n = l[0] + l[1] + l[2];
+  double ki;
+  if (n == 0)
+    ki = R[(size_t)gf * Ntot + row.base];
+  else if (n <= NGHOSTS)
+    ki = nrpy_som_walk<NGHOSTS>(row, l, F, n, N0, N1, Ntot, gf, R);
+  else
+    ki = nrpy_som_walk<3 * NGHOSTS>(row, l, F, n, N0, N1, Ntot, gf, R);
+  if (row.negmask & (1 << gfp.p[gf])) ki = -ki;
+  if (S == 0) {
+    rt[i] = ki * dt * (1.0 / 6.0);
+    out[i] = yv + ki * dt * (1.0 / 2.0);
+  } else if (S == 1) {
+    rt[i] = rv + ki * dt * (1.0 / 3.0);
+    out[i] = yv + ki * dt * (1.0 / 2.0);
+  } else if (S == 2) {
+    rt[i] = rv + ki * dt * (1.0 / 3.0);
+    out[i] = yv + ki * dt;
+  } else {
+    out[i] = rv + ki * dt * (1.0 / 6.0);
+  }
+}
+
+// The geometry table, at the ghost points and the interior points next to them.
+__global__ void __launch_bounds__(256)
+nrpy_sommerfeld_geometry_kernel(const paramstruct params, const double *__restrict__ xx0,
+                                const double *__restrict__ xx1, const double *__restrict__ xx2,
+                                double *__restrict__ geo) {
+  const int N0 = params.Nxx_plus_2NGHOSTS0, N1 = params.Nxx_plus_2NGHOSTS1, N2 = params.Nxx_plus_2NGHOSTS2;
+  const size_t Ntot = (size_t)N0 * N1 * N2, at = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (at >= Ntot) return;
+  const int i0 = (int)(at % N0), i1 = (int)((at / N0) % N1), i2 = (int)(at / ((size_t)N0 * N1));
+  if (i0 > NGHOSTS && i0 < N0 - 1 - NGHOSTS && i1 > NGHOSTS && i1 < N1 - 1 - NGHOSTS && i2 > NGHOSTS &&
+      i2 < N2 - 1 - NGHOSTS)
+    return;
+  double g[5];
+  nrpy_sommerfeld_geometry(params, xx0[i0], xx1[i1], xx2[i2], g);
+#pragma unroll
+  for (int k = 0; k < 5; k++) geo[k * Ntot + at] = g[k];
+}
+
+// Whether the two launches cover the grid's ghost points: each is an outer point or a copy of
+// an outer or interior point (no generic row), each outer point's FACE is the one its indices
+// give, and every interior point a chain or copy ends at lies within NGHOSTS of an edge.
+static bool nrpy_sommerfeld_chainable(const bc_struct *bc) {
+  const int *N = bc->N;
+  for (int gz = 0; gz < NGHOSTS; gz++)
+    for (const outer_bc &o : bc->outer[gz]) {
+      const int i[3] = {o.outer_bc_dest_pt.i0, o.outer_bc_dest_pt.i1, o.outer_bc_dest_pt.i2};
+      const int F[3] = {o.FACEi0, o.FACEi1, o.FACEi2};
+      int far = 0, axis = -1, sign = 0;
+      for (int d = 0; d < 3; d++) {
+        const int m = i[d] < NGHOSTS ? NGHOSTS - i[d] : i[d] >= N[d] - NGHOSTS ? i[d] - (N[d] - NGHOSTS - 1) : 0;
+        if (m > 0 && m >= far) {
+          far = m;
+          axis = d;
+          sign = i[d] < NGHOSTS ? 1 : -1;
+        }
+      }
+      for (int d = 0; d < 3; d++)
+        if (F[d] != (d == axis ? sign : 0)) return false;
+    }
+  for (const nrpy_fill_row &R : bc->fill_all.h_rows) {
+    if (R.code == NRPY_FILL_GENERIC) return false;
+    const int i[3] = {R.base % N[0], (R.base / N[0]) % N[1], R.base / (N[0] * N[1])};
+    bool rim = false;
+    for (int d = 0; d < 3; d++) rim = rim || i[d] < 2 * NGHOSTS || i[d] >= N[d] - 2 * NGHOSTS;
+    if (!rim) return false;
+  }
+  return true;
+}
+
+// Device memory of a captured step on the grid, its geometry table filled before this returns.
+// nullptr where the two launches do not cover the grid, or without memory: the caller takes
+// the unfused step.
+static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc,
+                                             hipStream_t stream) {
+  if (!params || !bc || !xx || !xx[0] || !xx[1] || !xx[2] || nrpy_check_params(params)) return nullptr;
+  if (bc->N[0] != params->Nxx_plus_2NGHOSTS0 || bc->N[1] != params->Nxx_plus_2NGHOSTS1 ||
+      bc->N[2] != params->Nxx_plus_2NGHOSTS2 || bc->N[0] < NRPY_SOMMERFELD_MIN_N || bc->N[1] < NRPY_SOMMERFELD_MIN_N ||
+      bc->N[2] < NRPY_SOMMERFELD_MIN_N || bc->fill_all.n == 0 || !nrpy_sommerfeld_chainable(bc))
+    return nullptr;
+  const size_t Ntot = (size_t)bc->N[0] * bc->N[1] * bc->N[2];
+  double *p = nullptr;
+  if (hipMalloc((void **)&p, sizeof(double) * NRPY_SOM_NSCRATCH * Ntot) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
+                     xx[0], xx[1], xx[2], p + 2 * NUM_EVOL_GFS * Ntot);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
+    (void)hipFree(p);
+    return nullptr;
+  }
+  return p;
+}
+
+static int nrpy_sommerfeld_chain(const int S, const paramstruct *params, const bc_struct *bc, const int8_t *gfs_parity,
+                                 double *R, double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
+  nrpy_gf_parity_args gfp;
+  memset(&gfp, 0, sizeof(gfp));
+  const int rc = nrpy_bc_check(params, bc, NUM_EVOL_GFS, gfs_parity, R, &gfp);
+  if (rc) return rc;
+  const nrpy_fill_list &L = bc->fill_all;
+  const int B = 64;
+  const dim3 grid((unsigned)((L.n + B - 1) / B), NUM_EVOL_GFS);
+  switch (S) {
+    case 0: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<0>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    case 1: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<1>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    case 2: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<2>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp, R,
+                               y_n, rt, out, dt); break;
+    default: hipLaunchKernelGGL(nrpy_sommerfeld_chain_kernel<3>, grid, dim3(B), 0, stream, *params, L.n, L.d_rows, gfp,
+                                R, y_n, rt, out, dt); break;
+  }
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+template <int S>
+__global__ void __launch_bounds__(256) rhs_eval_rk4_substep_rim__gpu(const paramstruct params, const rfm_struct rfmstruct, const double *__restrict__ auxevol_gfs, const double *__restrict__ in_gfs, double *rk_yn, double *rk_rt, double *rk_out, const double dt, double *rim_rhs, const int rim_blocks, const int rim_n, const int *__restrict__ rim_dest, const int8_t *__restrict__ rim_face) {
+  if ((int)blockIdx.x >= rim_blocks) {
+    const int nrpy_t = (int)threadIdx.x + (int)blockDim.x * ((int)threadIdx.y + (int)blockDim.y * (int)threadIdx.z);
+    nrpy_sommerfeld_eval(params, (size_t)((int)blockIdx.x - rim_blocks) * (blockDim.x * blockDim.y * blockDim.z) + nrpy_t, rim_n, rim_dest, rim_face, in_gfs, rim_rhs);
+    return;
+  }
+  const int Nxx0 = params.Nxx0;
+  const int Nxx1 = params.Nxx1;
+  const int Nxx2 = params.Nxx2;
+  const double invdx0 = params.invdx0;
+  const double invdx1 = params.invdx1;
+  const double invdx2 = params.invdx2;
+  const double wavespeed = params.wavespeed;
+  const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
+  const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
+  const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
+  NRPY_BLOCK_COORDS_OF(rim_blocks, Nxx0, Nxx1, Nxx2);
+  const int i0 = NGHOSTS + nrpy_bx*(int)blockDim.x + (int)threadIdx.x;
+  const int i1 = NGHOSTS + nrpy_by*(int)blockDim.y + (int)threadIdx.y;
+  const int i2 = NGHOSTS + nrpy_bz*(int)blockDim.z + (int)threadIdx.z;
+  if (i0 >= Nxx0 + NGHOSTS || i1 >= Nxx1 + NGHOSTS || i2 >= Nxx2 + NGHOSTS) return;
+  const double f0_of_xx0 = rfmstruct.f0_of_xx0[i0];
+  const double f0_of_xx0__D0 = rfmstruct.f0_of_xx0__D0[i0];
+  const double f0_of_xx0__DD00 = rfmstruct.f0_of_xx0__DD00[i0];
+  const double f1_of_xx1 = rfmstruct.f1_of_xx1[i1];
+  const double f1_of_xx1__D1 = rfmstruct.f1_of_xx1__D1[i1];
+  {
+    /* Step 1 of 2: read gridfunctions and compute finite-difference stencils */
+    const double uu_i0_i1_i2m2 = in_gfs[IDX4(UUGF, i0,i1,i2-2)];
+    const double uu_i0_i1_i2m1 = in_gfs[IDX4(UUGF, i0,i1,i2-1)];
+    const double uu_i0_i1m2_i2 = in_gfs[IDX4(UUGF, i0,i1-2,i2)];
+    const double uu_i0_i1m1_i2 = in_gfs[IDX4(UUGF, i0,i1-1,i2)];
+    const double uu_i0m2_i1_i2 = in_gfs[IDX4(UUGF, i0-2,i1,i2)];
+    const double uu_i0m1_i1_i2 = in_gfs[IDX4(UUGF, i0-1,i1,i2)];
+    const double uu = in_gfs[IDX4(UUGF, i0,i1,i2)];
+    const double uu_i0p1_i1_i2 = in_gfs[IDX4(UUGF, i0+1,i1,i2)];
+    const double uu_i0p2_i1_i2 = in_gfs[IDX4(UUGF, i0+2,i1,i2)];
+    const double uu_i0_i1p1_i2 = in_gfs[IDX4(UUGF, i0,i1+1,i2)];
+    const double uu_i0_i1p2_i2 = in_gfs[IDX4(UUGF, i0,i1+2,i2)];
+    const double uu_i0_i1_i2p1 = in_gfs[IDX4(UUGF, i0,i1,i2+1)];
+    const double uu_i0_i1_i2p2 = in_gfs[IDX4(UUGF, i0,i1,i2+2)];
+    const double vv = in_gfs[IDX4(VVGF, i0,i1,i2)];
+    const double FDPart1_Rational_1_12 = 1.0/12.0;
+    const double FDPart1_Rational_2_3 = 2.0/3.0;
+    const double FDPart1_Rational_4_3 = 4.0/3.0;
+    const double FDPart1_Rational_m1_12 = -1.0/12.0;
+    const double FDPart1_Rational_m2_3 = -2.0/3.0;
+    const double FDPart1_Rational_m5_2 = -5.0/2.0;
+    const double FDPart1_0 = FDPart1_Rational_m1_12*uu_i0p2_i1_i2;
+    const double FDPart1_1 = FDPart1_Rational_m1_12*uu_i0_i1p2_i2;
+    const double FDPart1_2 = FDPart1_Rational_m5_2*uu;
+    const double uu_dD0 = invdx0*(FDPart1_0 + FDPart1_Rational_1_12*uu_i0m2_i1_i2 + FDPart1_Rational_2_3*uu_i0p1_i1_i2 + FDPart1_Rational_m2_3*uu_i0m1_i1_i2);
+    const double uu_dD1 = invdx1*(FDPart1_1 + FDPart1_Rational_1_12*uu_i0_i1m2_i2 + FDPart1_Rational_2_3*uu_i0_i1p1_i2 + FDPart1_Rational_m2_3*uu_i0_i1m1_i2);
+    const double uu_dDD00 = ((invdx0)*(invdx0))*(FDPart1_0 + FDPart1_2 + FDPart1_Rational_4_3*uu_i0m1_i1_i2 + FDPart1_Rational_4_3*uu_i0p1_i1_i2 + FDPart1_Rational_m1_12*uu_i0m2_i1_i2);
+    const double uu_dDD11 = ((invdx1)*(invdx1))*(FDPart1_1 + FDPart1_2 + FDPart1_Rational_4_3*uu_i0_i1m1_i2 + FDPart1_Rational_4_3*uu_i0_i1p1_i2 + FDPart1_Rational_m1_12*uu_i0_i1m2_i2);
+    const double uu_dDD22 = ((invdx2)*(invdx2))*(FDPart1_2 + FDPart1_Rational_4_3*uu_i0_i1_i2m1 + FDPart1_Rational_4_3*uu_i0_i1_i2p1 + FDPart1_Rational_m1_12*uu_i0_i1_i2m2 + FDPart1_Rational_m1_12*uu_i0_i1_i2p2);
+    /* Step 2 of 2: evaluate right-hand sides and write to memory */
+    const double FDPart3_0 = (1.0/((f0_of_xx0)*(f0_of_xx0)));
+  const double __rhs_UU = vv;
+  const double __rhs_VV = ((wavespeed)*(wavespeed))*(FDPart3_0*uu_dDD11 + FDPart3_0*f1_of_xx1__D1*uu_dD1/f1_of_xx1 + FDPart3_0*uu_dDD22/((f1_of_xx1)*(f1_of_xx1)) - uu_dD0*(f0_of_xx0__DD00/((f0_of_xx0__D0)*(f0_of_xx0__D0)*(f0_of_xx0__D0)) - 2/(f0_of_xx0*f0_of_xx0__D0)) + uu_dDD00/((f0_of_xx0__D0)*(f0_of_xx0__D0)));
+  __builtin_amdgcn_sched_barrier(0);
+  NRPY_RK4_PRELOAD(S, UUGF, 0)
+  NRPY_RK4_PRELOAD(S, VVGF, 1)
+  NRPY_RK4_STORE(S, 0, __rhs_UU);
+  NRPY_RK4_STORE(S, 1, __rhs_VV);
+  if (i0 < 2*NGHOSTS || i0 >= Nxx0 || i1 < 2*NGHOSTS || i1 >= Nxx1 || i2 < 2*NGHOSTS || i2 >= Nxx2) {
+    rim_rhs[IDX4(UUGF, i0, i1, i2)] = __rhs_UU;
+    rim_rhs[IDX4(VVGF, i0, i1, i2)] = __rhs_VV;
+  }
+  }
+}
+static int rhs_eval_rk4_substep_rim(const int S, const rfm_struct *rfmstruct, const paramstruct *params, const bc_struct *bc, const double *auxevol_gfs, const double *in_gfs, double *y_n, double *rt, double *out, double *rim_rhs, const double dt, hipStream_t stream) {
+  if (!params || !bc || !y_n || !rt || !out || !rim_rhs) return NRPY_ERR_NULL;
+  if (S < 0 || S > 3) return NRPY_ERR_PARAM;
+  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
+  const dim3 block = nrpy_block(1, 64, 1, 4);
+  const unsigned nb = nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2);
+  const int n = bc->ob_off[NGHOSTS];
+  const size_t threads = (size_t)block.x * block.y * block.z;
+  const dim3 grid(nb + (unsigned)(((size_t)n * NUM_EVOL_GFS + threads - 1) / threads));
+  switch (S) {
+    case 0: hipLaunchKernelGGL(rhs_eval_rk4_substep_rim__gpu<0>, grid, block, 0, stream, *params, *rfmstruct, auxevol_gfs, in_gfs, y_n, rt, out, dt, rim_rhs, (int)nb, n, bc->d_ob_dest, bc->d_ob_face); break;
+    case 1: hipLaunchKernelGGL(rhs_eval_rk4_substep_rim__gpu<1>, grid, block, 0, stream, *params, *rfmstruct, auxevol_gfs, in_gfs, y_n, rt, out, dt, rim_rhs, (int)nb, n, bc->d_ob_dest, bc->d_ob_face); break;
+    case 2: hipLaunchKernelGGL(rhs_eval_rk4_substep_rim__gpu<2>, grid, block, 0, stream, *params, *rfmstruct, auxevol_gfs, in_gfs, y_n, rt, out, dt, rim_rhs, (int)nb, n, bc->d_ob_dest, bc->d_ob_face); break;
+    case 3: hipLaunchKernelGGL(rhs_eval_rk4_substep_rim__gpu<3>, grid, block, 0, stream, *params, *rfmstruct, auxevol_gfs, in_gfs, y_n, rt, out, dt, rim_rhs, (int)nb, n, bc->d_ob_dest, bc->d_ob_face); break;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
+}
 extern "C" int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, hipStream_t stream) {
   if (!params || !y_n_gfs || !k_odd_gfs || !k_even_gfs || !y_nplus1_running_total_gfs) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
@@ -1038,6 +1375,20 @@ extern "C" int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *pa
 extern "C" int MoL_step_forward_in_time_sommerfeld(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, hipStream_t stream) {
   return MoL_step_forward_in_time_sommerfeld_unfused(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs, k_even_gfs, y_nplus1_running_total_gfs, dt, stream);
 }
+// The same step as two launches per substep (values those of the unfused step); R:
+// the scratch of nrpy_sommerfeld_chain_scratch, not shared with a step on another stream.
+static int nrpy_sommerfeld_chain_step(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, double *R, const double dt, hipStream_t stream) {
+  int rc;
+  if ((rc = rhs_eval_rk4_substep_rim(0, rfmstruct, params, bcstruct, nullptr, y_n_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, R, dt, stream))) return rc;
+  if ((rc = nrpy_sommerfeld_chain(0, params, bcstruct, evol_gf_parity, R, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_rim(1, rfmstruct, params, bcstruct, nullptr, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, R, dt, stream))) return rc;
+  if ((rc = nrpy_sommerfeld_chain(1, params, bcstruct, evol_gf_parity, R, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_rim(2, rfmstruct, params, bcstruct, nullptr, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, R, dt, stream))) return rc;
+  if ((rc = nrpy_sommerfeld_chain(2, params, bcstruct, evol_gf_parity, R, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_rim(3, rfmstruct, params, bcstruct, nullptr, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, R, dt, stream))) return rc;
+  if ((rc = nrpy_sommerfeld_chain(3, params, bcstruct, evol_gf_parity, R, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
+  return NRPY_OK;
+}
 // The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; pointers, xx
 // and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.
 extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out) {
@@ -1047,10 +1398,15 @@ extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_
   if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return NRPY_ERR_LAUNCH;
   MoL_graph *g = new MoL_graph();
   int rc = NRPY_OK;
+  // without scratch memory, or on a grid the chain kernel does not cover: the unfused step
+  if (rfmstruct && y_n_gfs && k_odd_gfs && k_even_gfs && y_nplus1_running_total_gfs)
+    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct, s);
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = NRPY_ERR_LAUNCH;
   if (!rc) {
-    rc = MoL_step_forward_in_time_sommerfeld(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs, k_even_gfs,
-                                             y_nplus1_running_total_gfs, dt, s);
+    rc = g->scratch ? nrpy_sommerfeld_chain_step(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,
+                                                 k_even_gfs, y_nplus1_running_total_gfs, g->scratch, dt, s)
+                    : MoL_step_forward_in_time_sommerfeld(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,
+                                                          k_even_gfs, y_nplus1_running_total_gfs, dt, s);
     hipGraph_t gr;
     const hipError_t e = hipStreamEndCapture(s, &gr);
     if (!rc && e != hipSuccess) rc = NRPY_ERR_LAUNCH;
@@ -1060,7 +1416,7 @@ extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_
     }
   }
   (void)hipStreamDestroy(s);
-  if (rc) { delete g; return rc; }
+  if (rc) { (void)hipFree(g->scratch); delete g; return rc; }
   *out = g;
   return NRPY_OK;
 }

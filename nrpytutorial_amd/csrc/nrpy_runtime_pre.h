@@ -65,12 +65,14 @@ __device__ __forceinline__ double nrpy_vjp_select(const bool inside, const doubl
 // below gives each XCD a contiguous range of tiles (i2 slowest), so stencil
 // neighbours in i1 and i2 are mostly resident in the same XCD's L2.
 #define NRPY_NUM_XCD 8
-#define NRPY_BLOCK_COORDS(n0, n1, n2)                                                          \
+#define NRPY_BLOCK_COORDS(n0, n1, n2) NRPY_BLOCK_COORDS_OF((int)gridDim.x, n0, n1, n2)
+// the same for the first nblocks blocks of a launch
+#define NRPY_BLOCK_COORDS_OF(nblocks, n0, n1, n2)                                              \
   int nrpy_bx, nrpy_by, nrpy_bz;                                                               \
   {                                                                                            \
     const int nbx_ = ((n0) + (int)blockDim.x - 1) / (int)blockDim.x;                           \
     const int nby_ = ((n1) + (int)blockDim.y - 1) / (int)blockDim.y;                           \
-    const int nb_ = (int)gridDim.x;                                                            \
+    const int nb_ = (nblocks);                                                                 \
     const int b_ = (int)blockIdx.x;                                                            \
     const int q_ = nb_ / NRPY_NUM_XCD, r_ = nb_ % NRPY_NUM_XCD;                                \
     const int x_ = b_ % NRPY_NUM_XCD, l_ = b_ / NRPY_NUM_XCD;                                  \
