@@ -30,6 +30,7 @@ from .. import grid as gri
 from .. import finite_difference as fin
 from .. import outputC as oc
 from .. import reference_metric as rfm
+from . import schedule
 
 _PRINT = oc._Printer()
 
@@ -198,7 +199,7 @@ def vjp_transpose_bodies(slots, all_points=False):
 
 
 def vjp_kernels(name, exprs, upwindcontrolvec, pointwise_loopopts, rfm_args, all_points=False, groups=None,
-                split_transpose=False):
+                split_transpose=False, order=None):
     """Generated source of ``<name>_vjp`` (pass 1 + pass 2 + an extern "C" driver).
 
     all_points: the forward operation is pointwise at every point (AllPoints loop, no
@@ -209,6 +210,7 @@ def vjp_kernels(name, exprs, upwindcontrolvec, pointwise_loopopts, rfm_args, all
     those an earlier group introduced, so vjp_G holds each slot once.
     split_transpose: pass 2 as one kernel per cotangent gridfunction, so each lane sums the
     transposed stencils of one gridfunction instead of all of them.
+    order: prefetch distance and region length of pass 1's statement order (schedule.reorder).
     Returns (source, slots, output arrays {gftype: [gf names]}, state_dependent)."""
     groups = groups or [list(range(len(exprs)))]
     slots, state_dependent, p1, uses_auxevol, p1_names = [], False, "", False, []
@@ -219,7 +221,7 @@ def vjp_kernels(name, exprs, upwindcontrolvec, pointwise_loopopts, rfm_args, all
         slots += sl
         state_dependent = state_dependent or dep
         uses_auxevol = uses_auxevol or "auxevol_gfs[" in body1
-        bodies.append(body1)
+        bodies.append(schedule.reorder(body1, *order) if order else body1)
     for k, body1 in enumerate(bodies):
         kname = name + "_vjp_pointwise" + ("_g%d" % k if len(groups) > 1 else "")
         p1_names.append(kname)

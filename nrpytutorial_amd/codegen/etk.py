@@ -214,7 +214,7 @@ def entry_point(name, desc, args, fills, kernels, interior=True):
 def bssn_etk(bundle_name="bssn_etk"):
     from ..BSSN import BSSN_quantities as Bq, BSSN_RHSs as rhs, BSSN_gauge_RHSs as gaugerhs
     from ..BSSN import Enforce_Detgammabar_Constraint as EGC, BSSN_constraints as bssncon
-    from .systems import rhs_groups, ricci_groups, lds_tile_for_group, MIN_TWO_WAVES_OUTPUTS
+    from .systems import rhs_groups, ricci_groups, lds_tile_for_group, scheduled, MIN_TWO_WAVES_OUTPUTS
     t0 = time.time()
     par.set_parval_from_str("grid::DIM", 3)
     par.set_parval_from_str("finite_difference::FD_CENTDERIVS_ORDER", FD_ORDER)
@@ -267,6 +267,7 @@ def bssn_etk(bundle_name="bssn_etk"):
                                                for n in grp], params="outCverbose=False")
         flops += bd.count_body(body)["flops"]
         name = "Baikal_BSSN_Ricci_g%d" % k
+        body = scheduled(body, grp, "Cartesian")
         text, launch = etk_kernel(name, "Ricci tensor components %s" % ", ".join(grp), body, table)
         src.append(text)
         kernels.append((name, launch))
@@ -293,6 +294,7 @@ def bssn_etk(bundle_name="bssn_etk"):
         body = fin.FD_outputC("returnstring", sel, params="outCverbose=False", upwindcontrolvec=betaU)
         flops += bd.count_body(body)["flops"]
         name = "Baikal_BSSN_RHSs_g%d" % k
+        body = scheduled(body, grp, "Cartesian")
         text, launch = etk_kernel(name, "BSSN right-hand sides of %s" % ", ".join(grp), body, table)
         src.append(text)
         kernels.append((name, launch))

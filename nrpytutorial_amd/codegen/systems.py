@@ -37,6 +37,7 @@ from . import addressing
 from . import bundle as bd
 from . import adjoint as adj
 from . import batch as bt
+from . import schedule
 
 CURVI_SCALARWAVE = {"scalarwave_sinhsphericalv2": "SinhSphericalv2",
                     "scalarwave_sinhcylindricalv2": "SinhCylindricalv2",
@@ -515,6 +516,37 @@ TILE_ADDRESS_OUTPUTS = (
 )
 
 
+# Statement order of the group kernels (codegen/schedule.py), chosen by the outputs of a group
+# and the grid's kind: (prefetch distance, region length, workgroup barriers). Measured on
+# MI355X. Cartesian 192^3, fused RK4 substep: Ricci 542 + 518 -> 487 + 460 us (485 + 482 without
+# the workgroup barriers, which lose 0.1 ms in the Lambda-bar group), the aDD,trK group 1435 ->
+# 1373 us (longer distances need more registers than two waves per SIMD have: 1.53 ms at 40
+# without barriers, 2.17 ms at 100), the Lambda-bar group 2153 -> 1849 us (it runs one wave per
+# SIMD whatever it needs, so its loads go far ahead; 2.08 ms at 32). Spherical, 128x128x64:
+# Ricci 107 + 124 -> 69 + 66 us, Lambda-bar 332 -> 222 us, the others even; 72x12x2: 63 -> 57 us
+# for the five. The lane-move group keeps its own order (lds.sink_xshift_values).
+_RICCI_FIRST, _RICCI_SECOND = {"RbarDD00", "RbarDD01", "RbarDD02"}, {"RbarDD11", "RbarDD12", "RbarDD22"}
+_CURVATURE = {"aDD00", "aDD01", "aDD02", "aDD11", "aDD12", "aDD22", "trK"}
+_METRIC = {"hDD00", "hDD01", "hDD02", "hDD11", "hDD12", "hDD22", "alpha", "cf"}
+_SHIFT = {"betU0", "betU1", "betU2", "lambdaU0", "lambdaU1", "lambdaU2", "vetU0", "vetU1", "vetU2"}
+SCHEDULE_CARTESIAN = ((_RICCI_FIRST, (80, 40, True)), (_RICCI_SECOND, (80, 40, True)),
+                      (_CURVATURE, (40, 16, True)), (_SHIFT, (160, 80, False)))
+SCHEDULE_CURVILINEAR = ((_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24, False)),
+                        (_CURVATURE, (40, 24, False)), (_METRIC, (40, 24, False)), (_SHIFT, (150, 60, False)))
+# Pass 1 of the vector-Jacobian products, all groups: at 96^3 the RHS VJP 3729 -> 2926 us (its
+# Lambda-bar kernel spilled 364 bytes per lane), the Ricci VJP 1267 -> 1233 us.
+SCHEDULE_VJP = (60, 40)
+
+
+def scheduled(body, outputs, CoordSystem):
+    """The body of the kernel that computes ``outputs``, in the order measured best for it."""
+    table = SCHEDULE_CARTESIAN if CoordSystem == "Cartesian" else SCHEDULE_CURVILINEAR
+    for outs, how in table:
+        if set(outputs) == outs:
+            return schedule.reorder(body, *how)
+    return body
+
+
 def kernel_inputs(kernel_text):
     """Distinct (array, gridfunction) pairs a generated kernel reads: its stencil reads and
     the gridfunctions it copies into LDS."""
@@ -906,6 +938,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
         body = fin.FD_outputC("returnstring", sel, params="outCverbose=False", upwindcontrolvec=betaU)
         group_costs.append(bd.count_body(body))
         step_bodies.append(body)
+        body = scheduled(body, grp, CoordSystem)
         rhs_src += oc.outCfunction(outfile="returnstring", desc="BSSN RHSs of %s" % ", ".join(grp),
                                    name="rhs_eval_g%d" % k, params=rhs_params, body=body,
                                    loopopts="InteriorPoints,Enable_rfm_precompute")
@@ -941,6 +974,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                                                  for n in grp], params="outCverbose=False")
         ricci_costs.append(bd.count_body(body_k))
         step_bodies.append(body_k)
+        body_k = scheduled(body_k, grp, CoordSystem)
         ricci_src += oc.outCfunction(outfile="returnstring", desc="Evaluate the Ricci tensor components %s"
                                      % ", ".join(grp), name="Ricci_eval_g%d" % k, params=ricci_params, body=body_k,
                                      loopopts="InteriorPoints,Enable_rfm_precompute")
@@ -1021,11 +1055,12 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     vjp_src, vslots, _, _ = adj.vjp_kernels("rhs_eval", evol_rhss, betaU, "InteriorPoints,Enable_rfm_precompute",
                                             "rfm_struct *restrict rfmstruct,",
                                             groups=[[i for i, (n, _) in enumerate(pairs) if n in grp]
-                                                    for grp in vjp_groups], split_transpose=True)
+                                                    for grp in vjp_groups], split_transpose=True,
+                                            order=SCHEDULE_VJP)
     rvjp_src, rslots, _, _ = adj.vjp_kernels(
         "Ricci_eval", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n]) for n in ric_names], "",
         "InteriorPoints,Enable_rfm_precompute", "rfm_struct *restrict rfmstruct,",
-        groups=[[ric_names.index(n) for n in grp] for grp in ric_groups], split_transpose=True)
+        groups=[[ric_names.index(n) for n in grp] for grp in ric_groups], split_transpose=True, order=SCHEDULE_VJP)
     # det(gammabar) enforcement and the Hamiltonian constraint, for the adjoint of the BSSN RK4
     # step and of the H-L2 diagnostic; the mass derivatives of the initial data.
     dvjp_src, dslots, _, _ = adj.vjp_kernels("enforce_detgammabar_constraint", detg_exprs, "",
