@@ -301,6 +301,52 @@ def fused_rk4_kernel(name, args_decl, call_args, body_with_writes, loopopts="Int
     return kernel
 
 
+_EDGE_READ = re.compile(r"^(\s*)const double (\w+) = in_gfs\[IDX4\((\w+)GF, i0([+-]\d+)?,i1([+-]\d+)?,i2([+-]\d+)?\)\];$")
+
+
+def edge_body(body):
+    """An FD body whose input's ghost points hold nothing: a stencil value outside the interior is
+    extrapolated in registers from the interior values of the same stencil, as the ghost fill
+    extrapolates it (layers 1 and 2: 3 f0 - 3 f1 + f2 and 6 f0 - 8 f1 + 3 f2, f0 next to the edge,
+    in the fill kernel's order of operations). For bodies that read neighbours along one axis at
+    a time, at most two points away, on grids whose ghost points are all extrapolated ones. The
+    loads of ghost points stay (their values are replaced), so the body has no branch around a
+    load; only the few waves at an edge do the extra arithmetic."""
+    lines, names, last = body.splitlines(), {}, None
+    for k, l in enumerate(lines):
+        m = _EDGE_READ.match(l)
+        if m:
+            off = tuple(int(v or 0) for v in m.groups()[3:])
+            if sum(o != 0 for o in off) > 1 or max(map(abs, off)) > 2:
+                raise ValueError("edge_body: stencil read at " + str(off))
+            names[m.group(3), off] = m.group(2)
+            lines[k] = l.replace("const double", "double", 1)
+            indent, last = m.group(1), k
+        elif "in_gfs[" in l:
+            raise ValueError("edge_body: unrecognised read " + l.strip())
+    extra, fix = [], []
+    for gf, d in sorted({(g, [i for i in range(3) if o[i]][0]) for g, o in names if any(o)}):
+        def at(o):
+            off = [0, 0, 0]
+            off[d] = o
+            key = (gf, tuple(off))
+            if key not in names:
+                names[key] = "nrpy_%s_%s" % (gf, "c" if o == 0 else "i%d%s%d" % (d, "p" if o > 0 else "m", abs(o)))
+                extra.append("%sdouble %s = in_gfs[IDX4(%sGF, %s)];" % (indent, names[key], gf, ",".join(
+                    "i%d%s" % (i, "%+d" % v if v else "") for i, v in enumerate(off))))
+            return names[key]
+        for sign, first in ((-1, "NGHOSTS"), (1, "Nxx%d + NGHOSTS - 1" % d)):
+            inner = "%s + 1" % first if sign < 0 else "Nxx%d + NGHOSTS - 2" % d
+            f = [at(0), at(-sign), at(-2 * sign)]
+            fix.append("%sif (i%d == %s) {" % (indent, d, first))
+            fix.append("%s  %s = fma(1.0, %s, fma(-3.0, %s, 3.0 * %s));" % (indent, at(sign), f[2], f[1], f[0]))
+            fix.append("%s  %s = fma(3.0, %s, fma(-8.0, %s, 6.0 * %s));" % (indent, at(2 * sign), f[2], f[1], f[0]))
+            fix.append("%s} else if (i%d == %s) {" % (indent, d, inner))
+            fix.append("%s  %s = fma(1.0, %s, fma(-3.0, %s, 3.0 * %s));" % (indent, at(2 * sign), at(-sign), at(0), at(sign)))
+            fix.append("%s}" % indent)
+    return "\n".join(lines[:last + 1] + extra + fix + lines[last + 1:]) + "\n"
+
+
 _TOKEN = re.compile(r"[A-Za-z_][A-Za-z_0-9]*|\d+\.\d*(?:[eE][-+]?\d+)?|\d+|\S")
 _FUNCS = ("sqrt", "cbrt", "pow", "exp", "log", "sin", "cos", "tan", "fabs", "sinh", "cosh", "tanh", "asinh",
           "acos", "atan2")

@@ -50,7 +50,7 @@ BUNDLES = ("scalarwave_cartesian", "bssn_cartesian", "bssn_spherical_sym2", "max
     tuple(CURVI_SCALARWAVE) + ("bssn_etk",) + tuple(CURVI_MAXWELL)
 
 
-def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
+def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage="", edge=False):
     """MoL_step_forward_in_time + hipGraph replay for the diagonal RK4 schedule."""
     ricci = ("  if ((rc = Ricci_eval(rfmstruct, params, IN, auxevol_gfs, stream))) return rc;\n" if has_ricci else "")
     detg = ("  if ((rc = DETG(rfmstruct, params, OUT, stream))) return rc;\n"
@@ -58,13 +58,18 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
     sub = ("  /* substep S: IN -> OUT */\n" + ricci +
            "  if ((rc = rhs_eval_rk4_substep(S, " + rhs_call_args + ", y_n_gfs, y_nplus1_running_total_gfs, OUT, dt, "
            "stream))) return rc;\n"
-           "  if ((rc = FILL(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, OUT, stream))) return rc;\n" + detg)
+           "FILLCALL" + detg)
+    fill = "  if ((rc = FILL(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, OUT, stream))) return rc;\n"
     steps = ""
     # The stage states (substeps 0-2) are read by the next right-hand side only: they get the
-    # ghosts its stencils reach. The new state gets every ghost.
+    # ghosts its stencils reach, or none where it extrapolates them itself (edge). The new state
+    # gets every ghost.
     for s, (i, o) in enumerate((("y_n_gfs", "k_odd_gfs"), ("k_odd_gfs", "k_even_gfs"),
                                 ("k_even_gfs", "k_odd_gfs"), ("k_odd_gfs", "y_n_gfs"))):
-        steps += sub.replace("IN", i).replace("OUT", o).replace("substep S", "substep %d" % s) \
+        call = sub.replace("FILLCALL", "" if edge and s < 3 else fill)
+        if edge and s > 0:
+            call = call.replace("rhs_eval_rk4_substep(", "rhs_eval_rk4_substep_edge(")
+        steps += call.replace("IN", i).replace("OUT", o).replace("substep S", "substep %d" % s) \
             .replace("(S,", "(%d," % s).replace("FILL", "nrpy_stage_fill" if s < 3 else "apply_bcs_curvilinear_composed") \
             .replace("DETG", "enforce_detgammabar_constraint" + (detg_stage if s < 3 else ""))
     sig = ("const rfm_struct *rfmstruct, const paramstruct *params, const bc_struct *bcstruct, double *y_n_gfs, "
@@ -77,7 +82,11 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage=""):
         "  if (!rfmstruct || !params || !bcstruct || !y_n_gfs || !k_odd_gfs || !k_even_gfs ||\n"
         "      !y_nplus1_running_total_gfs) return NRPY_ERR_NULL;\n"
         + ("  if (!auxevol_gfs) return NRPY_ERR_NULL;\n" if has_ricci else "") +
-        "  int rc;\n" + steps + "  return NRPY_OK;\n}\n\n"
+        "  int rc;\n" +
+        ("  nrpy_gf_parity_args gfp;  // the boundary struct is the grid's: checked before the first substep\n"
+         "  memset(&gfp, 0, sizeof(gfp));\n"
+         "  if ((rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, &gfp))) return rc;\n"
+         if edge else "") + steps + "  return NRPY_OK;\n}\n\n"
         "struct MoL_graph {\n  hipGraph_t graph;\n  hipGraphExec_t exec;\n"
         "  double *scratch = nullptr;  // device memory of the captured step, owned by the graph\n};\n"
         "// Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed\n"
@@ -634,6 +643,10 @@ def scalarwave_cartesian():
     fused = bd.fused_rk4_kernel("rhs_eval_rk4_substep", args_decl, "", body, loopopts="InteriorPoints")
     fused += _fused_launcher("rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
                              "const double *auxevol_gfs, const double *in_gfs", "*params, in_gfs", "InteriorPoints")
+    fused += bd.fused_rk4_kernel("rhs_eval_rk4_substep_edge", args_decl, "", bd.edge_body(body),
+                                 loopopts="InteriorPoints")
+    fused += _fused_launcher("rhs_eval_rk4_substep_edge", "const rfm_struct *rfmstruct, const paramstruct *params, "
+                             "const double *auxevol_gfs, const double *in_gfs", "*params, in_gfs", "InteriorPoints")
     fused += _fused_shell_kernel(fused, "rhs_eval_rk4_substep") + _fused_shell_launcher(
         "rhs_eval_rk4_substep", "const paramstruct *params, const double *in_gfs", "*params, in_gfs")
     id_src = _initial_data_kernel([swid.uu_ID, swid.vv_ID], ["uu", "vv"])
@@ -643,7 +656,7 @@ def scalarwave_cartesian():
     pre, meta = _header(3, stage_offsets([body]))
     parts = [pre, bd.coord_host_functions("Cartesian"), '#include "../nrpy_runtime.h"', bd.rfm_struct_code(),
              rhs_src, fused, id_src, vjp_src,
-             _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"),
+             _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", edge=True),
              _mol_adjoint_glue(False, vdep, sorted(vouts["EVOL"]) == sorted(gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]
@@ -687,6 +700,10 @@ def maxwell_cartesian():
     fused = bd.fused_rk4_kernel("rhs_eval_rk4_substep", args_decl, "", body, loopopts="InteriorPoints")
     fused += _fused_launcher("rhs_eval_rk4_substep", "const rfm_struct *rfmstruct, const paramstruct *params, "
                              "const double *auxevol_gfs, const double *in_gfs", "*params, in_gfs", "InteriorPoints")
+    fused += bd.fused_rk4_kernel("rhs_eval_rk4_substep_edge", args_decl, "", bd.edge_body(body),
+                                 loopopts="InteriorPoints")
+    fused += _fused_launcher("rhs_eval_rk4_substep_edge", "const rfm_struct *rfmstruct, const paramstruct *params, "
+                             "const double *auxevol_gfs, const double *in_gfs", "*params, in_gfs", "InteriorPoints")
     fused += _fused_shell_kernel(fused, "rhs_eval_rk4_substep") + _fused_shell_launcher(
         "rhs_eval_rk4_substep", "const paramstruct *params, const double *in_gfs", "*params, in_gfs")
     id_src = _initial_data_kernel(id_rhss, names)
@@ -697,7 +714,7 @@ def maxwell_cartesian():
     pre, meta = _header(3, stage_offsets([body]))
     vjp_src, slots, vouts, vdep = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
     parts = [pre, coords, '#include "../nrpy_runtime.h"', bd.rfm_struct_code(), rhs_src, con_src, fused, id_src,
-             vjp_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"),
+             vjp_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", edge=True),
              _mol_adjoint_glue(False, vdep, sorted(vouts["EVOL"]) == sorted(gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]

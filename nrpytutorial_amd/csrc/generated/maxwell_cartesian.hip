@@ -562,6 +562,348 @@ extern "C" int rhs_eval_rk4_substep(const int S, const rfm_struct *rfmstruct, co
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
 }
 template <int S>
+__global__ void __launch_bounds__(256) rhs_eval_rk4_substep_edge__gpu(const paramstruct params, const double *__restrict__ in_gfs, double *rk_yn, double *rk_rt, double *rk_out, const double dt) {
+  const int Nxx0 = params.Nxx0;
+  const int Nxx1 = params.Nxx1;
+  const int Nxx2 = params.Nxx2;
+  const double invdx0 = params.invdx0;
+  const double invdx1 = params.invdx1;
+  const double invdx2 = params.invdx2;
+  const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
+  const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
+  const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
+  NRPY_BLOCK_COORDS(Nxx0, Nxx1, Nxx2);
+  const int i0 = NGHOSTS + nrpy_bx*(int)blockDim.x + (int)threadIdx.x;
+  const int i1 = NGHOSTS + nrpy_by*(int)blockDim.y + (int)threadIdx.y;
+  const int i2 = NGHOSTS + nrpy_bz*(int)blockDim.z + (int)threadIdx.z;
+  if (i0 >= Nxx0 + NGHOSTS || i1 >= Nxx1 + NGHOSTS || i2 >= Nxx2 + NGHOSTS) return;
+  {
+    /* Step 1 of 2: read gridfunctions and compute finite-difference stencils */
+    double EU0 = in_gfs[IDX4(EU0GF, i0,i1,i2)];
+    double EU1 = in_gfs[IDX4(EU1GF, i0,i1,i2)];
+    double EU2 = in_gfs[IDX4(EU2GF, i0,i1,i2)];
+    double AU0_i0_i1_i2m2 = in_gfs[IDX4(AU0GF, i0,i1,i2-2)];
+    double AU0_i0_i1_i2m1 = in_gfs[IDX4(AU0GF, i0,i1,i2-1)];
+    double AU0_i0_i1m2_i2 = in_gfs[IDX4(AU0GF, i0,i1-2,i2)];
+    double AU0_i0_i1m1_i2 = in_gfs[IDX4(AU0GF, i0,i1-1,i2)];
+    double AU0_i0m2_i1_i2 = in_gfs[IDX4(AU0GF, i0-2,i1,i2)];
+    double AU0_i0m1_i1_i2 = in_gfs[IDX4(AU0GF, i0-1,i1,i2)];
+    double AU0 = in_gfs[IDX4(AU0GF, i0,i1,i2)];
+    double AU0_i0p1_i1_i2 = in_gfs[IDX4(AU0GF, i0+1,i1,i2)];
+    double AU0_i0p2_i1_i2 = in_gfs[IDX4(AU0GF, i0+2,i1,i2)];
+    double AU0_i0_i1p1_i2 = in_gfs[IDX4(AU0GF, i0,i1+1,i2)];
+    double AU0_i0_i1p2_i2 = in_gfs[IDX4(AU0GF, i0,i1+2,i2)];
+    double AU0_i0_i1_i2p1 = in_gfs[IDX4(AU0GF, i0,i1,i2+1)];
+    double AU0_i0_i1_i2p2 = in_gfs[IDX4(AU0GF, i0,i1,i2+2)];
+    double AU1_i0_i1_i2m2 = in_gfs[IDX4(AU1GF, i0,i1,i2-2)];
+    double AU1_i0_i1_i2m1 = in_gfs[IDX4(AU1GF, i0,i1,i2-1)];
+    double AU1_i0_i1m2_i2 = in_gfs[IDX4(AU1GF, i0,i1-2,i2)];
+    double AU1_i0_i1m1_i2 = in_gfs[IDX4(AU1GF, i0,i1-1,i2)];
+    double AU1_i0m2_i1_i2 = in_gfs[IDX4(AU1GF, i0-2,i1,i2)];
+    double AU1_i0m1_i1_i2 = in_gfs[IDX4(AU1GF, i0-1,i1,i2)];
+    double AU1 = in_gfs[IDX4(AU1GF, i0,i1,i2)];
+    double AU1_i0p1_i1_i2 = in_gfs[IDX4(AU1GF, i0+1,i1,i2)];
+    double AU1_i0p2_i1_i2 = in_gfs[IDX4(AU1GF, i0+2,i1,i2)];
+    double AU1_i0_i1p1_i2 = in_gfs[IDX4(AU1GF, i0,i1+1,i2)];
+    double AU1_i0_i1p2_i2 = in_gfs[IDX4(AU1GF, i0,i1+2,i2)];
+    double AU1_i0_i1_i2p1 = in_gfs[IDX4(AU1GF, i0,i1,i2+1)];
+    double AU1_i0_i1_i2p2 = in_gfs[IDX4(AU1GF, i0,i1,i2+2)];
+    double AU2_i0_i1_i2m2 = in_gfs[IDX4(AU2GF, i0,i1,i2-2)];
+    double AU2_i0_i1_i2m1 = in_gfs[IDX4(AU2GF, i0,i1,i2-1)];
+    double AU2_i0_i1m2_i2 = in_gfs[IDX4(AU2GF, i0,i1-2,i2)];
+    double AU2_i0_i1m1_i2 = in_gfs[IDX4(AU2GF, i0,i1-1,i2)];
+    double AU2_i0m2_i1_i2 = in_gfs[IDX4(AU2GF, i0-2,i1,i2)];
+    double AU2_i0m1_i1_i2 = in_gfs[IDX4(AU2GF, i0-1,i1,i2)];
+    double AU2 = in_gfs[IDX4(AU2GF, i0,i1,i2)];
+    double AU2_i0p1_i1_i2 = in_gfs[IDX4(AU2GF, i0+1,i1,i2)];
+    double AU2_i0p2_i1_i2 = in_gfs[IDX4(AU2GF, i0+2,i1,i2)];
+    double AU2_i0_i1p1_i2 = in_gfs[IDX4(AU2GF, i0,i1+1,i2)];
+    double AU2_i0_i1p2_i2 = in_gfs[IDX4(AU2GF, i0,i1+2,i2)];
+    double AU2_i0_i1_i2p1 = in_gfs[IDX4(AU2GF, i0,i1,i2+1)];
+    double AU2_i0_i1_i2p2 = in_gfs[IDX4(AU2GF, i0,i1,i2+2)];
+    double psi_i0_i1_i2m2 = in_gfs[IDX4(PSIGF, i0,i1,i2-2)];
+    double psi_i0_i1_i2m1 = in_gfs[IDX4(PSIGF, i0,i1,i2-1)];
+    double psi_i0_i1m2_i2 = in_gfs[IDX4(PSIGF, i0,i1-2,i2)];
+    double psi_i0_i1m1_i2 = in_gfs[IDX4(PSIGF, i0,i1-1,i2)];
+    double psi_i0m2_i1_i2 = in_gfs[IDX4(PSIGF, i0-2,i1,i2)];
+    double psi_i0m1_i1_i2 = in_gfs[IDX4(PSIGF, i0-1,i1,i2)];
+    double psi = in_gfs[IDX4(PSIGF, i0,i1,i2)];
+    double psi_i0p1_i1_i2 = in_gfs[IDX4(PSIGF, i0+1,i1,i2)];
+    double psi_i0p2_i1_i2 = in_gfs[IDX4(PSIGF, i0+2,i1,i2)];
+    double psi_i0_i1p1_i2 = in_gfs[IDX4(PSIGF, i0,i1+1,i2)];
+    double psi_i0_i1p2_i2 = in_gfs[IDX4(PSIGF, i0,i1+2,i2)];
+    double psi_i0_i1_i2p1 = in_gfs[IDX4(PSIGF, i0,i1,i2+1)];
+    double psi_i0_i1_i2p2 = in_gfs[IDX4(PSIGF, i0,i1,i2+2)];
+    double Gamma_i0_i1_i2m2 = in_gfs[IDX4(GAMMAGF, i0,i1,i2-2)];
+    double Gamma_i0_i1_i2m1 = in_gfs[IDX4(GAMMAGF, i0,i1,i2-1)];
+    double Gamma_i0_i1m2_i2 = in_gfs[IDX4(GAMMAGF, i0,i1-2,i2)];
+    double Gamma_i0_i1m1_i2 = in_gfs[IDX4(GAMMAGF, i0,i1-1,i2)];
+    double Gamma_i0m2_i1_i2 = in_gfs[IDX4(GAMMAGF, i0-2,i1,i2)];
+    double Gamma_i0m1_i1_i2 = in_gfs[IDX4(GAMMAGF, i0-1,i1,i2)];
+    double Gamma = in_gfs[IDX4(GAMMAGF, i0,i1,i2)];
+    double Gamma_i0p1_i1_i2 = in_gfs[IDX4(GAMMAGF, i0+1,i1,i2)];
+    double Gamma_i0p2_i1_i2 = in_gfs[IDX4(GAMMAGF, i0+2,i1,i2)];
+    double Gamma_i0_i1p1_i2 = in_gfs[IDX4(GAMMAGF, i0,i1+1,i2)];
+    double Gamma_i0_i1p2_i2 = in_gfs[IDX4(GAMMAGF, i0,i1+2,i2)];
+    double Gamma_i0_i1_i2p1 = in_gfs[IDX4(GAMMAGF, i0,i1,i2+1)];
+    double Gamma_i0_i1_i2p2 = in_gfs[IDX4(GAMMAGF, i0,i1,i2+2)];
+    if (i0 == NGHOSTS) {
+      AU0_i0m1_i1_i2 = fma(1.0, AU0_i0p2_i1_i2, fma(-3.0, AU0_i0p1_i1_i2, 3.0 * AU0));
+      AU0_i0m2_i1_i2 = fma(3.0, AU0_i0p2_i1_i2, fma(-8.0, AU0_i0p1_i1_i2, 6.0 * AU0));
+    } else if (i0 == NGHOSTS + 1) {
+      AU0_i0m2_i1_i2 = fma(1.0, AU0_i0p1_i1_i2, fma(-3.0, AU0, 3.0 * AU0_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      AU0_i0p1_i1_i2 = fma(1.0, AU0_i0m2_i1_i2, fma(-3.0, AU0_i0m1_i1_i2, 3.0 * AU0));
+      AU0_i0p2_i1_i2 = fma(3.0, AU0_i0m2_i1_i2, fma(-8.0, AU0_i0m1_i1_i2, 6.0 * AU0));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      AU0_i0p2_i1_i2 = fma(1.0, AU0_i0m1_i1_i2, fma(-3.0, AU0, 3.0 * AU0_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      AU0_i0_i1m1_i2 = fma(1.0, AU0_i0_i1p2_i2, fma(-3.0, AU0_i0_i1p1_i2, 3.0 * AU0));
+      AU0_i0_i1m2_i2 = fma(3.0, AU0_i0_i1p2_i2, fma(-8.0, AU0_i0_i1p1_i2, 6.0 * AU0));
+    } else if (i1 == NGHOSTS + 1) {
+      AU0_i0_i1m2_i2 = fma(1.0, AU0_i0_i1p1_i2, fma(-3.0, AU0, 3.0 * AU0_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      AU0_i0_i1p1_i2 = fma(1.0, AU0_i0_i1m2_i2, fma(-3.0, AU0_i0_i1m1_i2, 3.0 * AU0));
+      AU0_i0_i1p2_i2 = fma(3.0, AU0_i0_i1m2_i2, fma(-8.0, AU0_i0_i1m1_i2, 6.0 * AU0));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      AU0_i0_i1p2_i2 = fma(1.0, AU0_i0_i1m1_i2, fma(-3.0, AU0, 3.0 * AU0_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      AU0_i0_i1_i2m1 = fma(1.0, AU0_i0_i1_i2p2, fma(-3.0, AU0_i0_i1_i2p1, 3.0 * AU0));
+      AU0_i0_i1_i2m2 = fma(3.0, AU0_i0_i1_i2p2, fma(-8.0, AU0_i0_i1_i2p1, 6.0 * AU0));
+    } else if (i2 == NGHOSTS + 1) {
+      AU0_i0_i1_i2m2 = fma(1.0, AU0_i0_i1_i2p1, fma(-3.0, AU0, 3.0 * AU0_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      AU0_i0_i1_i2p1 = fma(1.0, AU0_i0_i1_i2m2, fma(-3.0, AU0_i0_i1_i2m1, 3.0 * AU0));
+      AU0_i0_i1_i2p2 = fma(3.0, AU0_i0_i1_i2m2, fma(-8.0, AU0_i0_i1_i2m1, 6.0 * AU0));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      AU0_i0_i1_i2p2 = fma(1.0, AU0_i0_i1_i2m1, fma(-3.0, AU0, 3.0 * AU0_i0_i1_i2p1));
+    }
+    if (i0 == NGHOSTS) {
+      AU1_i0m1_i1_i2 = fma(1.0, AU1_i0p2_i1_i2, fma(-3.0, AU1_i0p1_i1_i2, 3.0 * AU1));
+      AU1_i0m2_i1_i2 = fma(3.0, AU1_i0p2_i1_i2, fma(-8.0, AU1_i0p1_i1_i2, 6.0 * AU1));
+    } else if (i0 == NGHOSTS + 1) {
+      AU1_i0m2_i1_i2 = fma(1.0, AU1_i0p1_i1_i2, fma(-3.0, AU1, 3.0 * AU1_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      AU1_i0p1_i1_i2 = fma(1.0, AU1_i0m2_i1_i2, fma(-3.0, AU1_i0m1_i1_i2, 3.0 * AU1));
+      AU1_i0p2_i1_i2 = fma(3.0, AU1_i0m2_i1_i2, fma(-8.0, AU1_i0m1_i1_i2, 6.0 * AU1));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      AU1_i0p2_i1_i2 = fma(1.0, AU1_i0m1_i1_i2, fma(-3.0, AU1, 3.0 * AU1_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      AU1_i0_i1m1_i2 = fma(1.0, AU1_i0_i1p2_i2, fma(-3.0, AU1_i0_i1p1_i2, 3.0 * AU1));
+      AU1_i0_i1m2_i2 = fma(3.0, AU1_i0_i1p2_i2, fma(-8.0, AU1_i0_i1p1_i2, 6.0 * AU1));
+    } else if (i1 == NGHOSTS + 1) {
+      AU1_i0_i1m2_i2 = fma(1.0, AU1_i0_i1p1_i2, fma(-3.0, AU1, 3.0 * AU1_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      AU1_i0_i1p1_i2 = fma(1.0, AU1_i0_i1m2_i2, fma(-3.0, AU1_i0_i1m1_i2, 3.0 * AU1));
+      AU1_i0_i1p2_i2 = fma(3.0, AU1_i0_i1m2_i2, fma(-8.0, AU1_i0_i1m1_i2, 6.0 * AU1));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      AU1_i0_i1p2_i2 = fma(1.0, AU1_i0_i1m1_i2, fma(-3.0, AU1, 3.0 * AU1_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      AU1_i0_i1_i2m1 = fma(1.0, AU1_i0_i1_i2p2, fma(-3.0, AU1_i0_i1_i2p1, 3.0 * AU1));
+      AU1_i0_i1_i2m2 = fma(3.0, AU1_i0_i1_i2p2, fma(-8.0, AU1_i0_i1_i2p1, 6.0 * AU1));
+    } else if (i2 == NGHOSTS + 1) {
+      AU1_i0_i1_i2m2 = fma(1.0, AU1_i0_i1_i2p1, fma(-3.0, AU1, 3.0 * AU1_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      AU1_i0_i1_i2p1 = fma(1.0, AU1_i0_i1_i2m2, fma(-3.0, AU1_i0_i1_i2m1, 3.0 * AU1));
+      AU1_i0_i1_i2p2 = fma(3.0, AU1_i0_i1_i2m2, fma(-8.0, AU1_i0_i1_i2m1, 6.0 * AU1));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      AU1_i0_i1_i2p2 = fma(1.0, AU1_i0_i1_i2m1, fma(-3.0, AU1, 3.0 * AU1_i0_i1_i2p1));
+    }
+    if (i0 == NGHOSTS) {
+      AU2_i0m1_i1_i2 = fma(1.0, AU2_i0p2_i1_i2, fma(-3.0, AU2_i0p1_i1_i2, 3.0 * AU2));
+      AU2_i0m2_i1_i2 = fma(3.0, AU2_i0p2_i1_i2, fma(-8.0, AU2_i0p1_i1_i2, 6.0 * AU2));
+    } else if (i0 == NGHOSTS + 1) {
+      AU2_i0m2_i1_i2 = fma(1.0, AU2_i0p1_i1_i2, fma(-3.0, AU2, 3.0 * AU2_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      AU2_i0p1_i1_i2 = fma(1.0, AU2_i0m2_i1_i2, fma(-3.0, AU2_i0m1_i1_i2, 3.0 * AU2));
+      AU2_i0p2_i1_i2 = fma(3.0, AU2_i0m2_i1_i2, fma(-8.0, AU2_i0m1_i1_i2, 6.0 * AU2));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      AU2_i0p2_i1_i2 = fma(1.0, AU2_i0m1_i1_i2, fma(-3.0, AU2, 3.0 * AU2_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      AU2_i0_i1m1_i2 = fma(1.0, AU2_i0_i1p2_i2, fma(-3.0, AU2_i0_i1p1_i2, 3.0 * AU2));
+      AU2_i0_i1m2_i2 = fma(3.0, AU2_i0_i1p2_i2, fma(-8.0, AU2_i0_i1p1_i2, 6.0 * AU2));
+    } else if (i1 == NGHOSTS + 1) {
+      AU2_i0_i1m2_i2 = fma(1.0, AU2_i0_i1p1_i2, fma(-3.0, AU2, 3.0 * AU2_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      AU2_i0_i1p1_i2 = fma(1.0, AU2_i0_i1m2_i2, fma(-3.0, AU2_i0_i1m1_i2, 3.0 * AU2));
+      AU2_i0_i1p2_i2 = fma(3.0, AU2_i0_i1m2_i2, fma(-8.0, AU2_i0_i1m1_i2, 6.0 * AU2));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      AU2_i0_i1p2_i2 = fma(1.0, AU2_i0_i1m1_i2, fma(-3.0, AU2, 3.0 * AU2_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      AU2_i0_i1_i2m1 = fma(1.0, AU2_i0_i1_i2p2, fma(-3.0, AU2_i0_i1_i2p1, 3.0 * AU2));
+      AU2_i0_i1_i2m2 = fma(3.0, AU2_i0_i1_i2p2, fma(-8.0, AU2_i0_i1_i2p1, 6.0 * AU2));
+    } else if (i2 == NGHOSTS + 1) {
+      AU2_i0_i1_i2m2 = fma(1.0, AU2_i0_i1_i2p1, fma(-3.0, AU2, 3.0 * AU2_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      AU2_i0_i1_i2p1 = fma(1.0, AU2_i0_i1_i2m2, fma(-3.0, AU2_i0_i1_i2m1, 3.0 * AU2));
+      AU2_i0_i1_i2p2 = fma(3.0, AU2_i0_i1_i2m2, fma(-8.0, AU2_i0_i1_i2m1, 6.0 * AU2));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      AU2_i0_i1_i2p2 = fma(1.0, AU2_i0_i1_i2m1, fma(-3.0, AU2, 3.0 * AU2_i0_i1_i2p1));
+    }
+    if (i0 == NGHOSTS) {
+      Gamma_i0m1_i1_i2 = fma(1.0, Gamma_i0p2_i1_i2, fma(-3.0, Gamma_i0p1_i1_i2, 3.0 * Gamma));
+      Gamma_i0m2_i1_i2 = fma(3.0, Gamma_i0p2_i1_i2, fma(-8.0, Gamma_i0p1_i1_i2, 6.0 * Gamma));
+    } else if (i0 == NGHOSTS + 1) {
+      Gamma_i0m2_i1_i2 = fma(1.0, Gamma_i0p1_i1_i2, fma(-3.0, Gamma, 3.0 * Gamma_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      Gamma_i0p1_i1_i2 = fma(1.0, Gamma_i0m2_i1_i2, fma(-3.0, Gamma_i0m1_i1_i2, 3.0 * Gamma));
+      Gamma_i0p2_i1_i2 = fma(3.0, Gamma_i0m2_i1_i2, fma(-8.0, Gamma_i0m1_i1_i2, 6.0 * Gamma));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      Gamma_i0p2_i1_i2 = fma(1.0, Gamma_i0m1_i1_i2, fma(-3.0, Gamma, 3.0 * Gamma_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      Gamma_i0_i1m1_i2 = fma(1.0, Gamma_i0_i1p2_i2, fma(-3.0, Gamma_i0_i1p1_i2, 3.0 * Gamma));
+      Gamma_i0_i1m2_i2 = fma(3.0, Gamma_i0_i1p2_i2, fma(-8.0, Gamma_i0_i1p1_i2, 6.0 * Gamma));
+    } else if (i1 == NGHOSTS + 1) {
+      Gamma_i0_i1m2_i2 = fma(1.0, Gamma_i0_i1p1_i2, fma(-3.0, Gamma, 3.0 * Gamma_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      Gamma_i0_i1p1_i2 = fma(1.0, Gamma_i0_i1m2_i2, fma(-3.0, Gamma_i0_i1m1_i2, 3.0 * Gamma));
+      Gamma_i0_i1p2_i2 = fma(3.0, Gamma_i0_i1m2_i2, fma(-8.0, Gamma_i0_i1m1_i2, 6.0 * Gamma));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      Gamma_i0_i1p2_i2 = fma(1.0, Gamma_i0_i1m1_i2, fma(-3.0, Gamma, 3.0 * Gamma_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      Gamma_i0_i1_i2m1 = fma(1.0, Gamma_i0_i1_i2p2, fma(-3.0, Gamma_i0_i1_i2p1, 3.0 * Gamma));
+      Gamma_i0_i1_i2m2 = fma(3.0, Gamma_i0_i1_i2p2, fma(-8.0, Gamma_i0_i1_i2p1, 6.0 * Gamma));
+    } else if (i2 == NGHOSTS + 1) {
+      Gamma_i0_i1_i2m2 = fma(1.0, Gamma_i0_i1_i2p1, fma(-3.0, Gamma, 3.0 * Gamma_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      Gamma_i0_i1_i2p1 = fma(1.0, Gamma_i0_i1_i2m2, fma(-3.0, Gamma_i0_i1_i2m1, 3.0 * Gamma));
+      Gamma_i0_i1_i2p2 = fma(3.0, Gamma_i0_i1_i2m2, fma(-8.0, Gamma_i0_i1_i2m1, 6.0 * Gamma));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      Gamma_i0_i1_i2p2 = fma(1.0, Gamma_i0_i1_i2m1, fma(-3.0, Gamma, 3.0 * Gamma_i0_i1_i2p1));
+    }
+    if (i0 == NGHOSTS) {
+      psi_i0m1_i1_i2 = fma(1.0, psi_i0p2_i1_i2, fma(-3.0, psi_i0p1_i1_i2, 3.0 * psi));
+      psi_i0m2_i1_i2 = fma(3.0, psi_i0p2_i1_i2, fma(-8.0, psi_i0p1_i1_i2, 6.0 * psi));
+    } else if (i0 == NGHOSTS + 1) {
+      psi_i0m2_i1_i2 = fma(1.0, psi_i0p1_i1_i2, fma(-3.0, psi, 3.0 * psi_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      psi_i0p1_i1_i2 = fma(1.0, psi_i0m2_i1_i2, fma(-3.0, psi_i0m1_i1_i2, 3.0 * psi));
+      psi_i0p2_i1_i2 = fma(3.0, psi_i0m2_i1_i2, fma(-8.0, psi_i0m1_i1_i2, 6.0 * psi));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      psi_i0p2_i1_i2 = fma(1.0, psi_i0m1_i1_i2, fma(-3.0, psi, 3.0 * psi_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      psi_i0_i1m1_i2 = fma(1.0, psi_i0_i1p2_i2, fma(-3.0, psi_i0_i1p1_i2, 3.0 * psi));
+      psi_i0_i1m2_i2 = fma(3.0, psi_i0_i1p2_i2, fma(-8.0, psi_i0_i1p1_i2, 6.0 * psi));
+    } else if (i1 == NGHOSTS + 1) {
+      psi_i0_i1m2_i2 = fma(1.0, psi_i0_i1p1_i2, fma(-3.0, psi, 3.0 * psi_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      psi_i0_i1p1_i2 = fma(1.0, psi_i0_i1m2_i2, fma(-3.0, psi_i0_i1m1_i2, 3.0 * psi));
+      psi_i0_i1p2_i2 = fma(3.0, psi_i0_i1m2_i2, fma(-8.0, psi_i0_i1m1_i2, 6.0 * psi));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      psi_i0_i1p2_i2 = fma(1.0, psi_i0_i1m1_i2, fma(-3.0, psi, 3.0 * psi_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      psi_i0_i1_i2m1 = fma(1.0, psi_i0_i1_i2p2, fma(-3.0, psi_i0_i1_i2p1, 3.0 * psi));
+      psi_i0_i1_i2m2 = fma(3.0, psi_i0_i1_i2p2, fma(-8.0, psi_i0_i1_i2p1, 6.0 * psi));
+    } else if (i2 == NGHOSTS + 1) {
+      psi_i0_i1_i2m2 = fma(1.0, psi_i0_i1_i2p1, fma(-3.0, psi, 3.0 * psi_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      psi_i0_i1_i2p1 = fma(1.0, psi_i0_i1_i2m2, fma(-3.0, psi_i0_i1_i2m1, 3.0 * psi));
+      psi_i0_i1_i2p2 = fma(3.0, psi_i0_i1_i2m2, fma(-8.0, psi_i0_i1_i2m1, 6.0 * psi));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      psi_i0_i1_i2p2 = fma(1.0, psi_i0_i1_i2m1, fma(-3.0, psi, 3.0 * psi_i0_i1_i2p1));
+    }
+    const double FDPart1_Rational_1_12 = 1.0/12.0;
+    const double FDPart1_Rational_2_3 = 2.0/3.0;
+    const double FDPart1_Rational_4_3 = 4.0/3.0;
+    const double FDPart1_Rational_m1_12 = -1.0/12.0;
+    const double FDPart1_Rational_m2_3 = -2.0/3.0;
+    const double FDPart1_Rational_m5_2 = -5.0/2.0;
+    const double FDPart1_0 = ((invdx0)*(invdx0));
+    const double FDPart1_1 = AU0*FDPart1_Rational_m5_2;
+    const double FDPart1_2 = ((invdx1)*(invdx1));
+    const double FDPart1_3 = ((invdx2)*(invdx2));
+    const double FDPart1_4 = AU1*FDPart1_Rational_m5_2;
+    const double FDPart1_5 = AU2*FDPart1_Rational_m5_2;
+    const double FDPart1_6 = FDPart1_Rational_m1_12*psi_i0p2_i1_i2;
+    const double FDPart1_7 = FDPart1_Rational_m1_12*psi_i0_i1p2_i2;
+    const double FDPart1_8 = FDPart1_Rational_m1_12*psi_i0_i1_i2p2;
+    const double FDPart1_9 = FDPart1_Rational_m5_2*psi;
+    const double AU_dDD000 = FDPart1_0*(AU0_i0m1_i1_i2*FDPart1_Rational_4_3 + AU0_i0m2_i1_i2*FDPart1_Rational_m1_12 + AU0_i0p1_i1_i2*FDPart1_Rational_4_3 + AU0_i0p2_i1_i2*FDPart1_Rational_m1_12 + FDPart1_1);
+    const double AU_dDD011 = FDPart1_2*(AU0_i0_i1m1_i2*FDPart1_Rational_4_3 + AU0_i0_i1m2_i2*FDPart1_Rational_m1_12 + AU0_i0_i1p1_i2*FDPart1_Rational_4_3 + AU0_i0_i1p2_i2*FDPart1_Rational_m1_12 + FDPart1_1);
+    const double AU_dDD022 = FDPart1_3*(AU0_i0_i1_i2m1*FDPart1_Rational_4_3 + AU0_i0_i1_i2m2*FDPart1_Rational_m1_12 + AU0_i0_i1_i2p1*FDPart1_Rational_4_3 + AU0_i0_i1_i2p2*FDPart1_Rational_m1_12 + FDPart1_1);
+    const double AU_dDD100 = FDPart1_0*(AU1_i0m1_i1_i2*FDPart1_Rational_4_3 + AU1_i0m2_i1_i2*FDPart1_Rational_m1_12 + AU1_i0p1_i1_i2*FDPart1_Rational_4_3 + AU1_i0p2_i1_i2*FDPart1_Rational_m1_12 + FDPart1_4);
+    const double AU_dDD111 = FDPart1_2*(AU1_i0_i1m1_i2*FDPart1_Rational_4_3 + AU1_i0_i1m2_i2*FDPart1_Rational_m1_12 + AU1_i0_i1p1_i2*FDPart1_Rational_4_3 + AU1_i0_i1p2_i2*FDPart1_Rational_m1_12 + FDPart1_4);
+    const double AU_dDD122 = FDPart1_3*(AU1_i0_i1_i2m1*FDPart1_Rational_4_3 + AU1_i0_i1_i2m2*FDPart1_Rational_m1_12 + AU1_i0_i1_i2p1*FDPart1_Rational_4_3 + AU1_i0_i1_i2p2*FDPart1_Rational_m1_12 + FDPart1_4);
+    const double AU_dDD200 = FDPart1_0*(AU2_i0m1_i1_i2*FDPart1_Rational_4_3 + AU2_i0m2_i1_i2*FDPart1_Rational_m1_12 + AU2_i0p1_i1_i2*FDPart1_Rational_4_3 + AU2_i0p2_i1_i2*FDPart1_Rational_m1_12 + FDPart1_5);
+    const double AU_dDD211 = FDPart1_2*(AU2_i0_i1m1_i2*FDPart1_Rational_4_3 + AU2_i0_i1m2_i2*FDPart1_Rational_m1_12 + AU2_i0_i1p1_i2*FDPart1_Rational_4_3 + AU2_i0_i1p2_i2*FDPart1_Rational_m1_12 + FDPart1_5);
+    const double AU_dDD222 = FDPart1_3*(AU2_i0_i1_i2m1*FDPart1_Rational_4_3 + AU2_i0_i1_i2m2*FDPart1_Rational_m1_12 + AU2_i0_i1_i2p1*FDPart1_Rational_4_3 + AU2_i0_i1_i2p2*FDPart1_Rational_m1_12 + FDPart1_5);
+    const double Gamma_dD0 = invdx0*(FDPart1_Rational_1_12*Gamma_i0m2_i1_i2 + FDPart1_Rational_2_3*Gamma_i0p1_i1_i2 + FDPart1_Rational_m1_12*Gamma_i0p2_i1_i2 + FDPart1_Rational_m2_3*Gamma_i0m1_i1_i2);
+    const double Gamma_dD1 = invdx1*(FDPart1_Rational_1_12*Gamma_i0_i1m2_i2 + FDPart1_Rational_2_3*Gamma_i0_i1p1_i2 + FDPart1_Rational_m1_12*Gamma_i0_i1p2_i2 + FDPart1_Rational_m2_3*Gamma_i0_i1m1_i2);
+    const double Gamma_dD2 = invdx2*(FDPart1_Rational_1_12*Gamma_i0_i1_i2m2 + FDPart1_Rational_2_3*Gamma_i0_i1_i2p1 + FDPart1_Rational_m1_12*Gamma_i0_i1_i2p2 + FDPart1_Rational_m2_3*Gamma_i0_i1_i2m1);
+    const double psi_dD0 = invdx0*(FDPart1_6 + FDPart1_Rational_1_12*psi_i0m2_i1_i2 + FDPart1_Rational_2_3*psi_i0p1_i1_i2 + FDPart1_Rational_m2_3*psi_i0m1_i1_i2);
+    const double psi_dD1 = invdx1*(FDPart1_7 + FDPart1_Rational_1_12*psi_i0_i1m2_i2 + FDPart1_Rational_2_3*psi_i0_i1p1_i2 + FDPart1_Rational_m2_3*psi_i0_i1m1_i2);
+    const double psi_dD2 = invdx2*(FDPart1_8 + FDPart1_Rational_1_12*psi_i0_i1_i2m2 + FDPart1_Rational_2_3*psi_i0_i1_i2p1 + FDPart1_Rational_m2_3*psi_i0_i1_i2m1);
+    const double psi_dDD00 = FDPart1_0*(FDPart1_6 + FDPart1_9 + FDPart1_Rational_4_3*psi_i0m1_i1_i2 + FDPart1_Rational_4_3*psi_i0p1_i1_i2 + FDPart1_Rational_m1_12*psi_i0m2_i1_i2);
+    const double psi_dDD11 = FDPart1_2*(FDPart1_7 + FDPart1_9 + FDPart1_Rational_4_3*psi_i0_i1m1_i2 + FDPart1_Rational_4_3*psi_i0_i1p1_i2 + FDPart1_Rational_m1_12*psi_i0_i1m2_i2);
+    const double psi_dDD22 = FDPart1_3*(FDPart1_8 + FDPart1_9 + FDPart1_Rational_4_3*psi_i0_i1_i2m1 + FDPart1_Rational_4_3*psi_i0_i1_i2p1 + FDPart1_Rational_m1_12*psi_i0_i1_i2m2);
+    /* Step 2 of 2: evaluate right-hand sides and write to memory */
+  const double __rhs_AU0 = -EU0 - psi_dD0;
+  const double __rhs_AU1 = -EU1 - psi_dD1;
+  const double __rhs_AU2 = -EU2 - psi_dD2;
+  const double __rhs_EU0 = -AU_dDD000 - AU_dDD011 - AU_dDD022 + Gamma_dD0;
+  const double __rhs_EU1 = -AU_dDD100 - AU_dDD111 - AU_dDD122 + Gamma_dD1;
+  const double __rhs_EU2 = -AU_dDD200 - AU_dDD211 - AU_dDD222 + Gamma_dD2;
+  const double __rhs_GAMMA = -psi_dDD00 - psi_dDD11 - psi_dDD22;
+  const double __rhs_PSI = -Gamma;
+  __builtin_amdgcn_sched_barrier(0);
+  NRPY_RK4_PRELOAD(S, AU0GF, 0)
+  NRPY_RK4_PRELOAD(S, AU1GF, 1)
+  NRPY_RK4_PRELOAD(S, AU2GF, 2)
+  NRPY_RK4_PRELOAD(S, EU0GF, 3)
+  NRPY_RK4_PRELOAD(S, EU1GF, 4)
+  NRPY_RK4_PRELOAD(S, EU2GF, 5)
+  NRPY_RK4_PRELOAD(S, GAMMAGF, 6)
+  NRPY_RK4_PRELOAD(S, PSIGF, 7)
+  NRPY_RK4_STORE(S, 0, __rhs_AU0);
+  NRPY_RK4_STORE(S, 1, __rhs_AU1);
+  NRPY_RK4_STORE(S, 2, __rhs_AU2);
+  NRPY_RK4_STORE(S, 3, __rhs_EU0);
+  NRPY_RK4_STORE(S, 4, __rhs_EU1);
+  NRPY_RK4_STORE(S, 5, __rhs_EU2);
+  NRPY_RK4_STORE(S, 6, __rhs_GAMMA);
+  NRPY_RK4_STORE(S, 7, __rhs_PSI);
+  }
+}
+extern "C" int rhs_eval_rk4_substep_edge(const int S, const rfm_struct *rfmstruct, const paramstruct *params, const double *auxevol_gfs, const double *in_gfs, double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
+  if (!params || !y_n || !rt || !out) return NRPY_ERR_NULL;
+  if (S < 0 || S > 3) return NRPY_ERR_PARAM;
+  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
+  const dim3 block = nrpy_block(3, 64, 4, 1);
+  const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2));
+  switch (S) {
+    case 0: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<0>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 1: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<1>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 2: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<2>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 3: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<3>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
+}
+template <int S>
 __global__ void __launch_bounds__(256) rhs_eval_rk4_substep_shell__gpu(const paramstruct params, const double *__restrict__ in_gfs, double *rk_yn, double *rk_rt, double *rk_out, const double dt, double *__restrict__ shell_rhs) {
   const int Nxx0 = params.Nxx0;
   const int Nxx1 = params.Nxx1;
@@ -804,7 +1146,7 @@ extern "C" int initial_data(const paramstruct *params, double *xx[3], double *in
   if (!params) return NRPY_ERR_NULL;
   if (!in_gfs) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(3, 64, 4, 1);
+  const dim3 block = nrpy_block(4, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx_plus_2NGHOSTS0, params->Nxx_plus_2NGHOSTS1, params->Nxx_plus_2NGHOSTS2));
   hipLaunchKernelGGL(initial_data__gpu, grid, block, 0, stream, *params, xx[0], xx[1], xx[2], in_gfs);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -969,7 +1311,7 @@ extern "C" int rhs_eval_vjp_pointwise(const paramstruct *params, const double *i
   if (!params) return NRPY_ERR_NULL;
   if (!in_gfs || !cot_rhs_gfs || !vjp_G) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(4, 64, 4, 1);
+  const dim3 block = nrpy_block(5, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2));
   hipLaunchKernelGGL(rhs_eval_vjp_pointwise__gpu, grid, block, 0, stream, *params, in_gfs, cot_rhs_gfs, vjp_G);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -1021,7 +1363,7 @@ extern "C" int rhs_eval_vjp_transpose(const paramstruct *params, const double *v
   if (!params) return NRPY_ERR_NULL;
   if (!vjp_G || !cot_in_gfs) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(5, 64, 4, 1);
+  const dim3 block = nrpy_block(6, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx_plus_2NGHOSTS0, params->Nxx_plus_2NGHOSTS1, params->Nxx_plus_2NGHOSTS2));
   hipLaunchKernelGGL(rhs_eval_vjp_transpose__gpu, grid, block, 0, stream, *params, vjp_G, cot_in_gfs);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -1048,17 +1390,17 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
   if (!rfmstruct || !params || !bcstruct || !y_n_gfs || !k_odd_gfs || !k_even_gfs ||
       !y_nplus1_running_total_gfs) return NRPY_ERR_NULL;
   int rc;
+  nrpy_gf_parity_args gfp;  // the boundary struct is the grid's: checked before the first substep
+  memset(&gfp, 0, sizeof(gfp));
+  if ((rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, &gfp))) return rc;
   /* substep 0: y_n_gfs -> k_odd_gfs */
   if ((rc = rhs_eval_rk4_substep(0, rfmstruct, params, auxevol_gfs, y_n_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
   /* substep 1: k_odd_gfs -> k_even_gfs */
-  if ((rc = rhs_eval_rk4_substep(1, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_even_gfs, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(1, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
   /* substep 2: k_even_gfs -> k_odd_gfs */
-  if ((rc = rhs_eval_rk4_substep(2, rfmstruct, params, auxevol_gfs, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(2, rfmstruct, params, auxevol_gfs, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
   /* substep 3: k_odd_gfs -> y_n_gfs */
-  if ((rc = rhs_eval_rk4_substep(3, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(3, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
   if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, stream))) return rc;
   return NRPY_OK;
 }

@@ -301,6 +301,107 @@ extern "C" int rhs_eval_rk4_substep(const int S, const rfm_struct *rfmstruct, co
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
 }
 template <int S>
+__global__ void __launch_bounds__(256) rhs_eval_rk4_substep_edge__gpu(const paramstruct params, const double *__restrict__ in_gfs, double *rk_yn, double *rk_rt, double *rk_out, const double dt) {
+  const int Nxx0 = params.Nxx0;
+  const int Nxx1 = params.Nxx1;
+  const int Nxx2 = params.Nxx2;
+  const double invdx0 = params.invdx0;
+  const double invdx1 = params.invdx1;
+  const double invdx2 = params.invdx2;
+  const double wavespeed = params.wavespeed;
+  const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
+  const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
+  const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
+  NRPY_BLOCK_COORDS(Nxx0, Nxx1, Nxx2);
+  const int i0 = NGHOSTS + nrpy_bx*(int)blockDim.x + (int)threadIdx.x;
+  const int i1 = NGHOSTS + nrpy_by*(int)blockDim.y + (int)threadIdx.y;
+  const int i2 = NGHOSTS + nrpy_bz*(int)blockDim.z + (int)threadIdx.z;
+  if (i0 >= Nxx0 + NGHOSTS || i1 >= Nxx1 + NGHOSTS || i2 >= Nxx2 + NGHOSTS) return;
+  {
+    /* Step 1 of 2: read gridfunctions and compute finite-difference stencils */
+    double uu_i0_i1_i2m2 = in_gfs[IDX4(UUGF, i0,i1,i2-2)];
+    double uu_i0_i1_i2m1 = in_gfs[IDX4(UUGF, i0,i1,i2-1)];
+    double uu_i0_i1m2_i2 = in_gfs[IDX4(UUGF, i0,i1-2,i2)];
+    double uu_i0_i1m1_i2 = in_gfs[IDX4(UUGF, i0,i1-1,i2)];
+    double uu_i0m2_i1_i2 = in_gfs[IDX4(UUGF, i0-2,i1,i2)];
+    double uu_i0m1_i1_i2 = in_gfs[IDX4(UUGF, i0-1,i1,i2)];
+    double uu = in_gfs[IDX4(UUGF, i0,i1,i2)];
+    double uu_i0p1_i1_i2 = in_gfs[IDX4(UUGF, i0+1,i1,i2)];
+    double uu_i0p2_i1_i2 = in_gfs[IDX4(UUGF, i0+2,i1,i2)];
+    double uu_i0_i1p1_i2 = in_gfs[IDX4(UUGF, i0,i1+1,i2)];
+    double uu_i0_i1p2_i2 = in_gfs[IDX4(UUGF, i0,i1+2,i2)];
+    double uu_i0_i1_i2p1 = in_gfs[IDX4(UUGF, i0,i1,i2+1)];
+    double uu_i0_i1_i2p2 = in_gfs[IDX4(UUGF, i0,i1,i2+2)];
+    double vv = in_gfs[IDX4(VVGF, i0,i1,i2)];
+    if (i0 == NGHOSTS) {
+      uu_i0m1_i1_i2 = fma(1.0, uu_i0p2_i1_i2, fma(-3.0, uu_i0p1_i1_i2, 3.0 * uu));
+      uu_i0m2_i1_i2 = fma(3.0, uu_i0p2_i1_i2, fma(-8.0, uu_i0p1_i1_i2, 6.0 * uu));
+    } else if (i0 == NGHOSTS + 1) {
+      uu_i0m2_i1_i2 = fma(1.0, uu_i0p1_i1_i2, fma(-3.0, uu, 3.0 * uu_i0m1_i1_i2));
+    }
+    if (i0 == Nxx0 + NGHOSTS - 1) {
+      uu_i0p1_i1_i2 = fma(1.0, uu_i0m2_i1_i2, fma(-3.0, uu_i0m1_i1_i2, 3.0 * uu));
+      uu_i0p2_i1_i2 = fma(3.0, uu_i0m2_i1_i2, fma(-8.0, uu_i0m1_i1_i2, 6.0 * uu));
+    } else if (i0 == Nxx0 + NGHOSTS - 2) {
+      uu_i0p2_i1_i2 = fma(1.0, uu_i0m1_i1_i2, fma(-3.0, uu, 3.0 * uu_i0p1_i1_i2));
+    }
+    if (i1 == NGHOSTS) {
+      uu_i0_i1m1_i2 = fma(1.0, uu_i0_i1p2_i2, fma(-3.0, uu_i0_i1p1_i2, 3.0 * uu));
+      uu_i0_i1m2_i2 = fma(3.0, uu_i0_i1p2_i2, fma(-8.0, uu_i0_i1p1_i2, 6.0 * uu));
+    } else if (i1 == NGHOSTS + 1) {
+      uu_i0_i1m2_i2 = fma(1.0, uu_i0_i1p1_i2, fma(-3.0, uu, 3.0 * uu_i0_i1m1_i2));
+    }
+    if (i1 == Nxx1 + NGHOSTS - 1) {
+      uu_i0_i1p1_i2 = fma(1.0, uu_i0_i1m2_i2, fma(-3.0, uu_i0_i1m1_i2, 3.0 * uu));
+      uu_i0_i1p2_i2 = fma(3.0, uu_i0_i1m2_i2, fma(-8.0, uu_i0_i1m1_i2, 6.0 * uu));
+    } else if (i1 == Nxx1 + NGHOSTS - 2) {
+      uu_i0_i1p2_i2 = fma(1.0, uu_i0_i1m1_i2, fma(-3.0, uu, 3.0 * uu_i0_i1p1_i2));
+    }
+    if (i2 == NGHOSTS) {
+      uu_i0_i1_i2m1 = fma(1.0, uu_i0_i1_i2p2, fma(-3.0, uu_i0_i1_i2p1, 3.0 * uu));
+      uu_i0_i1_i2m2 = fma(3.0, uu_i0_i1_i2p2, fma(-8.0, uu_i0_i1_i2p1, 6.0 * uu));
+    } else if (i2 == NGHOSTS + 1) {
+      uu_i0_i1_i2m2 = fma(1.0, uu_i0_i1_i2p1, fma(-3.0, uu, 3.0 * uu_i0_i1_i2m1));
+    }
+    if (i2 == Nxx2 + NGHOSTS - 1) {
+      uu_i0_i1_i2p1 = fma(1.0, uu_i0_i1_i2m2, fma(-3.0, uu_i0_i1_i2m1, 3.0 * uu));
+      uu_i0_i1_i2p2 = fma(3.0, uu_i0_i1_i2m2, fma(-8.0, uu_i0_i1_i2m1, 6.0 * uu));
+    } else if (i2 == Nxx2 + NGHOSTS - 2) {
+      uu_i0_i1_i2p2 = fma(1.0, uu_i0_i1_i2m1, fma(-3.0, uu, 3.0 * uu_i0_i1_i2p1));
+    }
+    const double FDPart1_Rational_4_3 = 4.0/3.0;
+    const double FDPart1_Rational_m1_12 = -1.0/12.0;
+    const double FDPart1_Rational_m5_2 = -5.0/2.0;
+    const double FDPart1_0 = FDPart1_Rational_m5_2*uu;
+    const double uu_dDD00 = ((invdx0)*(invdx0))*(FDPart1_0 + FDPart1_Rational_4_3*uu_i0m1_i1_i2 + FDPart1_Rational_4_3*uu_i0p1_i1_i2 + FDPart1_Rational_m1_12*uu_i0m2_i1_i2 + FDPart1_Rational_m1_12*uu_i0p2_i1_i2);
+    const double uu_dDD11 = ((invdx1)*(invdx1))*(FDPart1_0 + FDPart1_Rational_4_3*uu_i0_i1m1_i2 + FDPart1_Rational_4_3*uu_i0_i1p1_i2 + FDPart1_Rational_m1_12*uu_i0_i1m2_i2 + FDPart1_Rational_m1_12*uu_i0_i1p2_i2);
+    const double uu_dDD22 = ((invdx2)*(invdx2))*(FDPart1_0 + FDPart1_Rational_4_3*uu_i0_i1_i2m1 + FDPart1_Rational_4_3*uu_i0_i1_i2p1 + FDPart1_Rational_m1_12*uu_i0_i1_i2m2 + FDPart1_Rational_m1_12*uu_i0_i1_i2p2);
+    /* Step 2 of 2: evaluate right-hand sides and write to memory */
+    const double FDPart3_0 = ((wavespeed)*(wavespeed));
+  const double __rhs_UU = vv;
+  const double __rhs_VV = FDPart3_0*uu_dDD00 + FDPart3_0*uu_dDD11 + FDPart3_0*uu_dDD22;
+  __builtin_amdgcn_sched_barrier(0);
+  NRPY_RK4_PRELOAD(S, UUGF, 0)
+  NRPY_RK4_PRELOAD(S, VVGF, 1)
+  NRPY_RK4_STORE(S, 0, __rhs_UU);
+  NRPY_RK4_STORE(S, 1, __rhs_VV);
+  }
+}
+extern "C" int rhs_eval_rk4_substep_edge(const int S, const rfm_struct *rfmstruct, const paramstruct *params, const double *auxevol_gfs, const double *in_gfs, double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
+  if (!params || !y_n || !rt || !out) return NRPY_ERR_NULL;
+  if (S < 0 || S > 3) return NRPY_ERR_PARAM;
+  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
+  const dim3 block = nrpy_block(2, 64, 4, 1);
+  const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2));
+  switch (S) {
+    case 0: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<0>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 1: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<1>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 2: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<2>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+    case 3: hipLaunchKernelGGL(rhs_eval_rk4_substep_edge__gpu<3>, grid, block, 0, stream, *params, in_gfs, y_n, rt, out, dt); break;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
+}
+template <int S>
 __global__ void __launch_bounds__(256) rhs_eval_rk4_substep_shell__gpu(const paramstruct params, const double *__restrict__ in_gfs, double *rk_yn, double *rk_rt, double *rk_out, const double dt, double *__restrict__ shell_rhs) {
   const int Nxx0 = params.Nxx0;
   const int Nxx1 = params.Nxx1;
@@ -408,7 +509,7 @@ extern "C" int initial_data(const paramstruct *params, double *xx[3], double *in
   if (!params) return NRPY_ERR_NULL;
   if (!in_gfs) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(2, 64, 4, 1);
+  const dim3 block = nrpy_block(3, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx_plus_2NGHOSTS0, params->Nxx_plus_2NGHOSTS1, params->Nxx_plus_2NGHOSTS2));
   hipLaunchKernelGGL(initial_data__gpu, grid, block, 0, stream, *params, xx[0], xx[1], xx[2], in_gfs);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -470,7 +571,7 @@ extern "C" int rhs_eval_vjp_pointwise(const paramstruct *params, const double *i
   if (!params) return NRPY_ERR_NULL;
   if (!in_gfs || !cot_rhs_gfs || !vjp_G) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(3, 64, 4, 1);
+  const dim3 block = nrpy_block(4, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2));
   hipLaunchKernelGGL(rhs_eval_vjp_pointwise__gpu, grid, block, 0, stream, *params, in_gfs, cot_rhs_gfs, vjp_G);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -504,7 +605,7 @@ extern "C" int rhs_eval_vjp_transpose(const paramstruct *params, const double *v
   if (!params) return NRPY_ERR_NULL;
   if (!vjp_G || !cot_in_gfs) return NRPY_ERR_NULL;
   if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
-  const dim3 block = nrpy_block(4, 64, 4, 1);
+  const dim3 block = nrpy_block(5, 64, 4, 1);
   const dim3 grid(nrpy_nblocks(block, params->Nxx_plus_2NGHOSTS0, params->Nxx_plus_2NGHOSTS1, params->Nxx_plus_2NGHOSTS2));
   hipLaunchKernelGGL(rhs_eval_vjp_transpose__gpu, grid, block, 0, stream, *params, vjp_G, cot_in_gfs);
   return hipGetLastError() == hipSuccess ? 0 : NRPY_ERR_LAUNCH;
@@ -531,17 +632,17 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
   if (!rfmstruct || !params || !bcstruct || !y_n_gfs || !k_odd_gfs || !k_even_gfs ||
       !y_nplus1_running_total_gfs) return NRPY_ERR_NULL;
   int rc;
+  nrpy_gf_parity_args gfp;  // the boundary struct is the grid's: checked before the first substep
+  memset(&gfp, 0, sizeof(gfp));
+  if ((rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, &gfp))) return rc;
   /* substep 0: y_n_gfs -> k_odd_gfs */
   if ((rc = rhs_eval_rk4_substep(0, rfmstruct, params, auxevol_gfs, y_n_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
   /* substep 1: k_odd_gfs -> k_even_gfs */
-  if ((rc = rhs_eval_rk4_substep(1, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_even_gfs, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(1, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_even_gfs, dt, stream))) return rc;
   /* substep 2: k_even_gfs -> k_odd_gfs */
-  if ((rc = rhs_eval_rk4_substep(2, rfmstruct, params, auxevol_gfs, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
-  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, k_odd_gfs, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(2, rfmstruct, params, auxevol_gfs, k_even_gfs, y_n_gfs, y_nplus1_running_total_gfs, k_odd_gfs, dt, stream))) return rc;
   /* substep 3: k_odd_gfs -> y_n_gfs */
-  if ((rc = rhs_eval_rk4_substep(3, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
+  if ((rc = rhs_eval_rk4_substep_edge(3, rfmstruct, params, auxevol_gfs, k_odd_gfs, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
   if ((rc = apply_bcs_curvilinear_composed(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, stream))) return rc;
   return NRPY_OK;
 }
