@@ -534,12 +534,17 @@ TILE_ADDRESS_OUTPUTS = (
 # SIMD whatever it needs, so its loads go far ahead; 2.08 ms at 32). Spherical, 128x128x64:
 # Ricci 107 + 124 -> 69 + 66 us, Lambda-bar 332 -> 222 us, the others even; 72x12x2: 63 -> 57 us
 # for the five. The lane-move group keeps its own order (lds.sink_xshift_values).
+# The aDD,trK kernels that only write right-hand sides, not fused with the RK4 substep, keep the
+# expression's order on Cartesian grids: in the toolkit form, whose 31 array pointers take the
+# scalar registers, the order above spills 316 bytes per lane (150^3: 558 us as it is, 827-975 us
+# in any order tried), and the SENR form has the same statements.
 _RICCI_FIRST, _RICCI_SECOND = {"RbarDD00", "RbarDD01", "RbarDD02"}, {"RbarDD11", "RbarDD12", "RbarDD22"}
 _CURVATURE = {"aDD00", "aDD01", "aDD02", "aDD11", "aDD12", "aDD22", "trK"}
 _METRIC = {"hDD00", "hDD01", "hDD02", "hDD11", "hDD12", "hDD22", "alpha", "cf"}
 _SHIFT = {"betU0", "betU1", "betU2", "lambdaU0", "lambdaU1", "lambdaU2", "vetU0", "vetU1", "vetU2"}
 SCHEDULE_CARTESIAN = ((_RICCI_FIRST, (80, 40, True)), (_RICCI_SECOND, (80, 40, True)),
-                      (_CURVATURE, (40, 16, True)), (_SHIFT, (160, 80, False)))
+                      (_SHIFT, (160, 80, False)))
+SCHEDULE_CARTESIAN_FUSED = SCHEDULE_CARTESIAN + ((_CURVATURE, (40, 16, True)),)
 SCHEDULE_CURVILINEAR = ((_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24, False)),
                         (_CURVATURE, (40, 24, False)), (_METRIC, (40, 24, False)), (_SHIFT, (150, 60, False)))
 # Pass 1 of the vector-Jacobian products, all groups: at 96^3 the RHS VJP 3729 -> 2926 us (its
@@ -547,9 +552,11 @@ SCHEDULE_CURVILINEAR = ((_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24
 SCHEDULE_VJP = (60, 40)
 
 
-def scheduled(body, outputs, CoordSystem):
-    """The body of the kernel that computes ``outputs``, in the order measured best for it."""
-    table = SCHEDULE_CARTESIAN if CoordSystem == "Cartesian" else SCHEDULE_CURVILINEAR
+def scheduled(body, outputs, CoordSystem, fused=False):
+    """The body of the kernel that computes ``outputs``, in the order measured best for it.
+    ``fused``: the kernel goes on to an RK4 substep with them."""
+    table = (SCHEDULE_CURVILINEAR if CoordSystem != "Cartesian" else
+             SCHEDULE_CARTESIAN_FUSED if fused else SCHEDULE_CARTESIAN)
     for outs, how in table:
         if set(outputs) == outs:
             return schedule.reorder(body, *how)
@@ -955,11 +962,12 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
         body = fin.FD_outputC("returnstring", sel, params="outCverbose=False", upwindcontrolvec=betaU)
         group_costs.append(bd.count_body(body))
         step_bodies.append(body)
-        body = scheduled(body, grp, CoordSystem)
         rhs_src += oc.outCfunction(outfile="returnstring", desc="BSSN RHSs of %s" % ", ".join(grp),
-                                   name="rhs_eval_g%d" % k, params=rhs_params, body=body,
+                                   name="rhs_eval_g%d" % k, params=rhs_params,
+                                   body=scheduled(body, grp, CoordSystem),
                                    loopopts="InteriorPoints,Enable_rfm_precompute")
-        kern = bd.fused_rk4_kernel("rhs_eval_rk4_substep_g%d" % k, args_decl, "", body,
+        kern = bd.fused_rk4_kernel("rhs_eval_rk4_substep_g%d" % k, args_decl, "",
+                                   scheduled(body, grp, CoordSystem, fused=True),
                                    loopopts="InteriorPoints,Enable_rfm_precompute")
         group_inputs.append(len(kernel_inputs(kern)))
         fused += kern
