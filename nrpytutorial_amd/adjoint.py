@@ -3,14 +3,15 @@
 The forward RK4 step and its adjoint are both compiled HIP code in the bundle:
 ``rhs_eval_vjp`` (SymPy-derived pointwise adjoint + transposed stencils),
 ``bc_apply_T`` (transpose of the ghost fill) and ``MoL_step_adjoint``, which
-recomputes the three stage states of one step from its starting state and
-runs the four stage adjoints (see the generated code for the algebra). This
-module adds what lies above one step:
+runs the four stage adjoints of one step (see the generated code for the
+algebra). This module adds what lies above one step:
 
 * ``forward_checkpointed``: N steps keeping every K-th state (K ~ sqrt(N));
 * ``backward_checkpointed``: for each segment, last first, recompute its
   states from the checkpoint, then step the cotangent back through them, so
-  memory holds ~2 sqrt(N) states and each forward step is run twice;
+  memory holds ~2 sqrt(N) states and each forward step is run twice; the step
+  adjoints of the linear systems (scalar wave, Maxwell) read no state, and
+  theirs are not recomputed;
 * ``RK4Evolve``: a ``torch.autograd.Function`` wrapping both, so a loss
   written in torch on the final state differentiates through the evolution.
 
@@ -35,6 +36,8 @@ class RK4Adjoint:
             raise NrpyError("bundle %s has no generated adjoint" % b.name)
         self.ev = ev
         self.lib = b.lib
+        # False: MoL_step_adjoint of a linear right-hand side, which needs no states
+        self.reads_state = b.meta.get("step_adjoint_reads_state", True)
         g = ev.g
         n = len(b.evol)
         self.U = [g.empty(n) for _ in range(3)]
@@ -90,11 +93,14 @@ def backward_checkpointed(ev, adj, cps, K, dt, nsteps, lam_T):
     adj.bc_T(lam)
     for start in sorted(cps, reverse=True):
         end = min(start + K, nsteps)
-        ev.y_n.copy_(cps[start])
         states = [cps[start]]
-        for _ in range(start, end - 1):
-            ev.step(dt, 1, use_graph=True)
-            states.append(ev.y_n.clone())
+        if adj.reads_state:
+            ev.y_n.copy_(cps[start])
+            for _ in range(start, end - 1):
+                ev.step(dt, 1, use_graph=True)
+                states.append(ev.y_n.clone())
+        else:
+            states *= end - start
         for s in reversed(states):
             adj.step_back(s, lam, dt)
     return lam

@@ -28,6 +28,7 @@ import sympy as sp
 
 from .. import grid as gri
 from .. import finite_difference as fin
+from .. import loop as lp
 from .. import outputC as oc
 from .. import reference_metric as rfm
 from . import schedule
@@ -282,3 +283,140 @@ def vjp_kernels(name, exprs, upwindcontrolvec, pointwise_loopopts, rfm_args, all
         "  return NRPY_OK;\n"
         "}\n" % (name, len(slots), name, rfm_decl, calls))
     return p1 + p2 + driver, slots, outputs, state_dependent
+
+
+def _linear_coefficients(exprs, slots):
+    """{slot name: {output gridfunction: d(output)/d(slot)}} of a right-hand side that is linear in
+    its slots with coefficients that are the same at every point; None if it is not one."""
+    outs = [_out_name(e.lhs) for e in exprs]
+    rhs = [sp.expand(sp.sympify(e.rhs)) for e in exprs]
+    syms = {str(a): a for r in rhs for a in r.free_symbols}
+    names = {s[0] for s in slots}
+    coeffs = {}
+    for name, kind, _, _ in slots:
+        if kind not in ("value", "deriv"):
+            return None
+        coeffs[name] = {o: c for o, c in ((o, sp.diff(r, syms[name])) for o, r in zip(outs, rhs)) if c != 0}
+        for c in coeffs[name].values():
+            if any(str(a) in names or gri.variable_type(a) != "Cparameter" for a in c.free_symbols):
+                return None
+    return coeffs
+
+
+# The ghost fill of an outer boundary: layers 1 and 2 from the three interior points next to it.
+_EXTRAPOLATION = ((3, -3, 1), (6, -8, 3))
+
+
+def _edge_terms(weights, d, at):
+    """C statements that add to s, the transposed stencil of one operator along axis d at a point, what
+    the ghost points hand back to it. Ghost layer g holds sum_p W(-g - p) cot(p) over the interior points
+    p = 0, 1 next to the boundary, and point m = 0, 1, 2 gets E_g(m) times that, E the extrapolation
+    above; the cotangents are among those the point's own stencil reads."""
+    lines = []
+    for side in (-1, 1):
+        W = {1: weights.get(side, 0), 2: weights.get(2 * side, 0)}
+        for m in range(3):
+            k0 = _EXTRAPOLATION[0][m] * W[1] + _EXTRAPOLATION[1][m] * W[2]
+            k1 = _EXTRAPOLATION[0][m] * W[2]
+            edge = "NGHOSTS + %d" % m if side < 0 else "Nxx%d + NGHOSTS - %d" % (d, 1 + m)
+            lines.append("if (i%d == %s) s += %s*%s + %s*%s;" % (
+                d, edge, _ccode(k0), at(side * m), _ccode(k1), at(side * (m - 1))))
+    return lines
+
+
+def linear_stage_kernel(exprs, slots, evol):
+    """Source of ``rhs_eval_vjp_rk4_stage``: one stage of the RK4 step adjoint of a right-hand side
+    that is linear with coefficients that are the same at every point, on a grid whose ghost points
+    are all extrapolated ones (None for any other right-hand side).
+
+    Pass 1 of the vector-Jacobian product is then a multiplication by constants, so the transposed
+    stencils read the cotangent itself and the constants join the stencil weights: no vjp_G. The
+    transposed ghost fill is a change of the weights at the three points next to a boundary
+    (_edge_terms), so no ghost cotangent is stored, and the sum w goes straight into the stage's
+    updates, acc_out = acc_in + w and kbar_out = a L + b w. kbar_out is not the array the stencils
+    read."""
+    coeffs = _linear_coefficients(exprs, slots)
+    if coeffs is None:
+        return None
+    invdx = [sp.Symbol("invdx%d" % d, real=True) for d in range(3)]
+    reads, body, sums = {}, [], {}
+
+    def cot(o, off):
+        name = "cot_%s" % o + "".join("_i%d%s%d" % (d, "p" if v > 0 else "m", abs(v)) for d, v in enumerate(off) if v)
+        reads[name] = "VJP_COT_AT(%sGF, %d, %d, %d)" % ((o.upper(),) + tuple(off))
+        return name
+
+    per_gf = {}
+    for name, kind, gf, op in slots:
+        for o, c in sorted(coeffs[name].items()):
+            if kind == "value":
+                term, fac = cot(o, (0, 0, 0)), c
+            else:
+                w, st = fin.compute_fdcoeffs_fdstencl(op)
+                d = int(op[-1])
+                weights = {s[d]: x for x, s in zip(w, st)}
+                if any(s[e] for s in st for e in range(3) if e != d) or max(map(abs, weights)) > 2:
+                    return None                      # _edge_terms: along one axis, two points at most
+                fac = c * (invdx[d]**2 if op.startswith("dDD") else invdx[d])
+
+                def at(v):
+                    return cot(o, tuple(v if e == d else 0 for e in range(3)))
+                if (o, op) not in sums:
+                    sums[o, op] = "t_%s_%s" % (o, op)
+                    body.append("double %s = %s;" % (sums[o, op], " + ".join(
+                        "%s*%s" % (_ccode(sp.Rational(x)), at(-v)) for v, x in sorted(weights.items()))))
+                    body += [l.replace(" s += ", " %s += " % sums[o, op]) for l in _edge_terms(weights, d, at)]
+                term = sums[o, op]
+            per_gf.setdefault(gf, []).append(term if fac == 1 else "%s*%s" % (_ccode(fac), term))
+    if sorted(per_gf) != sorted(evol):
+        return None
+    body = ["const double %s = %s;" % kv for kv in reads.items()] + body
+    body += ["const double w_%s = %s;" % (gf, " + ".join(per_gf[gf])) for gf in evol]
+    # every read of acc_in and L before the first store: the compiler cannot tell the arrays apart
+    body += ["const double acc_%s = acc_in[IDX4(%sGF, i0, i1, i2)], L_%s = S > 0 ? L[IDX4(%sGF, i0, i1, i2)] : 0.0;"
+             % (gf, gf.upper(), gf, gf.upper()) for gf in evol]
+    for gf in evol:
+        body += ["{", "  const double w = S == 3 ? scale * w_%s : w_%s;" % (gf, gf),
+                 "  acc_out[IDX4(%sGF, i0, i1, i2)] = acc_%s + w;" % (gf.upper(), gf),
+                 "  if (S > 0) kbar_out[IDX4(%sGF, i0, i1, i2)] = a * L_%s + b * w;" % (gf.upper(), gf), "}"]
+    body = "\n".join(body) + "\n"
+    unpack = "".join("  const %s %s = params.%s;\n" % (lp._ctype(t), n, n) for n, t in lp._used_cparams(body)
+                     if not n.startswith("Nxx"))
+    unpack += "".join("  const int %s%d = params.%s%d;\n" % (n, d, n, d) for n in ("Nxx", "Nxx_plus_2NGHOSTS")
+                      for d in range(3))
+    args = ("const double *cot, const double *L, const double *acc_in, double *acc_out, double *%skbar_out, "
+            "const double scale, const double a, const double b")
+    return r"""
+// A cotangent array, 0 outside the interior; the load stays in range as VJP_G_AT's does.
+#define VJP_COT_AT(gf, o0, o1, o2)                                                                  \
+  nrpy_vjp_select((i0) + (o0) >= NGHOSTS && (i0) + (o0) < Nxx0 + NGHOSTS && (i1) + (o1) >= NGHOSTS && \
+                      (i1) + (o1) < Nxx1 + NGHOSTS && (i2) + (o2) >= NGHOSTS &&                     \
+                      (i2) + (o2) < Nxx2 + NGHOSTS,                                                 \
+                  cot[IDX4(gf, (i0) + (o0), (i1) + (o1), (i2) + (o2))])
+// One stage of the RK4 step adjoint: w = (transposed ghost fill and stencils of rhs_eval) cot, times
+// scale in stage 3 (whose kbar is scale L). Bound by its arrays: five read or written per gridfunction
+// (three in stages 3 and 0) besides the stencil's neighbours, which the caches hold. Scalar wave at
+// 128^3: 30 us a stage; slots, transposed stencils, ghost transpose, clearing and the update as
+// launches of their own took 18 + 35 + 12 + 6 + 26 us. One point a lane and 64 x 4 tiles, as the
+// forward substep: neighbours along x in the same cache lines.
+template <int S>
+__global__ void __launch_bounds__(256) rhs_eval_vjp_rk4_stage__gpu(const paramstruct params, """ + args % "__restrict__ " + r""") {
+""" + unpack + _indent(r"""NRPY_BLOCK_COORDS(Nxx0, Nxx1, Nxx2);
+const int i0 = NGHOSTS + nrpy_bx*(int)blockDim.x + (int)threadIdx.x;
+const int i1 = NGHOSTS + nrpy_by*(int)blockDim.y + (int)threadIdx.y;
+const int i2 = NGHOSTS + nrpy_bz*(int)blockDim.z + (int)threadIdx.z;
+if (i0 >= Nxx0 + NGHOSTS || i1 >= Nxx1 + NGHOSTS || i2 >= Nxx2 + NGHOSTS) return;
+""" + body) + r"""}
+static int rhs_eval_vjp_rk4_stage(const int S, const paramstruct *params, """ + args % "" + r""", hipStream_t stream) {
+  const dim3 block(64, 4, 1);
+  const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2));
+  switch (S) {
+""" + "".join("    case %d: hipLaunchKernelGGL(rhs_eval_vjp_rk4_stage__gpu<%d>, grid, block, 0, stream, *params, cot, L, "
+              "acc_in, acc_out, kbar_out, scale, a, b); break;\n" % (s, s) for s in range(4)) + r"""  }
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+"""
+
+
+def _indent(text):
+    return "".join("  " + l + "\n" for l in text.splitlines())

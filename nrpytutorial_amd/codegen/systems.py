@@ -279,68 +279,45 @@ def _mol_batch_glue(n_ricci, n_rhs, detg_stage):
         "  *out = g;\n  return NRPY_OK;\n}\n")
 
 
-def _mol_adjoint_glue(has_rfm_vjp, state_dependent, writes_all):
+def _mol_adjoint_glue(stage_kernel):
     """MoL_step_adjoint: the adjoint of one RK4 step (diagonal schedule, ghost fill after
-    every substep) for systems whose step is [RHS + update -> ghost fill] per substep.
+    every substep) for systems whose step is [RHS + update -> ghost fill] per substep and whose
+    right-hand side has a ``stage_kernel`` (adjoint.linear_stage_kernel).
 
     With u the interior of y_n and E the ghost fill, the step is
       k1 = R(E u), u1 = u + dt/2 k1, k2 = R(E u1), u2 = u + dt/2 k2, k3 = R(E u2),
       u3 = u + dt k3, k4 = R(E u3), u_new = u + dt/6 (k1 + 2 k2 + 2 k3 + k4),
-    so for the cotangent L of u_new, with w_s = E^T R'(E u_s)^T kbar_s:
+    so for the cotangent L of u_new, with w_s = E^T R^T kbar_s (R is linear, so its transpose does
+    not depend on the state):
       kbar4 = dt/6 L, kbar3 = dt/3 L + dt w3, kbar2 = dt/3 L + dt/2 w2, kbar1 = dt/6 L + dt/2 w1,
-      L_n = L + w3 + w2 + w1 + w0.
-    When the right-hand side depends on the state (state_dependent), the stage states are
-    recomputed from y_n with the forward substep kernels; for a linear right-hand side the
-    adjoint does not read them. When the VJP writes every evolved gridfunction
-    (writes_all), its output needs no clearing."""
-    rfm_arg = "rfmstruct, " if has_rfm_vjp else ""
-    vjp = (("" if writes_all else "  if ((rc = nrpy_fill(n, w, 0.0, stream))) return rc;\n") +
-           "  if ((rc = rhs_eval_vjp(" + rfm_arg + "params, auxevol_gfs, STATE, kbar, vjp_G, w, nullptr, stream))) "
-           "return rc;\n"
-           "  if ((rc = nrpy_stage_apply_T(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, w, stream))) return rc;\n")
-    if state_dependent:
-        recompute = (
-            "  double *yn = (double *)y_n_gfs;  // substeps 0-2 read y_n only\n"
-            "  if ((rc = rhs_eval_rk4_substep(0, rfmstruct, params, auxevol_gfs, yn, yn, rt, U1, dt, stream))) "
-            "return rc;\n"
-            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U1, stream))) return rc;\n"
-            "  if ((rc = rhs_eval_rk4_substep(1, rfmstruct, params, auxevol_gfs, U1, yn, rt, U2, dt, stream))) "
-            "return rc;\n"
-            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U2, stream))) return rc;\n"
-            "  if ((rc = rhs_eval_rk4_substep(2, rfmstruct, params, auxevol_gfs, U2, yn, rt, U3, dt, stream))) "
-            "return rc;\n"
-            "  if ((rc = nrpy_stage_fill(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, U3, stream))) return rc;\n")
-        states = ("U3", "U2", "U1", "y_n_gfs")
-    else:
-        recompute = "  (void)U1; (void)U2; (void)U3; (void)rt;  // linear right-hand side: the adjoint ignores the state\n"
-        states = ("y_n_gfs",) * 4
+      L_n = L + w3 + w2 + w1 + w0."""
+    if stage_kernel is None:
+        raise ValueError("MoL_step_adjoint: the right-hand side is not linear with constant coefficients")
+    stages = ((3, "lambda_gfs", "lambda_gfs", "acc", "kbar", "dt / 6.0, dt / 3.0, dt"),
+              (2, "kbar", "acc", "acc", "U1", "1.0, dt / 3.0, dt / 2.0"),
+              (1, "U1", "acc", "acc", "kbar", "1.0, dt / 6.0, dt / 2.0"),
+              (0, "kbar", "acc", "lambda_gfs", "nullptr", "1.0, 0.0, 0.0"))
     return (
+        stage_kernel +
         "// Adjoint of one RK4 step. On entry lambda_gfs holds the cotangent of y_{n+1} (interior points;\n"
         "// ghost cotangents zero), y_n_gfs the state at the start of the step with its ghosts filled. On\n"
         "// exit lambda_gfs holds the cotangent of y_n. U1, U2, U3, rt, acc, kbar, w are caller-allocated\n"
-        "// scratch arrays of NUM_EVOL_GFS gridfunctions; vjp_G has the rhs_eval_vjp slot count.\n"
+        "// scratch arrays of NUM_EVOL_GFS gridfunctions; vjp_G has the rhs_eval_vjp slot count. (The\n"
+        "// right-hand side is linear: of them only U1, acc and kbar are used, and y_n_gfs is not read.)\n"
         'extern "C" int MoL_step_adjoint(const rfm_struct *rfmstruct, const paramstruct *params,\n'
         "    const bc_struct *bcstruct, const double *y_n_gfs, double *lambda_gfs, double *U1, double *U2,\n"
         "    double *U3, double *rt, double *acc, double *kbar, double *w, double *vjp_G, double *auxevol_gfs,\n"
         "    const double dt, hipStream_t stream) {\n"
         "  if (!rfmstruct || !params || !bcstruct || !y_n_gfs || !lambda_gfs || !U1 || !U2 || !U3 || !rt ||\n"
         "      !acc || !kbar || !w || !vjp_G) return NRPY_ERR_NULL;\n"
-        "  int rc;\n"
-        "  const size_t n = (size_t)NUM_EVOL_GFS * params->Nxx_plus_2NGHOSTS0 * params->Nxx_plus_2NGHOSTS1 *\n"
-        "                   params->Nxx_plus_2NGHOSTS2;\n"
-        + recompute +
-        "  /* stage 4: kbar4 = dt/6 L */\n"
-        "  if ((rc = nrpy_lincomb(n, kbar, dt / 6.0, lambda_gfs, 0.0, nullptr, stream))) return rc;\n"
-        + vjp.replace("STATE", states[0]) +
-        "  /* acc = L + w3; kbar3 = dt/3 L + dt w3 */\n"
-        "  if ((rc = nrpy_adjoint_combine(n, acc, lambda_gfs, w, kbar, dt / 3.0, dt, 1, stream))) return rc;\n"
-        + vjp.replace("STATE", states[1]) +
-        "  if ((rc = nrpy_adjoint_combine(n, acc, lambda_gfs, w, kbar, dt / 3.0, dt / 2.0, 0, stream))) return rc;\n"
-        + vjp.replace("STATE", states[2]) +
-        "  if ((rc = nrpy_adjoint_combine(n, acc, lambda_gfs, w, kbar, dt / 6.0, dt / 2.0, 0, stream))) return rc;\n"
-        + vjp.replace("STATE", states[3]) +
-        "  /* L_n = acc + w0 */\n"
-        "  return nrpy_lincomb(n, lambda_gfs, 1.0, acc, 1.0, w, stream);\n"
+        "  (void)auxevol_gfs;\n"
+        "  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;\n"
+        "  nrpy_gf_parity_args gfp;\n"
+        "  int rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, lambda_gfs, &gfp);\n"
+        "  if (rc) return rc;\n"
+        + "".join("  if ((rc = rhs_eval_vjp_rk4_stage(%d, params, %s, lambda_gfs, %s, %s, %s, %s, stream))) "
+                  "return rc;\n" % st for st in stages) +
+        "  return NRPY_OK;\n"
         "}\n")
 
 
@@ -657,16 +634,17 @@ def scalarwave_cartesian():
     fused += _fused_shell_kernel(fused, "rhs_eval_rk4_substep") + _fused_shell_launcher(
         "rhs_eval_rk4_substep", "const paramstruct *params, const double *in_gfs", "*params, in_gfs")
     id_src = _initial_data_kernel([swid.uu_ID, swid.vv_ID], ["uu", "vv"])
-    vjp_src, slots, vouts, vdep = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
+    vjp_src, slots, _, _ = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
     som_src, som_meta = _sommerfeld_glue(4, "rhs_eval(params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
                                          shell_call=SHELL_CALL)
     pre, meta = _header(3, stage_offsets([body]))
     parts = [pre, bd.coord_host_functions("Cartesian"), '#include "../nrpy_runtime.h"', bd.rfm_struct_code(),
              rhs_src, fused, id_src, vjp_src,
              _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", edge=True),
-             _mol_adjoint_glue(False, vdep, sorted(vouts["EVOL"]) == sorted(gri.gridfunction_lists()[0])), som_src]
+             _mol_adjoint_glue(adj.linear_stage_kernel(exprs, slots, gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]
+    meta["step_adjoint_reads_state"] = False
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta.update({"bundle": "scalarwave_cartesian", "CoordSystem": "Cartesian", "rfm_tables": [],
                  "kernels": ["rhs_eval", "initial_data"], "has_ricci": False, "has_detg": False})
@@ -719,12 +697,13 @@ def maxwell_cartesian():
     som_src, som_meta = _sommerfeld_glue(2, "rhs_eval(params, RK_INPUT_GFS, RK_OUTPUT_GFS, stream)",
                                          shell_call=SHELL_CALL)
     pre, meta = _header(3, stage_offsets([body]))
-    vjp_src, slots, vouts, vdep = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
+    vjp_src, slots, _, _ = adj.vjp_kernels("rhs_eval", exprs, "", "InteriorPoints", "")
     parts = [pre, coords, '#include "../nrpy_runtime.h"', bd.rfm_struct_code(), rhs_src, con_src, fused, id_src,
              vjp_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", edge=True),
-             _mol_adjoint_glue(False, vdep, sorted(vouts["EVOL"]) == sorted(gri.gridfunction_lists()[0])), som_src]
+             _mol_adjoint_glue(adj.linear_stage_kernel(exprs, slots, gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]
+    meta["step_adjoint_reads_state"] = False
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta["kernel_ids"] = dict(bd.lp.KERNEL_IDS)
     meta.update({"bundle": "maxwell_cartesian", "family": "maxwell", "CoordSystem": "Cartesian", "rfm_tables": [],

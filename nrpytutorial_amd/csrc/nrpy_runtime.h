@@ -82,7 +82,7 @@ struct nrpy_fill_list {
   nrpy_fill_row *d_rows = nullptr;
   nrpy_fill_term *d_terms = nullptr;
 };
-// Transpose of a set of ghost rows (CSR over the interior points they read).
+// Transpose of the composed ghost map (CSR over the interior points they read).
 struct nrpy_transpose_list {
   int n = 0;
   std::vector<int> h_src, h_rowptr, h_ghost, h_negmask;
@@ -121,8 +121,8 @@ struct bc_struct {
   std::vector<double> h_coeff;
   // the map as the fill kernel reads it: every ghost point, and those a stencil reaches
   nrpy_fill_list fill_all, fill_stage;
-  // its transpose, for bc_apply_T, and that of the reached ghosts, for the step adjoint
-  nrpy_transpose_list trans_all, trans_stage;
+  // its transpose, for bc_apply_T
+  nrpy_transpose_list trans;
   // right-hand-side scratch of the fused Sommerfeld RK4 step (nrpy_sommerfeld_scratch)
   double *d_som_rhs = nullptr;
   size_t som_rhs_n = 0;
@@ -278,13 +278,10 @@ static bool nrpy_stage_reads(const paramstruct *params, int idx) {
   return false;
 }
 
-static void nrpy_build_transpose(const bc_struct *bc, const int Ntot, const std::vector<char> &take,
-                                 nrpy_transpose_list *T) {
+static void nrpy_build_transpose(const bc_struct *bc, const int Ntot, nrpy_transpose_list *T) {
   // counting sort of the entries by the interior point they read
   std::vector<int> first(Ntot + 1, 0);
-  for (int r = 0; r < bc->nghost; r++)
-    if (take[r])
-      for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) first[bc->h_src[k] + 1]++;
+  for (const int src : bc->h_src) first[src + 1]++;
   T->h_rowptr.assign(1, 0);
   for (int i = 0; i < Ntot; i++) {
     if (first[i + 1]) {
@@ -298,13 +295,12 @@ static void nrpy_build_transpose(const bc_struct *bc, const int Ntot, const std:
   T->h_coeff.resize(n);
   T->h_negmask.resize(n);
   for (int r = 0; r < bc->nghost; r++)
-    if (take[r])
-      for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) {
-        const int at = first[bc->h_src[k]]++;
-        T->h_ghost[at] = bc->h_gdest[r];
-        T->h_coeff[at] = bc->h_coeff[k];
-        T->h_negmask[at] = bc->h_negmask[k];
-      }
+    for (int k = bc->h_rowptr[r]; k < bc->h_rowptr[r + 1]; k++) {
+      const int at = first[bc->h_src[k]]++;
+      T->h_ghost[at] = bc->h_gdest[r];
+      T->h_coeff[at] = bc->h_coeff[k];
+      T->h_negmask[at] = bc->h_negmask[k];
+    }
   T->n = (int)T->h_src.size();
 }
 
@@ -467,8 +463,7 @@ static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
   bc->nterms = (int)bc->h_src.size();
   std::vector<char> all(bc->nghost, 1), reached(bc->nghost);
   for (int r = 0; r < bc->nghost; r++) reached[r] = nrpy_stage_reads(params, bc->h_gdest[r]);
-  nrpy_build_transpose(bc, Ntot, all, &bc->trans_all);
-  nrpy_build_transpose(bc, Ntot, reached, &bc->trans_stage);
+  nrpy_build_transpose(bc, Ntot, &bc->trans);
   nrpy_build_fill(params, bc, anchor, all, &bc->fill_all);
   nrpy_build_fill(params, bc, anchor, reached, &bc->fill_stage);
   return NRPY_OK;
@@ -497,13 +492,11 @@ extern "C" void bcstruct_free(bc_struct *bc) {
     (void)hipFree(L->d_rows);
     (void)hipFree(L->d_terms);
   }
-  for (nrpy_transpose_list *T : {&bc->trans_all, &bc->trans_stage}) {
-    (void)hipFree(T->d_src);
-    (void)hipFree(T->d_rowptr);
-    (void)hipFree(T->d_ghost);
-    (void)hipFree(T->d_coeff);
-    (void)hipFree(T->d_negmask);
-  }
+  (void)hipFree(bc->trans.d_src);
+  (void)hipFree(bc->trans.d_rowptr);
+  (void)hipFree(bc->trans.d_ghost);
+  (void)hipFree(bc->trans.d_coeff);
+  (void)hipFree(bc->trans.d_negmask);
   (void)hipFree(bc->d_som_rhs);
   delete bc;
 }
@@ -607,12 +600,12 @@ extern "C" int bcstruct_create(const paramstruct *params, double *xx[3], bc_stru
   for (nrpy_fill_list *L : {&bc->fill_all, &bc->fill_stage})
     ok = ok && nrpy_upload(&L->d_rows, L->h_rows.data(), L->h_rows.size()) &&
          nrpy_upload(&L->d_terms, L->h_terms.data(), L->h_terms.size());
-  for (nrpy_transpose_list *T : {&bc->trans_all, &bc->trans_stage})
-    ok = ok && nrpy_upload(&T->d_src, T->h_src.data(), T->h_src.size()) &&
-         nrpy_upload(&T->d_rowptr, T->h_rowptr.data(), T->h_rowptr.size()) &&
-         nrpy_upload(&T->d_ghost, T->h_ghost.data(), T->h_ghost.size()) &&
-         nrpy_upload(&T->d_coeff, T->h_coeff.data(), T->h_coeff.size()) &&
-         nrpy_upload(&T->d_negmask, T->h_negmask.data(), T->h_negmask.size());
+  nrpy_transpose_list &T = bc->trans;
+  ok = ok && nrpy_upload(&T.d_src, T.h_src.data(), T.h_src.size()) &&
+       nrpy_upload(&T.d_rowptr, T.h_rowptr.data(), T.h_rowptr.size()) &&
+       nrpy_upload(&T.d_ghost, T.h_ghost.data(), T.h_ghost.size()) &&
+       nrpy_upload(&T.d_coeff, T.h_coeff.data(), T.h_coeff.size()) &&
+       nrpy_upload(&T.d_negmask, T.h_negmask.data(), T.h_negmask.size());
   if (!ok) {
     bcstruct_free(bc);
     return NRPY_ERR_ALLOC;
@@ -916,8 +909,12 @@ __global__ void nrpy_clear_ghosts_kernel(int nghost, const int *__restrict__ gde
   gfs[(size_t)(t / nghost) * Ntot + gdest[t % nghost]] = 0.0;
 }
 
-static int nrpy_transpose_launch(const paramstruct *params, const bc_struct *bc, const nrpy_transpose_list &T,
-                                 const int NUM_GFS, const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
+// Transpose of apply_bcs_curvilinear(_composed): folds the cotangents held at ghost
+// points onto the interior points the ghost values were computed from, then zeroes
+// the ghost cotangents. No counterpart in the reference (it has no adjoint).
+extern "C" int bc_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
+                          const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
+  if (!bc) return NRPY_ERR_NULL;
   nrpy_gf_parity_args gfp;
   memset(&gfp, 0, sizeof(gfp));
   int rc = nrpy_bc_check(params, bc, NUM_GFS, gfs_parity, cot_gfs, &gfp);
@@ -925,6 +922,7 @@ static int nrpy_transpose_launch(const paramstruct *params, const bc_struct *bc,
   if (bc->nghost == 0) return NRPY_OK;
   const size_t Ntot = (size_t)bc->N[0] * bc->N[1] * bc->N[2];
   const int B = 256;
+  const nrpy_transpose_list &T = bc->trans;
   if (T.n > 0) {
     const size_t work = (size_t)T.n * NUM_GFS;
     hipLaunchKernelGGL(nrpy_bc_transpose_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream, T.n,
@@ -934,23 +932,6 @@ static int nrpy_transpose_launch(const paramstruct *params, const bc_struct *bc,
   hipLaunchKernelGGL(nrpy_clear_ghosts_kernel, dim3((unsigned)((work + B - 1) / B)), dim3(B), 0, stream,
                      bc->nghost, bc->d_gdest, NUM_GFS, Ntot, cot_gfs);
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
-}
-
-// Transpose of apply_bcs_curvilinear(_composed): folds the cotangents held at ghost
-// points onto the interior points the ghost values were computed from, then zeroes
-// the ghost cotangents. No counterpart in the reference (it has no adjoint).
-extern "C" int bc_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
-                          const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
-  if (!bc) return NRPY_ERR_NULL;
-  return nrpy_transpose_launch(params, bc, bc->trans_all, NUM_GFS, gfs_parity, cot_gfs, stream);
-}
-
-// The same for a cotangent that a right-hand side's transposed stencils wrote: it is zero at
-// the ghost points they do not reach, so only the others are folded.
-static int nrpy_stage_apply_T(const paramstruct *params, const bc_struct *bc, const int NUM_GFS,
-                              const int8_t *gfs_parity, double *cot_gfs, hipStream_t stream) {
-  if (!bc) return NRPY_ERR_NULL;
-  return nrpy_transpose_launch(params, bc, bc->trans_stage, NUM_GFS, gfs_parity, cot_gfs, stream);
 }
 
 __global__ void nrpy_lincomb_kernel(size_t n, double *__restrict__ out, double a, const double *__restrict__ x,
