@@ -16,8 +16,8 @@ extern "C" {
  * RbarDD components into auxevol_gfs at interior points. */
 int Ricci_eval(const rfm_struct *rfmstruct, const paramstruct *params, const double *in_gfs, double *auxevol_gfs,
                hipStream_t stream);
-/* Ricci_eval runs as Ricci_eval_g0 (RbarDD00, 01, 02) and Ricci_eval_g1 (RbarDD11, 12, 22)
- * (groups listed in <bundle>.json "ricci_groups"). */
+/* The same by groups of components: g0 RbarDD00, 01, 02 and g1 RbarDD11, 12, 22 (listed in
+ * <bundle>.json "ricci_groups"). */
 int Ricci_eval_g0(const rfm_struct *rfmstruct, const paramstruct *params, const double *in_gfs, double *auxevol_gfs,
                   hipStream_t stream);
 int Ricci_eval_g1(const rfm_struct *rfmstruct, const paramstruct *params, const double *in_gfs, double *auxevol_gfs,

@@ -261,16 +261,20 @@ def bssn_etk(bundle_name="bssn_etk"):
     # Ricci tensor (BaikalETK_C_kernels_codegen.py:306-330)
     ric_names = ["RbarDD%d%d" % (i, j) for i in range(3) for j in range(i, 3)]
     ric_exprs = {"RbarDD%d%d" % (i, j): RbarDD[i][j] for i in range(3) for j in range(i, 3)}
+    # one kernel of all components; the groups' kernels are the SENR-layout bundle's counterparts
     kernels, flops = [], 0
-    for k, grp in enumerate(ricci_groups(ric_names)):
+    lp.MIN_WAVES_PER_EU["Baikal_BSSN_Ricci"] = 2
+    for k, grp in enumerate(ricci_groups(ric_names) + [ric_names]):
         body = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
                                                for n in grp], params="outCverbose=False")
-        flops += bd.count_body(body)["flops"]
-        name = "Baikal_BSSN_Ricci_g%d" % k
-        body = scheduled(body, grp, "Cartesian")
-        text, launch = etk_kernel(name, "Ricci tensor components %s" % ", ".join(grp), body, table)
+        name = "Baikal_BSSN_Ricci" + ("_g%d" % k if grp is not ric_names else "")
+        if grp is ric_names:
+            flops = bd.count_body(body)["flops"]
+        text, launch = etk_kernel(name, "Ricci tensor components %s" % ", ".join(grp),
+                                  scheduled(body, grp, "Cartesian"), table)
         src.append(text)
-        kernels.append((name, launch))
+        if grp is ric_names:
+            kernels.append((name, launch))
     fname = "Baikal_BSSN_Ricci_FD_order_%d" % FD_ORDER
     c, p = entry_point(fname, "Ricci tensor RbarDD at interior points (BaikalETK_BSSN_Ricci_FD_order_4)",
                        ["const double *const *evol_gfs", "double *const *auxevol_gfs"],

@@ -232,7 +232,7 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
             meta)
 
 
-def _mol_batch_glue(n_ricci, n_rhs, detg_stage):
+def _mol_batch_glue(n_rhs, detg_stage):
     """MoL_batch_step / MoL_batch_graph_create: one RK4 step of every instance of a batch,
     the diagonal schedule with one launch per kernel per substep for all instances."""
     sub = ""
@@ -241,9 +241,7 @@ def _mol_batch_glue(n_ricci, n_rhs, detg_stage):
                                 ("NRPY_BATCH_ROLE_KEVEN", "NRPY_BATCH_ROLE_KODD"),
                                 ("NRPY_BATCH_ROLE_KODD", "NRPY_BATCH_ROLE_YN"))):
         sub += "  /* substep %d */\n" % s
-        for k in range(n_ricci):
-            sub += ("  if ((rc = Ricci_eval_g%d_batched(b, %s, NRPY_BATCH_ROLE_AUXEVOL, stream))) return rc;\n"
-                    % (k, i))
+        sub += "  if ((rc = Ricci_eval_batched(b, %s, NRPY_BATCH_ROLE_AUXEVOL, stream))) return rc;\n" % i
         for k in range(n_rhs):
             sub += ("  if ((rc = rhs_eval_rk4_substep_g%d_batched(%d, b, NRPY_BATCH_ROLE_AUXEVOL, %s, NRPY_BATCH_ROLE_YN, "
                     "NRPY_BATCH_ROLE_RT, %s, stream))) return rc;\n" % (k, s, i, o))
@@ -515,14 +513,20 @@ TILE_ADDRESS_OUTPUTS = (
 # expression's order on Cartesian grids: in the toolkit form, whose 31 array pointers take the
 # scalar registers, the order above spills 316 bytes per lane (150^3: 558 us as it is, 827-975 us
 # in any order tried), and the SENR form has the same statements.
+# The Ricci tensor as one kernel reads the metric's stencils once where the two groups read them
+# twice. It fits two waves per SIMD with short distances only (192^3: 487 + 460 us as two kernels,
+# 636-708 us as one at 16 to 34, 913-947 us at 36 and above, where it runs one wave; 101x67x45:
+# 59 -> 40 us). On spherical grids, 128x128x64, 134 -> 118 us, 72x12x2 with the gap between them
+# 17 -> 11 us. The groups' kernels remain for callers of their own.
 _RICCI_FIRST, _RICCI_SECOND = {"RbarDD00", "RbarDD01", "RbarDD02"}, {"RbarDD11", "RbarDD12", "RbarDD22"}
+_RICCI = _RICCI_FIRST | _RICCI_SECOND
 _CURVATURE = {"aDD00", "aDD01", "aDD02", "aDD11", "aDD12", "aDD22", "trK"}
 _METRIC = {"hDD00", "hDD01", "hDD02", "hDD11", "hDD12", "hDD22", "alpha", "cf"}
 _SHIFT = {"betU0", "betU1", "betU2", "lambdaU0", "lambdaU1", "lambdaU2", "vetU0", "vetU1", "vetU2"}
-SCHEDULE_CARTESIAN = ((_RICCI_FIRST, (80, 40, True)), (_RICCI_SECOND, (80, 40, True)),
+SCHEDULE_CARTESIAN = ((_RICCI, (30, 16, False)), (_RICCI_FIRST, (80, 40, True)), (_RICCI_SECOND, (80, 40, True)),
                       (_SHIFT, (160, 80, False)))
 SCHEDULE_CARTESIAN_FUSED = SCHEDULE_CARTESIAN + ((_CURVATURE, (40, 16, True)),)
-SCHEDULE_CURVILINEAR = ((_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24, False)),
+SCHEDULE_CURVILINEAR = ((_RICCI, (100, 50, False)), (_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24, False)),
                         (_CURVATURE, (40, 24, False)), (_METRIC, (40, 24, False)), (_SHIFT, (150, 60, False)))
 # Pass 1 of the vector-Jacobian products, all groups: at 96^3 the RHS VJP 3729 -> 2926 us (its
 # Lambda-bar kernel spilled 364 bytes per lane), the Ricci VJP 1267 -> 1233 us.
@@ -972,22 +976,23 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     ric_groups = ricci_groups(ric_names)
     ricci_params = ("rfm_struct *restrict rfmstruct,const paramstruct *restrict params,"
                     "const REAL *restrict in_gfs,REAL *restrict auxevol_gfs")
-    ricci_src, ricci_costs = "", []
+    ricci_src = ""
     for k, grp in enumerate(ric_groups):
         body_k = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
                                                  for n in grp], params="outCverbose=False")
-        ricci_costs.append(bd.count_body(body_k))
         step_bodies.append(body_k)
         body_k = scheduled(body_k, grp, CoordSystem)
         ricci_src += oc.outCfunction(outfile="returnstring", desc="Evaluate the Ricci tensor components %s"
                                      % ", ".join(grp), name="Ricci_eval_g%d" % k, params=ricci_params, body=body_k,
                                      loopopts="InteriorPoints,Enable_rfm_precompute")
-    calls = "".join("  if ((rc = Ricci_eval_g%d(rfmstruct, params, in_gfs, auxevol_gfs, stream))) return rc;\n" % k
-                    for k in range(len(ric_groups)))
-    ricci_src += ("/* Evaluate the Ricci tensor (%d kernels, one per group of components). */\n"
-                  'extern "C" int Ricci_eval(const rfm_struct *rfmstruct, const paramstruct *params, '
-                  "const double *in_gfs, double *auxevol_gfs, hipStream_t stream) {\n"
-                  "  int rc;\n%s  return NRPY_OK;\n}\n" % (len(ric_groups), calls))
+    if CoordSystem == "Cartesian":
+        bd.lp.MIN_WAVES_PER_EU["Ricci_eval"] = 2
+    body = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
+                                           for n in ric_names], params="outCverbose=False")
+    ricci_cost = bd.count_body(body)
+    ricci_src += oc.outCfunction(outfile="returnstring", desc="Evaluate the Ricci tensor", name="Ricci_eval",
+                                 params=ricci_params, body=scheduled(body, ric_names, CoordSystem),
+                                 loopopts="InteriorPoints,Enable_rfm_precompute")
     print("(BENCH) Ricci codegen %.1fs (%d groups)" % (time.time() - t0, len(ric_groups)), flush=True)
     t0 = time.time()
     h_body = fin.FD_outputC("returnstring", lhrh(lhs=gri.gfaccess("aux_gfs", "H"), rhs=bssncon.H),
@@ -1075,8 +1080,8 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                                              "InteriorPoints,Enable_rfm_precompute", "rfm_struct *restrict rfmstruct,")
     print("(BENCH) VJP codegen %.1fs (%d + %d + %d + %d slots)" % (time.time() - t0, len(vslots), len(rslots),
                                                                   len(dslots), len(hslots)), flush=True)
-    batch_names = (["Ricci_eval_g%d" % k for k in range(len(ric_groups))] +
-                   ["rhs_eval_rk4_substep_g%d" % k for k in range(len(groups))] + ["enforce_detgammabar_constraint"] +
+    batch_names = (["Ricci_eval"] + ["rhs_eval_rk4_substep_g%d" % k for k in range(len(groups))] +
+                   ["enforce_detgammabar_constraint"] +
                    (["enforce_detgammabar_constraint_stage"] if detg_stage else []))
     batch_src, batch_table = bt.batched_kernels(batch_names)
     pre, meta = _header(FD_order // 2 + 1, offsets)
@@ -1085,7 +1090,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
              hvjp_src,
              _mol_glue(True, True, None, "rfmstruct, params, auxevol_gfs, IN", detg_stage),
              bt.instance_struct(), batch_table, '#include "../nrpy_batch.h"', batch_src,
-             _mol_batch_glue(len(ric_groups), len(groups), detg_stage)]
+             _mol_batch_glue(len(groups), detg_stage)]
     meta["rhs_groups"] = groups
     # distinct gridfunctions each group's kernel reads (evolved and RbarDD): its algorithmic
     # traffic is 8 (inputs + 4 outputs) bytes per point
@@ -1100,7 +1105,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     meta["xshift_kernels"] = sorted(lds.XSHIFT_KERNELS)
     meta["tile_addressing"] = dict(sorted(addressing.APPLIED.items()))
     meta["cost"] = {"rhs_eval": {"flops": sum(c["flops"] for c in group_costs), "groups": group_costs},
-                    "Ricci_eval": {"flops": sum(c["flops"] for c in ricci_costs), "groups": ricci_costs},
+                    "Ricci_eval": ricci_cost,
                     "Hamiltonian_constraint": bd.count_body(h_body),
                     "momentum_constraint": bd.count_body(mu_body),
                     "enforce_detgammabar_constraint": bd.count_body(detg_body)}
