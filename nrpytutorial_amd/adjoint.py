@@ -139,12 +139,6 @@ def RK4Evolve():
     return _RK4Evolve
 
 
-def torch_mul(x, a, out):
-    """out = a * x in one device pass."""
-    import torch
-    torch.mul(x, a, out=out)
-
-
 class BSSNStepAdjoint:
     """Adjoint of the BSSN RK4 step on one Evolution, orchestrated from the host over the
     bundle's kernels. Each substep of the forward step is
@@ -166,12 +160,14 @@ class BSSNStepAdjoint:
         g = ev.g
         n = len(b.evol)
         self.n = n
-        self.X = [g.empty(n) for _ in range(4)]          # X_0 = y_n copy, X_1..X_3
-        self.P = [g.empty(n) for _ in range(5)]          # P_1..P_4 (index 1..4)
+        self.X = [None] + [g.empty(n) for _ in range(3)]     # X_0 is y_n, X_1..X_3
+        # P_1..P_4 (index 1..4; 0 holds a cotangent that has to be copied); of P_1..P_3 only the gridfunctions that the enforcement reads
+        self.P = [g.empty(n) for _ in range(5)]
+        self.metric = slice(b.evol.index("hDD00"), b.evol.index("hDD22") + 1)
         self.Ric = [g.empty(6) for _ in range(4)]
-        self.rt, self.yw = g.empty(n), g.empty(n)
-        self.acc, self.c, self.cX, self.tmp = (g.empty(n) for _ in range(4))
-        self.ck = [g.empty(n) for _ in range(4)]
+        self.rt = g.empty(n)
+        self.acc, self.cX, self.tmp = (g.empty(n) for _ in range(3))
+        self.ck = g.empty(n)
         self.cRic = g.empty(6)
         nslots = max(len(b.meta["vjp_slots"]), len(b.meta["ricci_vjp_slots"]), len(b.meta["detg_vjp_slots"]),
                      len(b.meta.get("hamiltonian_vjp_slots", [])))
@@ -192,6 +188,9 @@ class BSSNStepAdjoint:
         L.bc_apply_T.restype = ctypes.c_int
         L.bc_apply_T.argtypes = [_VP, _VP, ctypes.c_int, _VP, _VP, _VP]
         L.rhs_eval_rk4_substep.restype = ctypes.c_int
+        for f, a in ((L.nrpy_lincomb, [ctypes.c_size_t, _VP, ctypes.c_double, _VP, ctypes.c_double, _VP, _VP]),
+                     (L.nrpy_adjoint_combine, [ctypes.c_size_t] + [_VP] * 4 + [ctypes.c_double] * 2 + [ctypes.c_int, _VP])):
+            f.restype, f.argtypes = ctypes.c_int, a
 
     def _E(self, y):
         self.ev.apply_bcs(y, composed=True)
@@ -220,40 +219,53 @@ class BSSNStepAdjoint:
         for a, b in self.ricci_in:
             out[a:b].add_(self.tmp[a:b])
 
+    def _usable(self, a):
+        """Whether the kernels can take the tensor a as it is (others are copied in and out)."""
+        return (a.dtype, a.device, a.shape, a.is_contiguous()) == (self.cX.dtype, self.cX.device, self.cX.shape, True)
+
     def recompute(self, y_n, dt):
+        """Stage states X_0..X_3, their Ricci tensors, and P_1..P_4; y_n is read only."""
         ev, g, L = self.ev, self.ev.g, self.lib
-        self.X[0].copy_(y_n)
-        self.yw.copy_(y_n)
+        self.X[0] = y_n
         for s in range(4):
             X = self.X[s]
             check(L.Ricci_eval(g.rfm, g.pp(), ptr(X), ptr(self.Ric[s]), ev.s()), "Ricci_eval")
-            out = self.yw if s == 3 else self.X[s + 1]
-            check(L.rhs_eval_rk4_substep(s, g.rfm, g.pp(), ptr(self.Ric[s]), ptr(X), ptr(self.yw), ptr(self.rt),
+            out = self.P[4] if s == 3 else self.X[s + 1]
+            check(L.rhs_eval_rk4_substep(s, g.rfm, g.pp(), ptr(self.Ric[s]), ptr(X), ptr(y_n), ptr(self.rt),
                                          ptr(out), float(dt), ev.s()), "rhs_eval_rk4_substep")
             self._E(out)
-            self.P[s + 1].copy_(out)
-            ev.post_bcs(out)
+            if s < 3:                                    # y_{n+1} = D(P_4) itself is not needed
+                self.P[s + 1][self.metric].copy_(out[self.metric])
+                ev.post_bcs(out)
 
     def step_back(self, y_n, lam, dt):
         """lam (cotangent of y_{n+1}, full array) <- cotangent of y_n (full array)."""
+        ev, L = self.ev, self.lib
+        given = lam
+        if not self._usable(lam):
+            lam = self.P[0].copy_(lam)
+        if not self._usable(y_n) or y_n.untyped_storage().data_ptr() == lam.untyped_storage().data_ptr():
+            y_n = ev.g.empty(self.n).copy_(y_n)
         self.recompute(y_n, dt)
-        c = self.c
-        c.copy_(lam)
-        self._DT(self.P[4], c)
-        self._ET(c)                                  # cotangent of u4 (interior)
-        self.acc.copy_(c)
+        self._DT(self.P[4], lam)
+        self._ET(lam)                                # cotangent of u4 (interior)
+        size = lam.numel()
+        # lam = c: k_{s+1}'s cotangent is w_s c + b_s (cotangent of u_{s+1}), u_{s+1} = y_n + b_s k_{s+1}
         w = (dt / 6.0, dt / 3.0, dt / 3.0, dt / 6.0)
-        for s in range(4):
-            torch_mul(c, w[s], self.ck[s])
-        coef = (dt / 2.0, dt / 2.0, dt)               # u_{s+1} = y_n + coef[s] * dt-weighted k_{s+1}
+        b = (dt / 2.0, dt / 2.0, dt)
+        check(L.nrpy_lincomb(size, ptr(self.ck), w[3], ptr(lam), 0.0, None, ev.s()), "nrpy_lincomb")
         for s in (3, 2, 1):                         # stage input X_s -> k_{s+1}
-            self._RT(self.X[s], self.Ric[s], self.ck[s], self.cX)
+            self._RT(self.X[s], self.Ric[s], self.ck, self.cX)
             self._DT(self.P[s], self.cX)
             self._ET(self.cX)                        # cotangent of u_s
-            self.acc.add_(self.cX)
-            self.ck[s - 1].add_(self.cX, alpha=coef[s - 1])
-        self._RT(self.X[0], self.Ric[0], self.ck[0], self.cX)
-        lam.copy_(self.cX).add_(self.acc)
+            # acc (= c before the first) += cX and the cotangent of k_s, in one pass
+            check(L.nrpy_adjoint_combine(size, ptr(self.acc), ptr(lam), ptr(self.cX), ptr(self.ck), w[s - 1],
+                                         b[s - 1], int(s == 3), ev.s()), "nrpy_adjoint_combine")
+        self._RT(self.X[0], self.Ric[0], self.ck, self.cX)
+        self.X[0] = None
+        check(L.nrpy_lincomb(size, ptr(lam), 1.0, ptr(self.acc), 1.0, ptr(self.cX), ev.s()), "nrpy_lincomb")
+        if lam is not given:
+            given.copy_(lam)
 
 
 def bssn_hl2_mass_gradient(ev, nsteps, CFL=0.5):

@@ -528,8 +528,11 @@ SCHEDULE_CARTESIAN = ((_RICCI, (30, 16, False)), (_RICCI_FIRST, (80, 40, True)),
 SCHEDULE_CARTESIAN_FUSED = SCHEDULE_CARTESIAN + ((_CURVATURE, (40, 16, True)),)
 SCHEDULE_CURVILINEAR = ((_RICCI, (100, 50, False)), (_RICCI_FIRST, (40, 24, False)), (_RICCI_SECOND, (40, 24, False)),
                         (_CURVATURE, (40, 24, False)), (_METRIC, (40, 24, False)), (_SHIFT, (150, 60, False)))
-# Pass 1 of the vector-Jacobian products, all groups: at 96^3 the RHS VJP 3729 -> 2926 us (its
-# Lambda-bar kernel spilled 364 bytes per lane), the Ricci VJP 1267 -> 1233 us.
+# Pass 1 of the right-hand sides' vector-Jacobian product, all groups: at 96^3 828 -> 538, 395 ->
+# 390 and 1444 -> 929 us (the Lambda-bar kernel spilled 364 bytes per lane). The Ricci tensor's is
+# one kernel on Cartesian grids, in the order its reverse sweep has: 563 us; 297 + 475 us by the
+# forward groups in this order, 1.08 ms as one kernel in it. On spherical grids it is by groups: the
+# whole product takes 189 us at 128x64x32, 232 us with one kernel, and the same at 64x16x2.
 SCHEDULE_VJP = (60, 40)
 
 
@@ -1053,7 +1056,8 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
     # Vector-Jacobian products of the whole RHS (all outputs, inputs in_gfs and RbarDD) and of
     # the Ricci tensor (inputs in_gfs), for adjoints through rhs_eval and Ricci_eval.
     t0 = time.time()
-    # Pass 1 runs per output group, as the forward kernels do; pass 2 per cotangent gridfunction.
+    # Pass 1 of the RHS runs per output group, as the forward kernels do; pass 2 per cotangent
+    # gridfunction.
     # Tile-relative addressing (Cartesian grids), measured on one 96^3 adjoint RK4 step: 38.5 ms
     # without; 37.8 with the transposes in form "xc" (38.3 in "xl"); 36.5 with the RHS pass-1
     # kernels in "xl" as well (41.7 in "xc"); 37.2 with the Ricci pass-1 kernels in "xl" too.
@@ -1068,8 +1072,9 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                                             order=SCHEDULE_VJP)
     rvjp_src, rslots, _, _ = adj.vjp_kernels(
         "Ricci_eval", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n]) for n in ric_names], "",
-        "InteriorPoints,Enable_rfm_precompute", "rfm_struct *restrict rfmstruct,",
-        groups=[[ric_names.index(n) for n in grp] for grp in ric_groups], split_transpose=True, order=SCHEDULE_VJP)
+        "InteriorPoints,Enable_rfm_precompute", "rfm_struct *restrict rfmstruct,", split_transpose=True,
+        **({} if CoordSystem == "Cartesian" else {
+            "groups": [[ric_names.index(n) for n in grp] for grp in ric_groups], "order": SCHEDULE_VJP}))
     # det(gammabar) enforcement and the Hamiltonian constraint, for the adjoint of the BSSN RK4
     # step and of the H-L2 diagnostic; the mass derivatives of the initial data.
     dvjp_src, dslots, _, _ = adj.vjp_kernels("enforce_detgammabar_constraint", detg_exprs, "",
