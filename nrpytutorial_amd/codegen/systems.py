@@ -341,6 +341,48 @@ def _fused_launcher(name, args_sig, call_args, loopopts):
             % (name, args_sig, block, n[0], n[1], n[2], cases))
 
 
+def _merged_substep(kernels, args_decl, args_sig, call_args):
+    """One launch of several fused RHS + RK4 kernels that do not depend on each other (text of each,
+    in the order in which their blocks start: the longest first). Row blockIdx.y of the grid runs the
+    statements of kernel blockIdx.y."""
+    src, names, ids = "", [], []
+    for k in kernels:
+        m = re.search(r"template <int S>\n__global__ void __launch_bounds__\([^)]*\) (\w+)__gpu\(", k)
+        names.append(m.group(1))
+        ids.append(bd.lp.kernel_id(m.group(1)))
+        src += ("template <int S>\nstatic __device__ __forceinline__ void %s__body(" % m.group(1)
+                + k[m.end():])
+    shape = "%d, %d, %d" % (bd.lp.BLOCK_X, bd.lp.BLOCK_Y, bd.lp.BLOCK_Z)
+    src += ("template <int S>\n__global__ void __launch_bounds__(256) rhs_eval_rk4_substep_merged__gpu(%s, double *rk_yn, "
+            "double *rk_rt, double *rk_out, const double dt) {\n" % args_decl
+            + "".join("  %sif (blockIdx.y == %d) %s__body<S>(params, rfmstruct, auxevol_gfs, in_gfs, rk_yn, rk_rt, rk_out, "
+                      "dt);\n" % ("else " if k else "", k, n) for k, n in enumerate(names)) + "}\n")
+    src += r"""
+// The blocks of all the kernels are on the chip together, so a small grid's substep takes as long as the
+// longest of them, without the gaps between launches; a large one fills the last wave of one kernel with
+// blocks of the next. Spherical grids: 72x12x2 29.5 us as three launches, 13.1 as one; 128x64x2 22.0, 11.6;
+// 256x128x2 39.3, 38.5; 128x64x16 58.4, 55.6; 128x64x64 235.5, 226.9. It has one tile shape: kernels whose
+// shapes were set to different ones are launched one by one.
+static bool nrpy_substep_merged(dim3 *block) {
+""" + "".join("  const dim3 b%d = nrpy_block(%d, %s);\n" % (k, i, shape) for k, i in enumerate(ids)) + "".join(
+        "  if (b%d.x != b0.x || b%d.y != b0.y || b%d.z != b0.z) return false;\n" % (k, k, k)
+        for k in range(1, len(ids))) + r"""  *block = b0;
+  return true;
+}
+static int rhs_eval_rk4_substep_merged(const int S, const dim3 block, """ + args_sig + r""", double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
+  if (!params || !y_n || !rt || !out) return NRPY_ERR_NULL;
+  if (S < 0 || S > 3) return NRPY_ERR_PARAM;
+  if (nrpy_check_params(params)) return NRPY_ERR_SHAPE;
+  const dim3 grid(nrpy_nblocks(block, params->Nxx0, params->Nxx1, params->Nxx2), """ + str(len(ids)) + r""");
+  switch (S) {
+""" + "".join("    case %d: hipLaunchKernelGGL(rhs_eval_rk4_substep_merged__gpu<%d>, grid, block, 0, stream, %s, y_n, rt, "
+              "out, dt); break;\n" % (s, s, call_args) for s in range(4)) + r"""  }
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+"""
+    return src
+
+
 # the fused Sommerfeld step's interior substep in the Cartesian scalar-wave and Maxwell bundles
 SHELL_CALL = ("rhs_eval_rk4_substep_shell(SUBSTEP, params, IN, y_n_gfs, y_nplus1_running_total_gfs, OUT, R, dt, "
               "stream)")
@@ -919,7 +961,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                   "const REAL *restrict auxevol_gfs,const REAL *restrict in_gfs,REAL *restrict rhs_gfs")
     args_decl = ("const paramstruct params, const rfm_struct rfmstruct, const double *__restrict__ auxevol_gfs, "
                  "const double *__restrict__ in_gfs")
-    rhs_src, fused, group_costs, group_inputs = "", "", [], []
+    rhs_src, fused, fused_kernels, group_costs, group_inputs = "", "", [], [], []
     step_bodies = []
     # Large Cartesian grids: the RHS, Ricci and Hamiltonian kernels read their
     # mixed-derivative stencils from LDS tiles (codegen/lds.py). The small
@@ -956,6 +998,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                                    scheduled(body, grp, CoordSystem, fused=True),
                                    loopopts="InteriorPoints,Enable_rfm_precompute")
         group_inputs.append(len(kernel_inputs(kern)))
+        fused_kernels.append(kern)
         fused += kern
         fused += _fused_launcher("rhs_eval_rk4_substep_g%d" % k, "const rfm_struct *rfmstruct, "
                                  "const paramstruct *params, const double *auxevol_gfs, const double *in_gfs",
@@ -970,9 +1013,18 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
                 "  int rc;\n%s  return NRPY_OK;\n}\n" % (len(groups), calls))
     calls = "".join("  if ((rc = rhs_eval_rk4_substep_g%d(S, rfmstruct, params, auxevol_gfs, in_gfs, y_n, rt, out, "
                     "dt, stream))) return rc;\n" % k for k in range(len(groups)))
+    merged = ""
+    if CoordSystem != "Cartesian":                       # (the Cartesian kernels have tiles of their own in LDS)
+        order = sorted(range(len(groups)), key=lambda k: -group_costs[k]["flops"])
+        fused += _merged_substep([fused_kernels[k] for k in order], args_decl,
+                                 "const rfm_struct *rfmstruct, const paramstruct *params, const double *auxevol_gfs, "
+                                 "const double *in_gfs", "*params, *rfmstruct, auxevol_gfs, in_gfs")
+        merged = ("  dim3 block;\n  if (nrpy_substep_merged(&block))\n"
+                  "    return rhs_eval_rk4_substep_merged(S, block, rfmstruct, params, auxevol_gfs, in_gfs, y_n, rt, out, "
+                  "dt, stream);\n")
     fused += ('extern "C" int rhs_eval_rk4_substep(const int S, const rfm_struct *rfmstruct, const paramstruct *params, '
               "const double *auxevol_gfs, const double *in_gfs, double *y_n, double *rt, double *out, "
-              "const double dt, hipStream_t stream) {\n  int rc;\n%s  return NRPY_OK;\n}\n" % calls)
+              "const double dt, hipStream_t stream) {\n%s  int rc;\n%s  return NRPY_OK;\n}\n" % (merged, calls))
     t0 = time.time()
     ric_names = ["RbarDD%d%d" % (i, j) for i in range(3) for j in range(i, 3)]
     ric_exprs = {"RbarDD%d%d" % (i, j): RbarDD[i][j] for i in range(3) for j in range(i, 3)}
