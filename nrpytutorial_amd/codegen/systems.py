@@ -358,16 +358,20 @@ def _merged_substep(kernels, args_decl, args_sig, call_args):
             + "".join("  %sif (blockIdx.y == %d) %s__body<S>(params, rfmstruct, auxevol_gfs, in_gfs, rk_yn, rk_rt, rk_out, "
                       "dt);\n" % ("else " if k else "", k, n) for k, n in enumerate(names)) + "}\n")
     src += r"""
-// The blocks of all the kernels are on the chip together, so a small grid's substep takes as long as the
-// longest of them, without the gaps between launches; a large one fills the last wave of one kernel with
-// blocks of the next. Spherical grids: 72x12x2 29.5 us as three launches, 13.1 as one; 128x64x2 22.0, 11.6;
-// 256x128x2 39.3, 38.5; 128x64x16 58.4, 55.6; 128x64x64 235.5, 226.9. It has one tile shape: kernels whose
-// shapes were set to different ones are launched one by one.
-static bool nrpy_substep_merged(dim3 *block) {
+// On a small grid the blocks of all the kernels are on the chip together, so a substep takes as long as
+// the longest of them, without the gaps between launches; on one of a few waves of blocks, the last wave of
+// one kernel is filled with blocks of the next. On a large grid the launch runs at the registers of the
+// largest kernel, which the others need fewer of. Spherical grids, three launches and one: 72x12x2 (72
+// blocks) 29.5, 13.1 us; 128x64x2 22.0, 11.6; 256x128x2 39.3, 38.5; 128x64x16 58.4, 55.6; 128x64x64 (6144)
+// 235.5, 226.9; 192x128x64 (18432) 755, 793; 256x128x128 2012, 2142. The line is at 24 blocks per CU.
+// The launch has one tile shape: kernels whose shapes were set to different ones go one by one.
+#define NRPY_MERGED_BLOCKS (24 * 256)
+static bool nrpy_substep_merged(const paramstruct *params, dim3 *block) {
+  if (!params || nrpy_check_params(params)) return false;
 """ + "".join("  const dim3 b%d = nrpy_block(%d, %s);\n" % (k, i, shape) for k, i in enumerate(ids)) + "".join(
         "  if (b%d.x != b0.x || b%d.y != b0.y || b%d.z != b0.z) return false;\n" % (k, k, k)
         for k in range(1, len(ids))) + r"""  *block = b0;
-  return true;
+  return (size_t)nrpy_nblocks(b0, params->Nxx0, params->Nxx1, params->Nxx2) * """ + str(len(ids)) + r""" <= NRPY_MERGED_BLOCKS;
 }
 static int rhs_eval_rk4_substep_merged(const int S, const dim3 block, """ + args_sig + r""", double *y_n, double *rt, double *out, const double dt, hipStream_t stream) {
   if (!params || !y_n || !rt || !out) return NRPY_ERR_NULL;
@@ -1019,7 +1023,7 @@ def bssn(CoordSystem, symmetry_axes, bundle_name, FD_order=4):
         fused += _merged_substep([fused_kernels[k] for k in order], args_decl,
                                  "const rfm_struct *rfmstruct, const paramstruct *params, const double *auxevol_gfs, "
                                  "const double *in_gfs", "*params, *rfmstruct, auxevol_gfs, in_gfs")
-        merged = ("  dim3 block;\n  if (nrpy_substep_merged(&block))\n"
+        merged = ("  dim3 block;\n  if (nrpy_substep_merged(params, &block))\n"
                   "    return rhs_eval_rk4_substep_merged(S, block, rfmstruct, params, auxevol_gfs, in_gfs, y_n, rt, out, "
                   "dt, stream);\n")
     fused += ('extern "C" int rhs_eval_rk4_substep(const int S, const rfm_struct *rfmstruct, const paramstruct *params, '

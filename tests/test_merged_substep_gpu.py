@@ -1,6 +1,7 @@
 """rhs_eval_rk4_substep of the spherical BSSN bundle, one launch of its three kernels, against the
 kernels launched one by one on the GPU: the same statements per output, so equal bit for bit, for
-every substep, on grids of one partial tile, whole tiles and a remainder in each direction, and
+every substep, on grids of one partial tile, whole tiles, a remainder in each direction and more
+tiles than one launch takes, and
 with a tile shape set for one kernel only (then they are launched one by one)."""
 import ctypes
 
@@ -10,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape", [None, (16, 4, 4)])
-@pytest.mark.parametrize("Nxx", [(12, 8, 2), (64, 4, 4), (70, 6, 10)])
+@pytest.mark.parametrize("Nxx", [(12, 8, 2), (64, 4, 4), (70, 6, 10), (66, 128, 80)])
 def test_merged_equals_separate(torch_cuda, Nxx, shape):
     torch = torch_cuda
     from nrpytutorial_amd.runtime import Bundle, Evolution, Grid, check, ptr
