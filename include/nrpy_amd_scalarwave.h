@@ -86,8 +86,10 @@ int apply_bcs_sommerfeld_rk4(const int S, const paramstruct *params, double *xx[
                              double *out, const double dt, hipStream_t stream);
 
 
-/* The Sommerfeld step above captured into a hipGraph (no counterpart in the reference; pointers, xx
- * and dt fixed at capture), replayed nsteps times per MoL_graph_launch, freed with MoL_graph_free. */
+/* The Sommerfeld step above captured into a hipGraph (no counterpart in the reference; the pointers,
+ * those in xx among them, and dt are fixed at capture), replayed nsteps times per MoL_graph_launch,
+ * freed with MoL_graph_free. Creating it reads no device memory; a launch reads all of it, the
+ * coordinates too, in its stream's order. */
 int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3],
                                 const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs,
                                 double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out);

@@ -46,8 +46,10 @@ int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *params, const
                                                 hipStream_t stream);
 
 
-/* The Sommerfeld step above captured into a hipGraph (no counterpart in the reference; pointers, xx
- * and dt fixed at capture), replayed nsteps times per MoL_graph_launch, freed with MoL_graph_free.
+/* The Sommerfeld step above captured into a hipGraph (no counterpart in the reference; the pointers,
+ * those in xx among them, and dt are fixed at capture), replayed nsteps times per MoL_graph_launch,
+ * freed with MoL_graph_free. Creating it reads no device memory; a launch reads all of it, the
+ * coordinates too, in its stream's order.
  * The captured step takes two launches per substep instead of one per layer and face group, with
  * the same values. It allocates device memory that the graph owns until MoL_graph_free
  * (2 NUM_EVOL_GFS + 5 gridfunctions); without that memory it captures the step above. */

@@ -704,7 +704,9 @@ _SOMMERFELD_CHAIN = r'''
 // Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
 // launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
 // chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table
-// (geo, 5 values per point, written once per captured step) instead of the Jacobian.
+// (geo, 5 values per point) instead of the Jacobian. MoL_graph_launch fills the table before its
+// replays, on their stream, so that the coordinates are read when and where the step reads its
+// other arrays (one launch of about 5 us per call, not per step).
 // Scratch of a captured step: R, NUM_EVOL_GFS gridfunctions: the RHS at the interior points a
 // chain or copy ends at (rhs_eval_rk4_substep_rim), A at the outer points; then B, as many; then geo.
 #define NRPY_SOM_NSCRATCH (2 * NUM_EVOL_GFS + 5)
@@ -873,11 +875,19 @@ static bool nrpy_sommerfeld_chainable(const bc_struct *bc) {
   return true;
 }
 
-// Device memory of a captured step on the grid, its geometry table filled before this returns.
-// nullptr where the two launches do not cover the grid, or without memory: the caller takes
-// the unfused step.
-static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc,
-                                             hipStream_t stream) {
+// The geometry table in the scratch of a captured step.
+static int nrpy_sommerfeld_geometry_fill(const paramstruct *params, const double *const xx[3], double *scratch,
+                                         hipStream_t stream) {
+  const size_t Ntot =
+      (size_t)params->Nxx_plus_2NGHOSTS0 * params->Nxx_plus_2NGHOSTS1 * params->Nxx_plus_2NGHOSTS2;
+  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
+                     xx[0], xx[1], xx[2], scratch + 2 * NUM_EVOL_GFS * Ntot);
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+
+// Device memory of a captured step on the grid, nothing in it yet. nullptr where the two launches do
+// not cover the grid, or without memory: the caller takes the unfused step.
+static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc) {
   if (!params || !bc || !xx || !xx[0] || !xx[1] || !xx[2] || nrpy_check_params(params)) return nullptr;
   if (bc->N[0] != params->Nxx_plus_2NGHOSTS0 || bc->N[1] != params->Nxx_plus_2NGHOSTS1 ||
       bc->N[2] != params->Nxx_plus_2NGHOSTS2 || bc->N[0] < NRPY_SOMMERFELD_MIN_N || bc->N[1] < NRPY_SOMMERFELD_MIN_N ||
@@ -887,12 +897,6 @@ static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *
   double *p = nullptr;
   if (hipMalloc((void **)&p, sizeof(double) * NRPY_SOM_NSCRATCH * Ntot) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
-  }
-  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
-                     xx[0], xx[1], xx[2], p + 2 * NUM_EVOL_GFS * Ntot);
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
-    (void)hipFree(p);
     return nullptr;
   }
   return p;

@@ -50,8 +50,10 @@ BUNDLES = ("scalarwave_cartesian", "bssn_cartesian", "bssn_spherical_sym2", "max
     tuple(CURVI_SCALARWAVE) + ("bssn_etk",) + tuple(CURVI_MAXWELL)
 
 
-def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage="", edge=False):
-    """MoL_step_forward_in_time + hipGraph replay for the diagonal RK4 schedule."""
+def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage="", edge=False, geometry=False):
+    """MoL_step_forward_in_time + hipGraph replay for the diagonal RK4 schedule. geometry: the
+    bundle's captured Sommerfeld step reads a table of the grid's geometry (_sommerfeld_glue's
+    ``rim``), which a launch fills before its replays."""
     ricci = ("  if ((rc = Ricci_eval(rfmstruct, params, IN, auxevol_gfs, stream))) return rc;\n" if has_ricci else "")
     detg = ("  if ((rc = DETG(rfmstruct, params, OUT, stream))) return rc;\n"
             if has_detg else "")
@@ -88,7 +90,11 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage="", 
          "  if ((rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, y_n_gfs, &gfp))) return rc;\n"
          if edge else "") + steps + "  return NRPY_OK;\n}\n\n"
         "struct MoL_graph {\n  hipGraph_t graph;\n  hipGraphExec_t exec;\n"
-        "  double *scratch = nullptr;  // device memory of the captured step, owned by the graph\n};\n"
+        + ("  double *scratch = nullptr;  // device memory of the captured Sommerfeld step, owned by the graph\n"
+           "  paramstruct params;         // what its geometry table is computed from at each launch\n"
+           "  const double *xx[3];\n};\n"
+           "static int nrpy_sommerfeld_geometry_fill(const paramstruct *params, const double *const xx[3], double *scratch, "
+           "hipStream_t stream);\n" if geometry else "};\n") +
         "// Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed\n"
         "// at capture time.\n"
         'extern "C" int MoL_graph_create(' + sig + ", MoL_graph **out) {\n"
@@ -114,12 +120,17 @@ def _mol_glue(has_ricci, has_detg, rhs_args_decl, rhs_call_args, detg_stage="", 
         "  *out = g;\n  return NRPY_OK;\n}\n"
         'extern "C" int MoL_graph_launch(MoL_graph *g, const int nsteps, hipStream_t stream) {\n'
         "  if (!g) return NRPY_ERR_NULL;\n  if (nsteps < 0) return NRPY_ERR_PARAM;\n"
+        + ("  // in the stream's order, as the replays themselves: the coordinates are those of this launch\n"
+           "  if (g->scratch && nsteps > 0) {\n"
+           "    const int rc = nrpy_sommerfeld_geometry_fill(&g->params, g->xx, g->scratch, stream);\n"
+           "    if (rc) return rc;\n"
+           "  }\n" if geometry else "") +
         "  for (int n = 0; n < nsteps; n++)\n"
         "    if (hipGraphLaunch(g->exec, stream) != hipSuccess) return NRPY_ERR_LAUNCH;\n"
         "  return NRPY_OK;\n}\n"
         'extern "C" void MoL_graph_free(MoL_graph *g) {\n'
         "  if (!g) return;\n  (void)hipGraphExecDestroy(g->exec);\n  (void)hipGraphDestroy(g->graph);\n"
-        "  (void)hipFree(g->scratch);\n  delete g;\n}\n")
+        + ("  (void)hipFree(g->scratch);\n" if geometry else "") + "  delete g;\n}\n")
 
 
 def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
@@ -190,8 +201,8 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
             "radial_falloff_power": list(bcs.vars_radial_falloff_power.values()),
             "speed": list(bcs.vars_speed.values())}
     graph = (
-        "// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; pointers, xx\n"
-        "// and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.\n"
+        "// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; the pointers, those of\n"
+        "// xx among them, and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.\n"
         'extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, '
         "double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, "
         "double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out) {\n"
@@ -207,7 +218,11 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
         "  int rc = NRPY_OK;\n" +
         ("  // without scratch memory, or on a grid the chain kernel does not cover: the unfused step\n"
          "  if (rfmstruct && y_n_gfs && k_odd_gfs && k_even_gfs && y_nplus1_running_total_gfs)\n"
-         "    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct, s);\n" if rim is not None else "") +
+         "    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct);\n"
+         "  if (g->scratch) {\n"
+         "    g->params = *params;\n"
+         "    for (int d = 0; d < 3; d++) g->xx[d] = xx[d];\n"
+         "  }\n" if rim is not None else "") +
         "  if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = NRPY_ERR_LAUNCH;\n"
         "  if (!rc) {\n"
         + ("    rc = g->scratch ? nrpy_sommerfeld_chain_step(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,\n"
@@ -226,10 +241,10 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
         "    }\n"
         "  }\n"
         "  (void)hipStreamDestroy(s);\n"
-        "  if (rc) { (void)hipFree(g->scratch); delete g; return rc; }\n"
+        "  if (rc) { " + ("(void)hipFree(g->scratch); " if rim is not None else "") + "delete g; return rc; }\n"
         "  *out = g;\n  return NRPY_OK;\n}\n")
-    return ("// One RK4 step with the Sommerfeld radiation condition on the RHS.\n" + bcs.hip_source(chain=rim is not None) + (rim or "") + step + graph,
-            meta)
+    return ("// One RK4 step with the Sommerfeld radiation condition on the RHS.\n" +
+            bcs.hip_source(chain=rim is not None) + (rim or "") + step + graph, meta)
 
 
 def _mol_batch_glue(n_rhs, detg_stage):
@@ -810,7 +825,7 @@ def scalarwave_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
                                          rim=rim)
     pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code,
-             rhs_src, fused, id_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]
+             rhs_src, fused, id_src, _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", geometry=True), som_src]
     meta["sommerfeld"] = som_meta
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta["kernel_ids"] = dict(bd.lp.KERNEL_IDS)
@@ -880,7 +895,7 @@ def maxwell_curvilinear(CoordSystem, bundle_name, NGHOSTS=3):
                                          rim=rim)
     pre, meta = _header(NGHOSTS, stage_offsets([body]))
     parts = [pre, coords, '#include "../nrpy_runtime.h"', rfm_code, rhs_src, con_src, fused, id_src,
-             _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN"), som_src]
+             _mol_glue(False, False, None, "rfmstruct, params, auxevol_gfs, IN", geometry=True), som_src]
     meta["sommerfeld"] = som_meta
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta["kernel_ids"] = dict(bd.lp.KERNEL_IDS)

@@ -950,8 +950,11 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
 struct MoL_graph {
   hipGraph_t graph;
   hipGraphExec_t exec;
-  double *scratch = nullptr;  // device memory of the captured step, owned by the graph
+  double *scratch = nullptr;  // device memory of the captured Sommerfeld step, owned by the graph
+  paramstruct params;         // what its geometry table is computed from at each launch
+  const double *xx[3];
 };
+static int nrpy_sommerfeld_geometry_fill(const paramstruct *params, const double *const xx[3], double *scratch, hipStream_t stream);
 // Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed
 // at capture time.
 extern "C" int MoL_graph_create(const rfm_struct *rfmstruct, const paramstruct *params, const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, double *auxevol_gfs, const double dt, MoL_graph **out) {
@@ -981,6 +984,11 @@ extern "C" int MoL_graph_create(const rfm_struct *rfmstruct, const paramstruct *
 extern "C" int MoL_graph_launch(MoL_graph *g, const int nsteps, hipStream_t stream) {
   if (!g) return NRPY_ERR_NULL;
   if (nsteps < 0) return NRPY_ERR_PARAM;
+  // in the stream's order, as the replays themselves: the coordinates are those of this launch
+  if (g->scratch && nsteps > 0) {
+    const int rc = nrpy_sommerfeld_geometry_fill(&g->params, g->xx, g->scratch, stream);
+    if (rc) return rc;
+  }
   for (int n = 0; n < nsteps; n++)
     if (hipGraphLaunch(g->exec, stream) != hipSuccess) return NRPY_ERR_LAUNCH;
   return NRPY_OK;
@@ -1507,7 +1515,9 @@ extern "C" int apply_bcs_sommerfeld(const paramstruct *params, double *xx[3], co
 // Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
 // launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
 // chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table
-// (geo, 5 values per point, written once per captured step) instead of the Jacobian.
+// (geo, 5 values per point) instead of the Jacobian. MoL_graph_launch fills the table before its
+// replays, on their stream, so that the coordinates are read when and where the step reads its
+// other arrays (one launch of about 5 us per call, not per step).
 // Scratch of a captured step: R, NUM_EVOL_GFS gridfunctions: the RHS at the interior points a
 // chain or copy ends at (rhs_eval_rk4_substep_rim), A at the outer points; then B, as many; then geo.
 #define NRPY_SOM_NSCRATCH (2 * NUM_EVOL_GFS + 5)
@@ -1676,11 +1686,19 @@ static bool nrpy_sommerfeld_chainable(const bc_struct *bc) {
   return true;
 }
 
-// Device memory of a captured step on the grid, its geometry table filled before this returns.
-// nullptr where the two launches do not cover the grid, or without memory: the caller takes
-// the unfused step.
-static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc,
-                                             hipStream_t stream) {
+// The geometry table in the scratch of a captured step.
+static int nrpy_sommerfeld_geometry_fill(const paramstruct *params, const double *const xx[3], double *scratch,
+                                         hipStream_t stream) {
+  const size_t Ntot =
+      (size_t)params->Nxx_plus_2NGHOSTS0 * params->Nxx_plus_2NGHOSTS1 * params->Nxx_plus_2NGHOSTS2;
+  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
+                     xx[0], xx[1], xx[2], scratch + 2 * NUM_EVOL_GFS * Ntot);
+  return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+
+// Device memory of a captured step on the grid, nothing in it yet. nullptr where the two launches do
+// not cover the grid, or without memory: the caller takes the unfused step.
+static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *xx[3], const bc_struct *bc) {
   if (!params || !bc || !xx || !xx[0] || !xx[1] || !xx[2] || nrpy_check_params(params)) return nullptr;
   if (bc->N[0] != params->Nxx_plus_2NGHOSTS0 || bc->N[1] != params->Nxx_plus_2NGHOSTS1 ||
       bc->N[2] != params->Nxx_plus_2NGHOSTS2 || bc->N[0] < NRPY_SOMMERFELD_MIN_N || bc->N[1] < NRPY_SOMMERFELD_MIN_N ||
@@ -1690,12 +1708,6 @@ static double *nrpy_sommerfeld_chain_scratch(const paramstruct *params, double *
   double *p = nullptr;
   if (hipMalloc((void **)&p, sizeof(double) * NRPY_SOM_NSCRATCH * Ntot) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
-  }
-  hipLaunchKernelGGL(nrpy_sommerfeld_geometry_kernel, dim3((unsigned)((Ntot + 255) / 256)), dim3(256), 0, stream, *params,
-                     xx[0], xx[1], xx[2], p + 2 * NUM_EVOL_GFS * Ntot);
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
-    (void)hipFree(p);
     return nullptr;
   }
   return p;
@@ -1991,8 +2003,8 @@ static int nrpy_sommerfeld_chain_step(const paramstruct *params, const rfm_struc
   if ((rc = nrpy_sommerfeld_chain(3, params, bcstruct, evol_gf_parity, R, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
   return NRPY_OK;
 }
-// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; pointers, xx
-// and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.
+// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; the pointers, those of
+// xx among them, and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.
 extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out) {
   if (!out) return NRPY_ERR_NULL;
   *out = nullptr;
@@ -2002,7 +2014,11 @@ extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_
   int rc = NRPY_OK;
   // without scratch memory, or on a grid the chain kernel does not cover: the unfused step
   if (rfmstruct && y_n_gfs && k_odd_gfs && k_even_gfs && y_nplus1_running_total_gfs)
-    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct, s);
+    g->scratch = nrpy_sommerfeld_chain_scratch(params, xx, bcstruct);
+  if (g->scratch) {
+    g->params = *params;
+    for (int d = 0; d < 3; d++) g->xx[d] = xx[d];
+  }
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = NRPY_ERR_LAUNCH;
   if (!rc) {
     rc = g->scratch ? nrpy_sommerfeld_chain_step(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs,

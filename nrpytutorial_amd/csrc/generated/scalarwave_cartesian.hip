@@ -650,7 +650,6 @@ extern "C" int MoL_step_forward_in_time(const rfm_struct *rfmstruct, const param
 struct MoL_graph {
   hipGraph_t graph;
   hipGraphExec_t exec;
-  double *scratch = nullptr;  // device memory of the captured step, owned by the graph
 };
 // Capture one RK4 step into a hipGraph; replay with MoL_graph_launch. Pointers and dt are fixed
 // at capture time.
@@ -689,7 +688,6 @@ extern "C" void MoL_graph_free(MoL_graph *g) {
   if (!g) return;
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
-  (void)hipFree(g->scratch);
   delete g;
 }
 
@@ -1296,8 +1294,8 @@ extern "C" int MoL_step_forward_in_time_sommerfeld(const paramstruct *params, co
   if ((rc = apply_bcs_sommerfeld_rk4(3, params, xx, bcstruct, NUM_EVOL_GFS, k_odd_gfs, R, y_n_gfs, y_nplus1_running_total_gfs, y_n_gfs, dt, stream))) return rc;
   return NRPY_OK;
 }
-// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; pointers, xx
-// and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.
+// The Sommerfeld RK4 step captured into a hipGraph (every launch is a kernel; the pointers, those of
+// xx among them, and dt are fixed at capture); replay with MoL_graph_launch, free with MoL_graph_free.
 extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, MoL_graph **out) {
   if (!out) return NRPY_ERR_NULL;
   *out = nullptr;
@@ -1323,7 +1321,7 @@ extern "C" int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_
     }
   }
   (void)hipStreamDestroy(s);
-  if (rc) { (void)hipFree(g->scratch); delete g; return rc; }
+  if (rc) { delete g; return rc; }
   *out = g;
   return NRPY_OK;
 }

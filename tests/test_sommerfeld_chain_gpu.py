@@ -40,3 +40,40 @@ def test_captured_step_equals_unfused(torch_cuda, bundle, pars, Nxx):
                 assert off < 1e-13, "step %d: %.2e" % (step, off)
     ev.free_graph()
     other.free_graph()
+
+
+@pytest.mark.parametrize("bundle,pars", CURVILINEAR, ids=[c[0] for c in CURVILINEAR])
+def test_captured_step_reads_xx_at_launch(torch_cuda, bundle, pars):
+    """The coordinates that enter a replay are those in xx when the launch's stream comes to it: not
+    those of the graph's creation (NaN here), nor of an earlier launch (stretched in between), and
+    with the writes still queued on the launch's stream."""
+    torch = torch_cuda
+    from nrpytutorial_amd.runtime import Evolution
+    Nxx = (9, 4, 10)
+    print("case: %s captured Sommerfeld step, xx changed between launches" % bundle, flush=True)
+    b, g, ev, og, y = _setup(torch, bundle, pars, Nxx)
+    first = torch.from_numpy(y).cuda()
+    ref = Evolution(g)
+    for e in (ev, ref):
+        e.y_n.copy_(first)
+    dt = 0.25 * g.find_timestep(0.5)
+    saved = [x.clone() for x in g.xx_dev]
+    for x in g.xx_dev:
+        x.fill_(float("nan"))
+    ev.step_sommerfeld(dt, 0)                   # creates the graph
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    for scale in (1.0, 1.01):
+        with torch.cuda.stream(stream):
+            queue = torch.ones(1 << 24, device="cuda")
+            for _ in range(20):                 # work in front of the writes
+                queue.mul_(1.0001)
+            for x, s in zip(g.xx_dev, saved):
+                x.copy_(s * scale)
+            ev.step_sommerfeld(dt, 2)
+            ref.step_sommerfeld(dt, 2, unfused=True)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(ref.y_n).all())
+        off = float((ev.y_n - ref.y_n).abs().max() / ref.y_n.abs().max())
+        assert off < 1e-13, "scale %g: %.2e" % (scale, off)
+    ev.free_graph()
