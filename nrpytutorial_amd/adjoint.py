@@ -240,9 +240,13 @@ class BSSNStepAdjoint:
 
     def step_back(self, y_n, lam, dt):
         """lam (cotangent of y_{n+1}, full array) <- cotangent of y_n (full array)."""
-        ev, L = self.ev, self.lib
+        ev, L, torch = self.ev, self.lib, self.ev.g.torch
+        if torch.is_grad_enabled() and lam.requires_grad:
+            raise RuntimeError("step_back: lam requires grad and would be changed in place")
         given = lam
-        if not self._usable(lam):
+        if self._usable(lam):
+            lam[:0].zero_()                          # autograd's record of the write that the kernels do
+        else:
             lam = self.P[0].copy_(lam)
         if not self._usable(y_n) or y_n.untyped_storage().data_ptr() == lam.untyped_storage().data_ptr():
             y_n = ev.g.empty(self.n).copy_(y_n)

@@ -42,3 +42,41 @@ def test_step_back_takes_any_tensor(torch_cuda):
     other = y.clone()
     adj.step_back(y, other, dt)
     assert bool(torch.equal(same, other))
+
+
+def test_step_back_is_seen_by_autograd(torch_cuda):
+    """The kernels write lam through its pointer; for autograd that is an in-place operation like any
+    other: refused on a cotangent that requires grad, and found by a graph that saved it before."""
+    torch = torch_cuda
+    from nrpytutorial_amd.adjoint import BSSNStepAdjoint
+    from nrpytutorial_amd.runtime import Bundle, Evolution, Grid
+    from nrpytutorial_amd.workloads import bssn_gaussian_state_torch
+    print("case: step_back and autograd", flush=True)
+    b = Bundle("bssn_cartesian")
+    g = Grid(b, (9, 6, 5))
+    ev = Evolution(g)
+    bssn_gaussian_state_torch(ev.y_n, g.xx_dev, b.evol, 3)
+    ev.apply_bcs(ev.y_n, composed=True)
+    ev.post_bcs(ev.y_n)
+    dt = g.find_timestep(0.5)
+    adj = BSSNStepAdjoint(ev)
+    start = torch.zeros_like(ev.y_n)
+    g.interior(start).fill_(0.25)
+    want = start.clone()
+    adj.step_back(ev.y_n, want, dt)
+    for leaf in (start.clone().requires_grad_(), start.permute(0, 3, 2, 1).contiguous().permute(0, 3, 2, 1).requires_grad_()):
+        before = leaf.detach().clone()
+        with pytest.raises(RuntimeError):
+            adj.step_back(ev.y_n, leaf, dt)
+        assert bool(torch.equal(leaf.detach(), before))
+        with torch.no_grad():
+            adj.step_back(ev.y_n, leaf, dt)
+        assert bool(torch.equal(leaf.detach(), want))
+    lam = start.clone()
+    x = torch.ones_like(lam).requires_grad_()
+    out = (x * lam).sum()                               # saves lam
+    version = lam._version
+    adj.step_back(ev.y_n, lam, dt)
+    assert lam._version > version and bool(torch.equal(lam, want))
+    with pytest.raises(RuntimeError):
+        out.backward()
