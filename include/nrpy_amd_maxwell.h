@@ -31,7 +31,8 @@ int rhs_eval_vjp(const paramstruct *params, const double *auxevol_gfs, const dou
 
 /* Adjoint of one RK4 step (MoL_step_forward_in_time): lambda_gfs holds the cotangent of
  * y_{n+1} on entry and that of y_n on exit; y_n_gfs is the state at the start of the step.
- * U1..U3, rt, acc, kbar, w: scratch states; vjp_G as for rhs_eval_vjp. */
+ * acc, kbar, w: three scratch states. The right-hand side is linear, so the state is not read, and
+ * U1..U3, rt and vjp_G are neither read nor written (not NULL). */
 int MoL_step_adjoint(const rfm_struct *rfmstruct, const paramstruct *params, const bc_struct *bcstruct,
                      const double *y_n_gfs, double *lambda_gfs, double *U1, double *U2, double *U3, double *rt,
                      double *acc, double *kbar, double *w, double *vjp_G, double *auxevol_gfs, const double dt,

@@ -307,8 +307,8 @@ def _mol_adjoint_glue(stage_kernel):
     if stage_kernel is None:
         raise ValueError("MoL_step_adjoint: the right-hand side is not linear with constant coefficients")
     stages = ((3, "lambda_gfs", "lambda_gfs", "acc", "kbar", "dt / 6.0, dt / 3.0, dt"),
-              (2, "kbar", "acc", "acc", "U1", "1.0, dt / 3.0, dt / 2.0"),
-              (1, "U1", "acc", "acc", "kbar", "1.0, dt / 6.0, dt / 2.0"),
+              (2, "kbar", "acc", "acc", "w", "1.0, dt / 3.0, dt / 2.0"),
+              (1, "w", "acc", "acc", "kbar", "1.0, dt / 6.0, dt / 2.0"),
               (0, "kbar", "acc", "lambda_gfs", "nullptr", "1.0, 0.0, 0.0"))
     return (
         stage_kernel +
@@ -316,7 +316,7 @@ def _mol_adjoint_glue(stage_kernel):
         "// ghost cotangents zero), y_n_gfs the state at the start of the step with its ghosts filled. On\n"
         "// exit lambda_gfs holds the cotangent of y_n. U1, U2, U3, rt, acc, kbar, w are caller-allocated\n"
         "// scratch arrays of NUM_EVOL_GFS gridfunctions; vjp_G has the rhs_eval_vjp slot count. (The\n"
-        "// right-hand side is linear: of them only U1, acc and kbar are used, and y_n_gfs is not read.)\n"
+        "// right-hand side is linear: of them only acc, kbar and w are used, and y_n_gfs is not read.)\n"
         'extern "C" int MoL_step_adjoint(const rfm_struct *rfmstruct, const paramstruct *params,\n'
         "    const bc_struct *bcstruct, const double *y_n_gfs, double *lambda_gfs, double *U1, double *U2,\n"
         "    double *U3, double *rt, double *acc, double *kbar, double *w, double *vjp_G, double *auxevol_gfs,\n"

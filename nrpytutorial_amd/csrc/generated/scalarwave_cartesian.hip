@@ -786,7 +786,7 @@ static int rhs_eval_vjp_rk4_stage(const int S, const paramstruct *params, const 
 // ghost cotangents zero), y_n_gfs the state at the start of the step with its ghosts filled. On
 // exit lambda_gfs holds the cotangent of y_n. U1, U2, U3, rt, acc, kbar, w are caller-allocated
 // scratch arrays of NUM_EVOL_GFS gridfunctions; vjp_G has the rhs_eval_vjp slot count. (The
-// right-hand side is linear: of them only U1, acc and kbar are used, and y_n_gfs is not read.)
+// right-hand side is linear: of them only acc, kbar and w are used, and y_n_gfs is not read.)
 extern "C" int MoL_step_adjoint(const rfm_struct *rfmstruct, const paramstruct *params,
     const bc_struct *bcstruct, const double *y_n_gfs, double *lambda_gfs, double *U1, double *U2,
     double *U3, double *rt, double *acc, double *kbar, double *w, double *vjp_G, double *auxevol_gfs,
@@ -799,8 +799,8 @@ extern "C" int MoL_step_adjoint(const rfm_struct *rfmstruct, const paramstruct *
   int rc = nrpy_bc_check(params, bcstruct, NUM_EVOL_GFS, evol_gf_parity, lambda_gfs, &gfp);
   if (rc) return rc;
   if ((rc = rhs_eval_vjp_rk4_stage(3, params, lambda_gfs, lambda_gfs, lambda_gfs, acc, kbar, dt / 6.0, dt / 3.0, dt, stream))) return rc;
-  if ((rc = rhs_eval_vjp_rk4_stage(2, params, kbar, lambda_gfs, acc, acc, U1, 1.0, dt / 3.0, dt / 2.0, stream))) return rc;
-  if ((rc = rhs_eval_vjp_rk4_stage(1, params, U1, lambda_gfs, acc, acc, kbar, 1.0, dt / 6.0, dt / 2.0, stream))) return rc;
+  if ((rc = rhs_eval_vjp_rk4_stage(2, params, kbar, lambda_gfs, acc, acc, w, 1.0, dt / 3.0, dt / 2.0, stream))) return rc;
+  if ((rc = rhs_eval_vjp_rk4_stage(1, params, w, lambda_gfs, acc, acc, kbar, 1.0, dt / 6.0, dt / 2.0, stream))) return rc;
   if ((rc = rhs_eval_vjp_rk4_stage(0, params, kbar, lambda_gfs, acc, lambda_gfs, nullptr, 1.0, 0.0, 0.0, stream))) return rc;
   return NRPY_OK;
 }
