@@ -214,7 +214,7 @@ def entry_point(name, desc, args, fills, kernels, interior=True):
 def bssn_etk(bundle_name="bssn_etk"):
     from ..BSSN import BSSN_quantities as Bq, BSSN_RHSs as rhs, BSSN_gauge_RHSs as gaugerhs
     from ..BSSN import Enforce_Detgammabar_Constraint as EGC, BSSN_constraints as bssncon
-    from .systems import rhs_groups, ricci_groups, lds_tile_for_group, scheduled, MIN_TWO_WAVES_OUTPUTS
+    from .systems import rhs_groups, lds_tile_for_group, scheduled, MIN_TWO_WAVES_OUTPUTS
     t0 = time.time()
     par.set_parval_from_str("grid::DIM", 3)
     par.set_parval_from_str("finite_difference::FD_CENTDERIVS_ORDER", FD_ORDER)
@@ -261,27 +261,20 @@ def bssn_etk(bundle_name="bssn_etk"):
     # Ricci tensor (BaikalETK_C_kernels_codegen.py:306-330)
     ric_names = ["RbarDD%d%d" % (i, j) for i in range(3) for j in range(i, 3)]
     ric_exprs = {"RbarDD%d%d" % (i, j): RbarDD[i][j] for i in range(3) for j in range(i, 3)}
-    # one kernel of all components; the groups' kernels are the SENR-layout bundle's counterparts
-    kernels, flops = [], 0
-    lp.MIN_WAVES_PER_EU["Baikal_BSSN_Ricci"] = 2
-    for k, grp in enumerate(ricci_groups(ric_names) + [ric_names]):
-        body = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
-                                               for n in grp], params="outCverbose=False")
-        name = "Baikal_BSSN_Ricci" + ("_g%d" % k if grp is not ric_names else "")
-        if grp is ric_names:
-            flops = bd.count_body(body)["flops"]
-        text, launch = etk_kernel(name, "Ricci tensor components %s" % ", ".join(grp),
-                                  scheduled(body, grp, "Cartesian"), table)
-        src.append(text)
-        if grp is ric_names:
-            kernels.append((name, launch))
+    name = "Baikal_BSSN_Ricci"
+    lp.MIN_WAVES_PER_EU[name] = 2
+    body = fin.FD_outputC("returnstring", [lhrh(lhs=gri.gfaccess("auxevol_gfs", n), rhs=ric_exprs[n])
+                                           for n in ric_names], params="outCverbose=False")
+    text, launch = etk_kernel(name, "Ricci tensor components %s" % ", ".join(ric_names),
+                              scheduled(body, ric_names, "Cartesian"), table)
+    src.append(text)
     fname = "Baikal_BSSN_Ricci_FD_order_%d" % FD_ORDER
     c, p = entry_point(fname, "Ricci tensor RbarDD at interior points (BaikalETK_BSSN_Ricci_FD_order_4)",
                        ["const double *const *evol_gfs", "double *const *auxevol_gfs"],
-                       [evol_fill, ("auxevol_gfs", 2 * NE, NAE)], kernels)
+                       [evol_fill, ("auxevol_gfs", 2 * NE, NAE)], [(name, launch)])
     src.append(c)
     protos.append(p)
-    costs[fname] = flops
+    costs[fname] = bd.count_body(body)["flops"]
     print("(BENCH) Ricci codegen %.1fs" % (time.time() - t0), flush=True)
 
     # BSSN right-hand sides (BaikalETK_C_kernels_codegen.py:264-304)

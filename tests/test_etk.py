@@ -100,7 +100,7 @@ def _statements(kernel, bounds):
     return [l.strip() for l in body.splitlines() if l.strip()]
 
 
-PAIRS = [("Baikal_BSSN_Ricci_g0", "Ricci_eval_g0"), ("Baikal_BSSN_Ricci_g1", "Ricci_eval_g1"),
+PAIRS = [("Baikal_BSSN_Ricci", "Ricci_eval"),
          ("Baikal_BSSN_RHSs_g0", "rhs_eval_g0"), ("Baikal_BSSN_RHSs_g1", "rhs_eval_g1"),
          ("Baikal_BSSN_RHSs_g2", "rhs_eval_g2"),
          ("Baikal_BSSN_constraints_H", "Hamiltonian_constraint"),
@@ -129,6 +129,14 @@ def test_plugin_kernels_equal_senr_kernels(etk_name, senr_name):
     lds_e = [x.upper() for x in re.findall(r"copy the .*? of ([\w, ]+) to LDS", ke)]
     lds_s = [x.upper() for x in re.findall(r"copy the .*? of ([\w, ]+) to LDS", ks)]
     assert lds_e == lds_s
+
+
+def test_pairs_are_the_kernels_that_are_launched():
+    """Every kernel of the plugin is launched by an entry point, and compared above."""
+    etk = open(os.path.join(GEN, "bssn_etk.hip")).read()
+    kernels = re.findall(r"__global__ void __launch_bounds__\([^)]*\) (Baikal_\w+)__gpu\(", etk)
+    launched = re.findall(r"hipLaunchKernelGGL\((Baikal_\w+)__gpu,", etk)
+    assert sorted(kernels) == sorted(set(launched)) == sorted(p[0] for p in PAIRS)
 
 
 def test_constraint_kernels_cover_h_and_mu():
