@@ -77,6 +77,7 @@ struct nrpy_fill_term {
 // Rows sorted by the number of extrapolated axes (0 or 1, then 2, 3, then generic ones).
 struct nrpy_fill_list {
   int n = 0;
+  bool near_edges = true;  // no generic row, and every base is within NGHOSTS points of the interior's edge
   std::vector<nrpy_fill_row> h_rows;
   std::vector<nrpy_fill_term> h_terms;
   nrpy_fill_row *d_rows = nullptr;
@@ -113,6 +114,9 @@ struct bc_struct {
   int *d_ob_xedge_dest = nullptr;
   int8_t *d_ob_xedge_face = nullptr;
   int ob_xedge_off[NGHOSTS + 1];
+  // every outer point's FACE is along the axis on which it lies farthest outside the interior (the
+  // last of equals), known when the maps are built
+  bool face_by_distance = true;
   // composed ghost map (CSR over ghost points); negmask bit t set: parity type t contributes
   // with a minus sign
   int nghost = 0, nterms = 0;
@@ -323,7 +327,7 @@ static void nrpy_build_fill(const paramstruct *params, const bc_struct *bc, cons
     const int b = bc->h_rowptr[r], n = bc->h_rowptr[r + 1] - b;
     const int i[3] = {anchor[r] % N0, (anchor[r] / N0) % N1, anchor[r] / (N0 * N1)};
     int base = 0, code = 0, axes = 0, layer[3], s[3];
-    bool product = n > 0;
+    bool product = n > 0, near_edge = false;
     for (int d = 0; d < 3; d++) {
       layer[d] = 0;
       s[d] = stride[d];
@@ -340,6 +344,7 @@ static void nrpy_build_fill(const paramstruct *params, const bc_struct *bc, cons
       }
       axes += layer[d] > 0;
       product = product && layer[d] <= 3;
+      near_edge = near_edge || at < 2 * NGHOSTS || at >= N[d] - 2 * NGHOSTS;
       base += at * stride[d];
     }
     product = product && n == (axes == 0 ? 1 : axes == 1 ? 3 : axes == 2 ? 9 : 27);
@@ -358,6 +363,7 @@ static void nrpy_build_fill(const paramstruct *params, const bc_struct *bc, cons
         found = found || (bc->h_src[q] == src && bc->h_coeff[q] == w && bc->h_negmask[q] == neg);
       product = found;
     }
+    L->near_edges = L->near_edges && product && near_edge;
     if (product) {
       kind[axes < 1 ? 0 : axes - 1].push_back({bc->h_gdest[r], base, code, neg});
     } else {
@@ -367,6 +373,23 @@ static void nrpy_build_fill(const paramstruct *params, const bc_struct *bc, cons
   }
   for (const auto &rows : kind) L->h_rows.insert(L->h_rows.end(), rows.begin(), rows.end());
   L->n = (int)L->h_rows.size();
+}
+
+static bool nrpy_face_by_distance(const int *N, const outer_bc &o) {
+  const int i[3] = {o.outer_bc_dest_pt.i0, o.outer_bc_dest_pt.i1, o.outer_bc_dest_pt.i2};
+  const int F[3] = {o.FACEi0, o.FACEi1, o.FACEi2};
+  int far = 0, axis = -1, sign = 0;
+  for (int d = 0; d < 3; d++) {
+    const int m = i[d] < NGHOSTS ? NGHOSTS - i[d] : i[d] >= N[d] - NGHOSTS ? i[d] - (N[d] - NGHOSTS - 1) : 0;
+    if (m > 0 && m >= far) {
+      far = m;
+      axis = d;
+      sign = i[d] < NGHOSTS ? 1 : -1;
+    }
+  }
+  for (int d = 0; d < 3; d++)
+    if (F[d] != (d == axis ? sign : 0)) return false;
+  return true;
 }
 
 static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
@@ -426,6 +449,7 @@ static int nrpy_build_composed_map(const paramstruct *params, bc_struct *bc) {
       if (!expand(dest + stride, 3.0, 0) || !expand(dest + 2 * stride, -3.0, 0) || !expand(dest + 3 * stride, 1.0, 0))
         return NRPY_ERR_BCMAP;
       finish(dest, dest);
+      bc->face_by_distance = bc->face_by_distance && nrpy_face_by_distance(bc->N, o);
     }
     for (const inner_bc &n : bc->inner[gz]) {
       const int dest = IDX3S(n.inner_bc_dest_pt.i0, n.inner_bc_dest_pt.i1, n.inner_bc_dest_pt.i2);
