@@ -53,8 +53,8 @@ int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *params, const
  * those in xx among them, and dt are fixed at capture), replayed nsteps times per MoL_graph_launch,
  * freed with MoL_graph_free. Creating it reads no device memory; a launch reads all of it, the
  * coordinates too, in its stream's order.
- * The captured step takes two launches per substep instead of one per layer and face group, with
- * the same values. It allocates device memory that the graph owns until MoL_graph_free
+ * The captured step takes two launches per substep instead of one per layer and face group, and
+ * equals it to rounding (1e-13 of the largest value). It allocates device memory that the graph owns until MoL_graph_free
  * (2 NUM_EVOL_GFS + 5 gridfunctions); without that memory it captures the step above. */
 int MoL_sommerfeld_graph_create(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3],
                                 const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs,

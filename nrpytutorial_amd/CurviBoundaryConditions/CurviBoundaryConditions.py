@@ -219,7 +219,8 @@ class sommerfeld_boundary_condition_class():
         (the three cofactors and the determinant, or the simplified contraction's three
         coefficients over 1), nrpy_sommerfeld_dfdr_from contracts the stencils with them, and
         nrpy_sommerfeld_r_dfdr is one after the other. The geometry is opaque to the compiler in
-        between, so that no multiply-add is contracted across and both uses round alike."""
+        between, so that no multiply-add is contracted across; within each part the compiler may
+        contract differently from use to use (1 ulp)."""
         from .. import outputC as oc
         from ..codegen import bundle as bd
         if self._simplified():
@@ -699,8 +700,8 @@ _SOMMERFELD_CHAIN = r'''
 // point's chain from the interior out, at most 3 NGHOSTS multiply-adds, an inner point that of
 // the point it copies, and does the RK4 update there. Every point's FACE follows from its
 // indices: the axis with the largest distance outside the interior, the last of equals
-// (nrpy_sommerfeld_chainable checks it against the lists). The arithmetic is that of
-// nrpy_sommerfeld_rhs.
+// (nrpy_sommerfeld_chainable: known from building the lists). The operations are those of
+// nrpy_sommerfeld_rhs; the results agree to rounding.
 // Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
 // launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
 // chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table

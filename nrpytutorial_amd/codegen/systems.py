@@ -192,7 +192,7 @@ def _sommerfeld_glue(fd_order, rhs_call, shell_call=None, rim=None, **defaults):
                            .replace("SUBSTEP", str(S)) +
                            "  if ((rc = nrpy_sommerfeld_chain(%d, params, bcstruct, evol_gf_parity, R, y_n_gfs, "
                            "y_nplus1_running_total_gfs, %s, dt, stream))) return rc;\n" % (S, o))
-        step += ("// The same step as two launches per substep (values those of the unfused step); R:\n"
+        step += ("// The same step as two launches per substep (equal to the unfused step to rounding); R:\n"
                  "// the scratch of nrpy_sommerfeld_chain_scratch, not shared with a step on another stream.\n"
                  "static int nrpy_sommerfeld_chain_step(const paramstruct *params, %s, double *y_n_gfs, double *k_odd_gfs, "
                  "double *k_even_gfs, double *y_nplus1_running_total_gfs, double *R, const double dt, "

@@ -1046,8 +1046,8 @@ extern "C" int apply_bcs_sommerfeld(const paramstruct *params, double *xx[3], co
 // point's chain from the interior out, at most 3 NGHOSTS multiply-adds, an inner point that of
 // the point it copies, and does the RK4 update there. Every point's FACE follows from its
 // indices: the axis with the largest distance outside the interior, the last of equals
-// (nrpy_sommerfeld_chainable checks it against the lists). The arithmetic is that of
-// nrpy_sommerfeld_rhs.
+// (nrpy_sommerfeld_chainable: known from building the lists). The operations are those of
+// nrpy_sommerfeld_rhs; the results agree to rounding.
 // Both launches are bound by latency. On the Maxwell 50x4x100 grid (MI355X) the condition's 9
 // launches of 4-7 us with gaps of 2.4 us took 70 us a substep; one launch that evaluated the
 // chains point after point 48 us, 25 us with r, the cofactors and the determinant from a table
@@ -1365,7 +1365,7 @@ extern "C" int MoL_step_forward_in_time_sommerfeld_unfused(const paramstruct *pa
 extern "C" int MoL_step_forward_in_time_sommerfeld(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, const double dt, hipStream_t stream) {
   return MoL_step_forward_in_time_sommerfeld_unfused(params, rfmstruct, xx, bcstruct, y_n_gfs, k_odd_gfs, k_even_gfs, y_nplus1_running_total_gfs, dt, stream);
 }
-// The same step as two launches per substep (values those of the unfused step); R:
+// The same step as two launches per substep (equal to the unfused step to rounding); R:
 // the scratch of nrpy_sommerfeld_chain_scratch, not shared with a step on another stream.
 static int nrpy_sommerfeld_chain_step(const paramstruct *params, const rfm_struct *rfmstruct, double *xx[3], const bc_struct *bcstruct, double *y_n_gfs, double *k_odd_gfs, double *k_even_gfs, double *y_nplus1_running_total_gfs, double *R, const double dt, hipStream_t stream) {
   int rc;

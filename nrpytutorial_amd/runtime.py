@@ -344,7 +344,8 @@ class Evolution:
         """nsteps RK4 steps with the Sommerfeld condition on the RHS and the update at every point,
         replayed from a captured hipGraph (or launched eagerly). unfused: launch the step in the
         reference's order of operations (MoL_step_forward_in_time_sommerfeld_unfused) eagerly;
-        the default step is fused where the grid allows it and gives the same values."""
+        the default step is fused where the grid allows it: the same values on Cartesian grids, on
+        curvilinear ones (replayed) the same to rounding."""
         if unfused:
             for _ in range(nsteps):
                 check(self.lib.MoL_step_forward_in_time_sommerfeld_unfused(

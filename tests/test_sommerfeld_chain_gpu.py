@@ -4,6 +4,8 @@ step in the reference's order (MoL_step_forward_in_time_sommerfeld_unfused), to 
 each of three steps, on grids that are not multiples of the tiles and on the shortest axes the
 radial stencils and the parity maps take. Two evolutions that share one grid are stepped in
 turn, so scratch memory that belonged to the grid would show."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -11,6 +13,14 @@ from test_sommerfeld_gpu import CASES, _setup
 
 pytestmark = pytest.mark.gpu
 CURVILINEAR = [c for c in CASES if "cartesian" not in c[0]]
+
+
+def _launches(b, graph):
+    """Nodes of a captured step (MoL_graph begins with its hipGraph_t)."""
+    n = ctypes.c_size_t()
+    handle = ctypes.cast(graph, ctypes.POINTER(ctypes.c_void_p))[0]
+    assert b.lib.hipGraphGetNodes(ctypes.c_void_p(handle), None, ctypes.byref(n)) == 0
+    return n.value
 
 
 @pytest.mark.parametrize("Nxx", [(20, 18, 16), (9, 4, 10), (33, 6, 12)], ids=str)
@@ -31,6 +41,8 @@ def test_captured_step_equals_unfused(torch_cuda, bundle, pars, Nxx):
         for e in (ref, ref2):
             e.step_sommerfeld(dt, 1, unfused=True)
         torch.cuda.synchronize()
+        for e in (ev, other):
+            assert _launches(b, e.som_graph) == 8       # two a substep: not the unfused step, captured
         for e, r in ((ev, ref), (other, ref2)):
             assert np.isfinite(r.y_n.cpu().numpy()).all()
             for got, want in ((e.y_n, r.y_n), (e.rt, r.rt)):
