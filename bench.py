@@ -174,9 +174,9 @@ def bench_bl(torch):
 
 def bench_adjoint(torch, N=128, nsteps=200):
     """Adjoint scalar wave: 128^3 on [-10,10]^3, 200 RK4 steps, J = 0.5 sum uu(T)^2 dx^3,
-    gradient w.r.t. 16 bump amplitudes through the checkpointed autograd evolution.
-    Reports forward-step and adjoint-step times (the adjoint step includes recomputing
-    its three stage states, and the checkpointed backward re-runs each forward step)."""
+    gradient w.r.t. 16 bump amplitudes through the autograd evolution.
+    Reports forward-step and adjoint-step times (the system is linear: neither the adjoint step
+    nor the backward pass recomputes a state)."""
     from nrpytutorial_amd.runtime import Bundle, Grid, Evolution
     from nrpytutorial_amd.adjoint import RK4Adjoint, RK4Evolve
     from nrpytutorial_amd.workloads import scalarwave_bump_parameters, scalarwave_bump_basis_torch

@@ -7,11 +7,10 @@ runs the four stage adjoints of one step (see the generated code for the
 algebra). This module adds what lies above one step:
 
 * ``forward_checkpointed``: N steps keeping every K-th state (K ~ sqrt(N));
-* ``backward_checkpointed``: for each segment, last first, recompute its
-  states from the checkpoint, then step the cotangent back through them, so
-  memory holds ~2 sqrt(N) states and each forward step is run twice; the step
-  adjoints of the linear systems (scalar wave, Maxwell) read no state, and
-  theirs are not recomputed;
+* ``backward_checkpointed``: the cotangent stepped back through all of them.
+  The systems with a ``MoL_step_adjoint`` (scalar wave, Maxwell) are linear
+  and their step adjoints read no state, so none is recomputed: each forward
+  step is run once, and the checkpoints are for the caller;
 * ``RK4Evolve``: a ``torch.autograd.Function`` wrapping both, so a loss
   written in torch on the final state differentiates through the evolution.
 
@@ -36,12 +35,12 @@ class RK4Adjoint:
             raise NrpyError("bundle %s has no generated adjoint" % b.name)
         self.ev = ev
         self.lib = b.lib
-        # False: MoL_step_adjoint of a linear right-hand side, which needs no states
-        self.reads_state = b.meta.get("step_adjoint_reads_state", True)
         g = ev.g
         n = len(b.evol)
-        self.U = [g.empty(n) for _ in range(3)]
-        self.rt, self.acc, self.kbar, self.w = (g.empty(n) for _ in range(4))
+        self.acc, self.kbar, self.w = (g.empty(n) for _ in range(3))
+        # arguments that the adjoint of a linear right-hand side neither reads nor writes
+        self.U = [self.w] * 3
+        self.rt = self.w
         self.G = g.empty(len(b.meta["vjp_slots"]))
         f = self.lib.MoL_step_adjoint
         f.restype = ctypes.c_int
@@ -92,17 +91,8 @@ def backward_checkpointed(ev, adj, cps, K, dt, nsteps, lam_T):
     lam = lam_T.clone()
     adj.bc_T(lam)
     for start in sorted(cps, reverse=True):
-        end = min(start + K, nsteps)
-        states = [cps[start]]
-        if adj.reads_state:
-            ev.y_n.copy_(cps[start])
-            for _ in range(start, end - 1):
-                ev.step(dt, 1, use_graph=True)
-                states.append(ev.y_n.clone())
-        else:
-            states *= end - start
-        for s in reversed(states):
-            adj.step_back(s, lam, dt)
+        for _ in range(start, min(start + K, nsteps)):
+            adj.step_back(cps[start], lam, dt)       # (the state is not read)
     return lam
 
 

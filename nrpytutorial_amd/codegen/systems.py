@@ -712,7 +712,6 @@ def scalarwave_cartesian():
              _mol_adjoint_glue(adj.linear_stage_kernel(exprs, slots, gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]
-    meta["step_adjoint_reads_state"] = False
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta.update({"bundle": "scalarwave_cartesian", "CoordSystem": "Cartesian", "rfm_tables": [],
                  "kernels": ["rhs_eval", "initial_data"], "has_ricci": False, "has_detg": False})
@@ -771,7 +770,6 @@ def maxwell_cartesian():
              _mol_adjoint_glue(adj.linear_stage_kernel(exprs, slots, gri.gridfunction_lists()[0])), som_src]
     meta["sommerfeld"] = som_meta
     meta["vjp_slots"] = [sl[0] for sl in slots]
-    meta["step_adjoint_reads_state"] = False
     meta["cost"] = {"rhs_eval": bd.count_body(body)}
     meta["kernel_ids"] = dict(bd.lp.KERNEL_IDS)
     meta.update({"bundle": "maxwell_cartesian", "family": "maxwell", "CoordSystem": "Cartesian", "rfm_tables": [],
