@@ -80,14 +80,88 @@ def test_fill_lists_are_the_composed_map(name, Nxx):
     print("%s: %d ghosts, %d read by stencils, %d generic rows" % (name, (~inside).sum(), read.sum(), generic))
 
 
-@pytest.mark.parametrize("name", ["scalarwave_cartesian", "bssn_cartesian", "bssn_spherical_sym2", "maxwell_sinhcylindrical"])
+# kernels of the RK4 step: substeps (also as one launch of several, "body", and over a batch) and
+# Ricci tensor; the merged kernel itself only calls the bodies
+STEP_KERNEL = re.compile(r"\n(?:__global__|static __device__) [^\n]*?\b((?:rhs_eval_rk4_substep\w*?|Ricci_eval(?:_g\d+)?)"
+                         r"__(?:gpu_batched|gpu|body))\(")
+PLAIN = re.compile(r"double (\w+) = (in_gfs|auxevol_gfs)\[IDX4\((\w+)GF, i0([+-]\d+)?,i1([+-]\d+)?,i2([+-]\d+)?\)\];")
+HALO = re.compile(r"in_gfs\[IDX4\(\w+GF, nrpy_xl < (\d+) \? i0 - (\d+) : i0 \+ (\d+),i1,i2\)\];")
+BOX = re.compile(r"copy the \((\d+) x (\d+) x (\d+)\)-point box")
+LDS = re.compile(r"double (\w+) = nrpy_lds\[\d+\]\[nrpy_li \+ (-?\d+)\];")
+MOVE = re.compile(r"double (\w+) = nrpy_xshift<\d+, \d+, (-?\d+)>\(")
+NAMED = re.compile(r"_i0(?:([pm])(\d+))?_i1(?:([pm])(\d+))?_i2(?:([pm])(\d+))?$")
+
+
+def _named(name):
+    """The offset in the name that the finite-difference emitter gives a read (none: the centre)."""
+    m = NAMED.search(name)
+    if not m:
+        return (0, 0, 0)
+    return tuple((-1 if m.group(2 * d + 1) == "m" else 1) * int(m.group(2 * d + 2) or 0) for d in range(3))
+
+
+def _kernel_offsets(kernel):
+    """(offsets a kernel reads gridfunctions at, number of reads by kind), from the addresses: plain reads,
+    reads of an LDS box (split into rows and planes of the box), lane moves and their halo loads."""
+    found, kinds = [], {"plain": 0, "lds": 0, "move": 0}
+    for name, _, _, *o in PLAIN.findall(kernel):
+        found.append((name, tuple(int(v or 0) for v in o)))
+        kinds["plain"] += 1
+    for a, b, c in HALO.findall(kernel):
+        assert a == b == c
+        found += [("nrpy_h", (int(a), 0, 0)), ("nrpy_h", (-int(a), 0, 0))]
+    box = [tuple(int(v) for v in m) for m in BOX.findall(kernel)]
+    assert len(box) <= 1
+    for name, k in LDS.findall(kernel):
+        bx, by, _ = box[0]
+        k, o = int(k), []
+        for n in (bx, by):
+            r = (k + n // 2) % n - n // 2
+            o.append(r)
+            k = (k - r) // n
+        found.append((name, tuple(o) + (k,)))
+        kinds["lds"] += 1
+    for name, k in MOVE.findall(kernel):
+        found.append((name, (int(k), 0, 0)))
+        kinds["move"] += 1
+    for name, o in found:
+        assert name.startswith("nrpy_") or _named(name) == o, (name, o)
+    # nothing that reads a gridfunction went unrecognised
+    assert len(re.findall(r"\bin_gfs\[IDX4\(|\bauxevol_gfs\[IDX4\(\w+GF, i0[^\]]*\)\];", kernel)) == \
+        kinds["plain"] + len(HALO.findall(kernel))
+    assert kernel.count("[nrpy_li + ") == kinds["lds"] and kernel.count("nrpy_xshift<") == kinds["move"]
+    return {o for _, o in found} - {(0, 0, 0)}, kinds
+
+
+SUBSTEP = ["rhs_eval_rk4_substep__gpu"]
+GROUPS = ["rhs_eval_rk4_substep_g%d__gpu" % k for k in range(3)]
+RICCI = ["Ricci_eval__gpu", "Ricci_eval_g0__gpu", "Ricci_eval_g1__gpu"]
+BATCHED = ["Ricci_eval__gpu_batched"] + [k + "_batched" for k in GROUPS]
+KERNELS = {"scalarwave_cartesian": SUBSTEP + ["rhs_eval_rk4_substep_edge__gpu", "rhs_eval_rk4_substep_shell__gpu"],
+           "maxwell_cartesian": SUBSTEP + ["rhs_eval_rk4_substep_edge__gpu", "rhs_eval_rk4_substep_shell__gpu"],
+           "bssn_cartesian": GROUPS + RICCI + BATCHED,
+           "bssn_spherical_sym2": GROUPS + RICCI + BATCHED + [k.replace("gpu", "body") for k in GROUPS],
+           "maxwell_sinhcylindrical": SUBSTEP + ["rhs_eval_rk4_substep_rim__gpu"],
+           "scalarwave_symtp": SUBSTEP + ["rhs_eval_rk4_substep_rim__gpu"],
+           "scalarwave_sinhsphericalv2": SUBSTEP + ["rhs_eval_rk4_substep_rim__gpu"]}
+
+
+@pytest.mark.parametrize("name", sorted(KERNELS))
 def test_stage_offsets_are_what_the_step_kernels_read(name):
-    """Every offset at which a substep kernel or Ricci kernel of the bundle reads a gridfunction
-    (plain reads, LDS boxes and lane moves) is in the list."""
+    """The list holds exactly the offsets at which the bundle's substep and Ricci kernels read gridfunctions
+    (plain reads, LDS boxes and lane moves), each kernel named above among them."""
     text = open(os.path.join(GENDIR, name + ".hip")).read()
-    offsets = set(_offsets(name))
-    for m in re.finditer(r"\n__global__ void __launch_bounds__\([^)]*\) (rhs_eval_rk4_substep\w*|Ricci_eval_g\d+)__gpu\(", text):
-        kernel = text[m.start():text.index("\n}\n", m.start())]
-        for o in re.findall(r"in_gfs\[IDX4\(\w+GF, i0([+-]\d+)?,i1([+-]\d+)?,i2([+-]\d+)?\)\]", kernel):
-            o = tuple(int(v or 0) for v in o)
-            assert o == (0, 0, 0) or o in offsets, (m.group(1), o)
+    offsets, read, kernels, kinds = set(_offsets(name)), set(), [], {"plain": 0, "lds": 0, "move": 0}
+    for m in STEP_KERNEL.finditer(text):
+        if m.group(1) == "rhs_eval_rk4_substep_merged__gpu":
+            continue
+        o, n = _kernel_offsets(text[m.start():text.index("\n}\n", m.start())])
+        assert o and o <= offsets, (m.group(1), sorted(o - offsets))
+        read |= o
+        kernels.append(m.group(1))
+        for k in kinds:
+            kinds[k] += n[k]
+    assert sorted(kernels) == sorted(KERNELS[name])
+    assert read == offsets
+    print("%s: %d offsets, %s" % (name, len(offsets), kinds))
+    assert kinds["plain"] > 0 and (kinds["lds"] > 0 and kinds["move"] > 0) == (name == "bssn_cartesian")
