@@ -56,9 +56,9 @@ static const int8_t MAXFACE = -1;
 static const int8_t NUL = +0;
 static const int8_t MINFACE = +1;
 
-// One ghost point of the composed map in the form the fill kernel reads (16 bytes). Almost
-// every row is a product of one-dimensional quadratic extrapolations (or a parity copy of
-// such a point, or of an interior point): its value is
+// One ghost point of the composed map in the form the fill kernel reads (16 bytes). With up to
+// three ghost layers a row is a product of one-dimensional quadratic extrapolations (or a parity
+// copy of such a point, or of an interior point); a fourth layer has generic rows. A product's value is
 //   sign * sum_{c,b,a} w_c w_b w_a f[base + a s0 + b s1 + c s2],
 // where along axis d the factor is one term (no extrapolation) or three, w the weights of
 // layer l = 1, 2, 3 outside the interior and s_d the index stride inwards. code holds 3 bits per
