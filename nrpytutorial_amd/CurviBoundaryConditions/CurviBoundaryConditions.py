@@ -214,13 +214,12 @@ class sommerfeld_boundary_condition_class():
                 "  (void)fdD0; (void)fdD1; (void)fdD2;\n" + text + "}\n")
 
     def geometry_functions(self):
-        """dfdr_function in two parts, for bundles with a kernel that keeps the geometry in a table:
+        """dfdr_function in two parts, for the kernels that keep the geometry in a table:
         nrpy_sommerfeld_geometry gives r and what the derivative needs of the Jacobian at a point
         (the three cofactors and the determinant, or the simplified contraction's three
-        coefficients over 1), nrpy_sommerfeld_dfdr_from contracts the stencils with them, and
-        nrpy_sommerfeld_r_dfdr is one after the other. The geometry is opaque to the compiler in
-        between, so that no multiply-add is contracted across; within each part the compiler may
-        contract differently from use to use (1 ulp)."""
+        coefficients over 1), nrpy_sommerfeld_dfdr_from contracts the stencils with them. The
+        other kernels keep dfdr_function: in two parts it issues the stencils' loads after the
+        geometry and divides once more per coefficient (eager steps 6 to 25% slower)."""
         from .. import outputC as oc
         from ..codegen import bundle as bd
         if self._simplified():
@@ -255,18 +254,7 @@ class sommerfeld_boundary_condition_class():
                 "const int F0, const int F1, const int F2, const int i0, const int i1, const int i2) {\n" + dunpack +
                 "  double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;\n" + coef + dirs +
                 "  const double cof0 = geo[1], cof1 = geo[2], cof2 = geo[3];\n"
-                "  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];\n}\n"
-                "// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's\n"
-                "// FACE (CurviBoundaryConditions.py:329-516).\n"
-                "template <typename FA>\n"
-                "static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ "
-                "xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, "
-                "const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, "
-                "double *dfdr_out) {\n"
-                "  double geo[5];\n  nrpy_sommerfeld_geometry(params, xx0_arr[i0], xx1_arr[i1], xx2_arr[i2], geo);\n"
-                "#pragma unroll\n  for (int k = 0; k < 5; k++) asm(\"\" : \"+v\"(geo[k]));\n"
-                "  *r_out = geo[0];\n"
-                "  *dfdr_out = nrpy_sommerfeld_dfdr_from(params, geo, fa, F0, F1, F2, i0, i1, i2);\n}\n")
+                "  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];\n}\n")
 
     @staticmethod
     def _stencil_constants(fd_order):
@@ -284,9 +272,8 @@ class sommerfeld_boundary_condition_class():
         # the one-sided stencils reach fd_order points inward from a point within NGHOSTS of an edge
         minn = ("#define NRPY_SOMMERFELD_MIN_N (NGHOSTS + %d + 1)\n#define NRPY_SOMMERFELD_FD %d\n"
                 % (self.fd_order, self.fd_order))
-        return (self.sommerfeld_params() + minn + (self.geometry_functions() if chain else self.dfdr_function()) +
-                _SOMMERFELD_KERNELS +
-                (_SOMMERFELD_CHAIN if chain else ""))
+        return (self.sommerfeld_params() + minn + self.dfdr_function() + _SOMMERFELD_KERNELS +
+                (self.geometry_functions() + _SOMMERFELD_CHAIN if chain else ""))
 
     def write_sommerfeld_main_Ccode(self, Ccodesdir):
         os.makedirs(os.path.join(Ccodesdir, "boundary_conditions"), exist_ok=True)

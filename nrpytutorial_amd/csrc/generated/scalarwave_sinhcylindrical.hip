@@ -581,65 +581,24 @@ static __constant__ double evolgf_radial_falloff_power[NUM_EVOL_GFS] = {3.0, 3.0
 static __constant__ double evolgf_speed[NUM_EVOL_GFS] = {1.0, 1.0};
 #define NRPY_SOMMERFELD_MIN_N (NGHOSTS + 4 + 1)
 #define NRPY_SOMMERFELD_FD 4
-// r and the radial derivative's geometry at a point: geo = r, then a_i and b of
-// d f/d r = sum_i fdD_i a_i / b.
-static __device__ void nrpy_sommerfeld_geometry(const paramstruct &params, const double xx0, const double xx1, const double xx2, double *geo) {
+// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's
+// FACE (CurviBoundaryConditions.py:329-516).
+template <typename FA>
+static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, double *dfdr_out) {
   const double AMPLRHO = params.AMPLRHO;
   const double AMPLZ = params.AMPLZ;
-  const double SINHWRHO = params.SINHWRHO;
-  const double SINHWZ = params.SINHWZ;
-  (void)xx0; (void)xx1; (void)xx2;
-  double J00, J01, J02, J10, J11, J12, J20, J21, J22;
-  const double tmp_0 = (1.0/((SINHWRHO)));
-  const double tmp_1 = tmp_0*xx0;
-  const double tmp_2 = exp(tmp_1);
-  const double tmp_3 = exp(-tmp_1);
-  const double tmp_4 = tmp_2 - tmp_3;
-  const double tmp_5 = ((AMPLRHO)*(AMPLRHO))/((exp(tmp_0) - exp(-tmp_0))*(exp(tmp_0) - exp(-tmp_0)));
-  const double tmp_6 = (1.0/((SINHWZ)));
-  const double tmp_7 = tmp_6*xx2;
-  const double tmp_8 = exp(tmp_7);
-  const double tmp_9 = exp(-tmp_7);
-  const double tmp_10 = tmp_8 - tmp_9;
-  const double tmp_11 = ((tmp_10)*(tmp_10));
-  const double tmp_12 = exp(tmp_6) - exp(-tmp_6);
-  const double tmp_13 = ((AMPLZ)*(AMPLZ))/((tmp_12)*(tmp_12));
-  const double tmp_14 = tmp_11*tmp_13;
-  const double tmp_15 = tmp_14 + ((tmp_4)*(tmp_4))*tmp_5;
-  const double tmp_16 = sqrt(tmp_15);
-  const double tmp_17 = (1.0/((tmp_16)));
-  const double tmp_18 = ((1.0/2.0))*tmp_17;
-  const double tmp_19 = 2*tmp_0;
-  const double tmp_20 = tmp_4*tmp_5*(tmp_19*tmp_2 + tmp_19*tmp_3);
-  const double tmp_21 = tmp_6*tmp_8;
-  const double tmp_22 = tmp_6*tmp_9;
-  const double tmp_23 = 2*tmp_21 + 2*tmp_22;
-  const double tmp_24 = (1.0/sqrt(-tmp_14/tmp_15 + 1));
-  const double tmp_25 = (1.0/((tmp_12)));
-  const double tmp_26 = ((1.0/2.0))/pow(tmp_15, (3.0/2.0));
-  geo[0] = tmp_16;
-  J00 = tmp_18*tmp_20;
-  J01 = 0;
-  J02 = tmp_10*tmp_13*tmp_18*tmp_23;
-  J10 = AMPLZ*tmp_10*tmp_20*tmp_24*tmp_25*tmp_26;
-  J11 = 0;
-  J12 = -tmp_24*(-((AMPLZ)*(AMPLZ)*(AMPLZ))*tmp_11*tmp_23*tmp_26/((tmp_12)*(tmp_12)*(tmp_12)) + AMPLZ*tmp_17*tmp_25*(tmp_21 + tmp_22));
-  J20 = 0;
-  J21 = 1;
-  J22 = 0;
-  const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;
-  geo[1] = cof0; geo[2] = cof1; geo[3] = cof2;
-  geo[4] = J00*cof0 + J01*cof1 + J02*cof2;
-}
-template <typename FA>
-static __device__ double nrpy_sommerfeld_dfdr_from(const paramstruct &params, const double *geo, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2) {
   const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
   const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
   const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
+  const double SINHWRHO = params.SINHWRHO;
+  const double SINHWZ = params.SINHWZ;
   const double invdx0 = params.invdx0;
   const double invdx1 = params.invdx1;
   const double invdx2 = params.invdx2;
+  const double xx0 = xx0_arr[i0], xx1 = xx1_arr[i1], xx2 = xx2_arr[i2];
+  (void)xx0; (void)xx1; (void)xx2; (void)F0; (void)F1; (void)F2;
   double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;
+  (void)fdD0; (void)fdD1; (void)fdD2;
   const double u0 = -25./12., u1 = 4., u2 = -3., u3 = 4./3., u4 = -1./4.;
   const double c1 = 2./3., c2 = 1./12.;
   {
@@ -672,19 +631,46 @@ static __device__ double nrpy_sommerfeld_dfdr_from(const paramstruct &params, co
     const double cen = (-c2*fa(i0,i1,nrpy_ic2+2) + c1*fa(i0,i1,nrpy_ic2+1) - c1*fa(i0,i1,nrpy_ic2+-1) + c2*fa(i0,i1,nrpy_ic2+-2))*invdx2;
     fdD2 = one_sided ? one : cen;
   }
-  const double cof0 = geo[1], cof1 = geo[2], cof2 = geo[3];
-  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];
-}
-// r and d f/d r at (i0,i1,i2) of one gridfunction f, read as fa(i0,i1,i2); F = the point's
-// FACE (CurviBoundaryConditions.py:329-516).
-template <typename FA>
-static __device__ void nrpy_sommerfeld_r_dfdr(const paramstruct &params, const double *__restrict__ xx0_arr, const double *__restrict__ xx1_arr, const double *__restrict__ xx2_arr, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2, double *r_out, double *dfdr_out) {
-  double geo[5];
-  nrpy_sommerfeld_geometry(params, xx0_arr[i0], xx1_arr[i1], xx2_arr[i2], geo);
-#pragma unroll
-  for (int k = 0; k < 5; k++) asm("" : "+v"(geo[k]));
-  *r_out = geo[0];
-  *dfdr_out = nrpy_sommerfeld_dfdr_from(params, geo, fa, F0, F1, F2, i0, i1, i2);
+  double J00, J01, J02, J10, J11, J12, J20, J21, J22;
+  const double tmp_0 = (1.0/((SINHWRHO)));
+  const double tmp_1 = tmp_0*xx0;
+  const double tmp_2 = exp(tmp_1);
+  const double tmp_3 = exp(-tmp_1);
+  const double tmp_4 = tmp_2 - tmp_3;
+  const double tmp_5 = ((AMPLRHO)*(AMPLRHO))/((exp(tmp_0) - exp(-tmp_0))*(exp(tmp_0) - exp(-tmp_0)));
+  const double tmp_6 = (1.0/((SINHWZ)));
+  const double tmp_7 = tmp_6*xx2;
+  const double tmp_8 = exp(tmp_7);
+  const double tmp_9 = exp(-tmp_7);
+  const double tmp_10 = tmp_8 - tmp_9;
+  const double tmp_11 = ((tmp_10)*(tmp_10));
+  const double tmp_12 = exp(tmp_6) - exp(-tmp_6);
+  const double tmp_13 = ((AMPLZ)*(AMPLZ))/((tmp_12)*(tmp_12));
+  const double tmp_14 = tmp_11*tmp_13;
+  const double tmp_15 = tmp_14 + ((tmp_4)*(tmp_4))*tmp_5;
+  const double tmp_16 = sqrt(tmp_15);
+  const double tmp_17 = (1.0/((tmp_16)));
+  const double tmp_18 = ((1.0/2.0))*tmp_17;
+  const double tmp_19 = 2*tmp_0;
+  const double tmp_20 = tmp_4*tmp_5*(tmp_19*tmp_2 + tmp_19*tmp_3);
+  const double tmp_21 = tmp_6*tmp_8;
+  const double tmp_22 = tmp_6*tmp_9;
+  const double tmp_23 = 2*tmp_21 + 2*tmp_22;
+  const double tmp_24 = (1.0/sqrt(-tmp_14/tmp_15 + 1));
+  const double tmp_25 = (1.0/((tmp_12)));
+  const double tmp_26 = ((1.0/2.0))/pow(tmp_15, (3.0/2.0));
+  *r_out = tmp_16;
+  J00 = tmp_18*tmp_20;
+  J01 = 0;
+  J02 = tmp_10*tmp_13*tmp_18*tmp_23;
+  J10 = AMPLZ*tmp_10*tmp_20*tmp_24*tmp_25*tmp_26;
+  J11 = 0;
+  J12 = -tmp_24*(-((AMPLZ)*(AMPLZ)*(AMPLZ))*tmp_11*tmp_23*tmp_26/((tmp_12)*(tmp_12)*(tmp_12)) + AMPLZ*tmp_17*tmp_25*(tmp_21 + tmp_22));
+  J20 = 0;
+  J21 = 1;
+  J22 = 0;
+  const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;
+  *dfdr_out = (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/(J00*cof0 + J01*cof1 + J02*cof2);
 }
 
 // The radiation condition's right-hand side at outer point (i0,i1,i2) of gridfunction gf
@@ -1070,6 +1056,100 @@ extern "C" int apply_bcs_sommerfeld(const paramstruct *params, double *xx[3], co
     }
   }
   return hipGetLastError() == hipSuccess ? NRPY_OK : NRPY_ERR_LAUNCH;
+}
+// r and the radial derivative's geometry at a point: geo = r, then a_i and b of
+// d f/d r = sum_i fdD_i a_i / b.
+static __device__ void nrpy_sommerfeld_geometry(const paramstruct &params, const double xx0, const double xx1, const double xx2, double *geo) {
+  const double AMPLRHO = params.AMPLRHO;
+  const double AMPLZ = params.AMPLZ;
+  const double SINHWRHO = params.SINHWRHO;
+  const double SINHWZ = params.SINHWZ;
+  (void)xx0; (void)xx1; (void)xx2;
+  double J00, J01, J02, J10, J11, J12, J20, J21, J22;
+  const double tmp_0 = (1.0/((SINHWRHO)));
+  const double tmp_1 = tmp_0*xx0;
+  const double tmp_2 = exp(tmp_1);
+  const double tmp_3 = exp(-tmp_1);
+  const double tmp_4 = tmp_2 - tmp_3;
+  const double tmp_5 = ((AMPLRHO)*(AMPLRHO))/((exp(tmp_0) - exp(-tmp_0))*(exp(tmp_0) - exp(-tmp_0)));
+  const double tmp_6 = (1.0/((SINHWZ)));
+  const double tmp_7 = tmp_6*xx2;
+  const double tmp_8 = exp(tmp_7);
+  const double tmp_9 = exp(-tmp_7);
+  const double tmp_10 = tmp_8 - tmp_9;
+  const double tmp_11 = ((tmp_10)*(tmp_10));
+  const double tmp_12 = exp(tmp_6) - exp(-tmp_6);
+  const double tmp_13 = ((AMPLZ)*(AMPLZ))/((tmp_12)*(tmp_12));
+  const double tmp_14 = tmp_11*tmp_13;
+  const double tmp_15 = tmp_14 + ((tmp_4)*(tmp_4))*tmp_5;
+  const double tmp_16 = sqrt(tmp_15);
+  const double tmp_17 = (1.0/((tmp_16)));
+  const double tmp_18 = ((1.0/2.0))*tmp_17;
+  const double tmp_19 = 2*tmp_0;
+  const double tmp_20 = tmp_4*tmp_5*(tmp_19*tmp_2 + tmp_19*tmp_3);
+  const double tmp_21 = tmp_6*tmp_8;
+  const double tmp_22 = tmp_6*tmp_9;
+  const double tmp_23 = 2*tmp_21 + 2*tmp_22;
+  const double tmp_24 = (1.0/sqrt(-tmp_14/tmp_15 + 1));
+  const double tmp_25 = (1.0/((tmp_12)));
+  const double tmp_26 = ((1.0/2.0))/pow(tmp_15, (3.0/2.0));
+  geo[0] = tmp_16;
+  J00 = tmp_18*tmp_20;
+  J01 = 0;
+  J02 = tmp_10*tmp_13*tmp_18*tmp_23;
+  J10 = AMPLZ*tmp_10*tmp_20*tmp_24*tmp_25*tmp_26;
+  J11 = 0;
+  J12 = -tmp_24*(-((AMPLZ)*(AMPLZ)*(AMPLZ))*tmp_11*tmp_23*tmp_26/((tmp_12)*(tmp_12)*(tmp_12)) + AMPLZ*tmp_17*tmp_25*(tmp_21 + tmp_22));
+  J20 = 0;
+  J21 = 1;
+  J22 = 0;
+  const double cof0 = J11*J22 - J12*J21, cof1 = -(J10*J22 - J12*J20), cof2 = J10*J21 - J11*J20;
+  geo[1] = cof0; geo[2] = cof1; geo[3] = cof2;
+  geo[4] = J00*cof0 + J01*cof1 + J02*cof2;
+}
+template <typename FA>
+static __device__ double nrpy_sommerfeld_dfdr_from(const paramstruct &params, const double *geo, FA fa, const int F0, const int F1, const int F2, const int i0, const int i1, const int i2) {
+  const int Nxx_plus_2NGHOSTS0 = params.Nxx_plus_2NGHOSTS0;
+  const int Nxx_plus_2NGHOSTS1 = params.Nxx_plus_2NGHOSTS1;
+  const int Nxx_plus_2NGHOSTS2 = params.Nxx_plus_2NGHOSTS2;
+  const double invdx0 = params.invdx0;
+  const double invdx1 = params.invdx1;
+  const double invdx2 = params.invdx2;
+  double fdD0 = 1e100, fdD1 = 1e100, fdD2 = 1e100;
+  const double u0 = -25./12., u1 = 4., u2 = -3., u3 = 4./3., u4 = -1./4.;
+  const double c1 = 2./3., c2 = 1./12.;
+  {
+    const bool one_sided = abs(F0) == 1 || i0 + NGHOSTS >= Nxx_plus_2NGHOSTS0 || i0 - NGHOSTS <= 0;
+    int S = F0;
+    if (i0 + NGHOSTS >= Nxx_plus_2NGHOSTS0) S = -1;
+    if (i0 - NGHOSTS <= 0) S = +1;
+    const int nrpy_ic0 = min(max(i0, 2), Nxx_plus_2NGHOSTS0 - 1 - 2);
+    const double one = S*(u0*fa(i0,i1,i2) + u1*fa(i0+1*S,i1,i2) + u2*fa(i0+2*S,i1,i2) + u3*fa(i0+3*S,i1,i2) + u4*fa(i0+4*S,i1,i2))*invdx0;
+    const double cen = (-c2*fa(nrpy_ic0+2,i1,i2) + c1*fa(nrpy_ic0+1,i1,i2) - c1*fa(nrpy_ic0+-1,i1,i2) + c2*fa(nrpy_ic0+-2,i1,i2))*invdx0;
+    fdD0 = one_sided ? one : cen;
+  }
+  {
+    const bool one_sided = abs(F1) == 1 || i1 + NGHOSTS >= Nxx_plus_2NGHOSTS1 || i1 - NGHOSTS <= 0;
+    int S = F1;
+    if (i1 + NGHOSTS >= Nxx_plus_2NGHOSTS1) S = -1;
+    if (i1 - NGHOSTS <= 0) S = +1;
+    const int nrpy_ic1 = min(max(i1, 2), Nxx_plus_2NGHOSTS1 - 1 - 2);
+    const double one = S*(u0*fa(i0,i1,i2) + u1*fa(i0,i1+1*S,i2) + u2*fa(i0,i1+2*S,i2) + u3*fa(i0,i1+3*S,i2) + u4*fa(i0,i1+4*S,i2))*invdx1;
+    const double cen = (-c2*fa(i0,nrpy_ic1+2,i2) + c1*fa(i0,nrpy_ic1+1,i2) - c1*fa(i0,nrpy_ic1+-1,i2) + c2*fa(i0,nrpy_ic1+-2,i2))*invdx1;
+    fdD1 = one_sided ? one : cen;
+  }
+  {
+    const bool one_sided = abs(F2) == 1 || i2 + NGHOSTS >= Nxx_plus_2NGHOSTS2 || i2 - NGHOSTS <= 0;
+    int S = F2;
+    if (i2 + NGHOSTS >= Nxx_plus_2NGHOSTS2) S = -1;
+    if (i2 - NGHOSTS <= 0) S = +1;
+    const int nrpy_ic2 = min(max(i2, 2), Nxx_plus_2NGHOSTS2 - 1 - 2);
+    const double one = S*(u0*fa(i0,i1,i2) + u1*fa(i0,i1,i2+1*S) + u2*fa(i0,i1,i2+2*S) + u3*fa(i0,i1,i2+3*S) + u4*fa(i0,i1,i2+4*S))*invdx2;
+    const double cen = (-c2*fa(i0,i1,nrpy_ic2+2) + c1*fa(i0,i1,nrpy_ic2+1) - c1*fa(i0,i1,nrpy_ic2+-1) + c2*fa(i0,i1,nrpy_ic2+-2))*invdx2;
+    fdD2 = one_sided ? one : cen;
+  }
+  const double cof0 = geo[1], cof1 = geo[2], cof2 = geo[3];
+  return (fdD0*cof0 + fdD1*cof1 + fdD2*cof2)/geo[4];
 }
 
 // The whole condition in two launches per substep, for grids with inner boundary points. The
