@@ -301,6 +301,12 @@ def fused_rk4_kernel(name, args_decl, call_args, body_with_writes, loopopts="Int
     return kernel
 
 
+def slab_min_plane(nevol):
+    """Points of a plane up to which tiles go through whole planes (NRPY_BLOCK_COORDS): 500 KB of the
+    evolved gridfunctions."""
+    return 500000 // (8 * nevol)
+
+
 _EDGE_READ = re.compile(r"^(\s*)const double (\w+) = in_gfs\[IDX4\((\w+)GF, i0([+-]\d+)?,i1([+-]\d+)?,i2([+-]\d+)?\)\];$")
 
 

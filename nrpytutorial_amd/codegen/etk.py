@@ -359,7 +359,8 @@ def bssn_etk(bundle_name="bssn_etk"):
     too_wide = addressing.bound_check_code("(A0)", "(A1)") or "0"
     pre = ('#include "../nrpy_runtime_pre.h"\n#define NGHOSTS %d\n#define NRPY_ETK_NPTRS %d\n'
            % (FD_ORDER // 2 + 1, table.size) + ps + "\n" +
-           "#define NRPY_ETK_TILE_TOO_WIDE(A0, A1) (%s)\n" % too_wide + GEOMETRY)
+           "#define NRPY_ETK_TILE_TOO_WIDE(A0, A1) (%s)\n" % too_wide +
+           "#define NRPY_SLAB_MIN_PLANE %d\n" % bd.slab_min_plane(table.n_evol) + GEOMETRY)
     meta = {"bundle": bundle_name, "family": "bssn_etk", "NGHOSTS": FD_ORDER // 2 + 1, "FD_order": FD_ORDER,
             "paramstruct": members,
             "gfs": {"evol": table.evol, "aux": table.aux, "auxevol": table.auxevol},

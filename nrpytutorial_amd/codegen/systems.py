@@ -659,6 +659,8 @@ def _header(NGHOSTS, offsets):
            % (len(offsets), ", ".join("{%d, %d, %d}" % o for o in offsets))
            + "".join("#define NRPY_STAGE_LO%d %s\n" % (d, "0" if a else "NGHOSTS")
                      for d, a in enumerate(stage_axes(offsets)))
+           + "#define NRPY_SLAB_MIN_PLANE %s\n" % (bd.slab_min_plane(len(lists["evol"])) if stage_axes(offsets)[2]
+                                                   else "0x7fffffff")
            + bd.check_params_code())
     meta = {"NGHOSTS": NGHOSTS, "paramstruct": members, "gfs": lists, "evol_parity": parity,
             "aux_parity": [bd.parity_type(n) for n in lists["aux"]],

@@ -40,6 +40,7 @@ static const int8_t nrpy_stage_offsets[12][3] = {{-2, 0, 0}, {-1, 0, 0}, {0, -2,
 #define NRPY_STAGE_LO0 0
 #define NRPY_STAGE_LO1 0
 #define NRPY_STAGE_LO2 0
+#define NRPY_SLAB_MIN_PLANE 31250
 static int nrpy_check_params(const paramstruct *p) {
   if (p->Nxx0 < 1 || p->Nxx1 < 1 || p->Nxx2 < 1) return 1;
   if (p->Nxx_plus_2NGHOSTS0 != p->Nxx0 + 2*NGHOSTS || p->Nxx_plus_2NGHOSTS1 != p->Nxx1 + 2*NGHOSTS ||
@@ -539,7 +540,7 @@ __global__ void __launch_bounds__(256) initial_data__gpu(const paramstruct param
   const int Nxx1 = params.Nxx1;
   const int Nxx2 = params.Nxx2;
   
-  NRPY_BLOCK_COORDS(Nxx_plus_2NGHOSTS0, Nxx_plus_2NGHOSTS1, Nxx_plus_2NGHOSTS2);
+  NRPY_BLOCK_COORDS_POINTWISE(Nxx_plus_2NGHOSTS0, Nxx_plus_2NGHOSTS1, Nxx_plus_2NGHOSTS2);
   const int i0 = 0 + nrpy_bx*(int)blockDim.x + (int)threadIdx.x;
   const int i1 = 0 + nrpy_by*(int)blockDim.y + (int)threadIdx.y;
   const int i2 = 0 + nrpy_bz*(int)blockDim.z + (int)threadIdx.z;

@@ -63,17 +63,28 @@ __device__ __forceinline__ double nrpy_vjp_select(const bool inside, const doubl
 // (BX, BY, BZ) tiling the (n0, n1, n2) index box. The hardware hands block b
 // to XCD b % 8, so consecutive blocks land on different L2 caches; the remap
 // below gives each XCD a contiguous range of tiles, so stencil neighbours in i1 and i2 are
-// mostly resident in the same XCD's L2. Within the range the tiles go along i0, then i1
-// through a slab of NRPY_SLAB tiles, then i2, then to the next slab: the planes that an i2
-// stencil reads again are a few slab rows old. With whole planes in between (i1 to its end before
-// i2) a plane's worth of every array passes through the 4 MB L2 first. MI355X, whole planes ->
-// slabs of 8 (4, 16): scalar wave 256^3 substep 320 -> 306 us (317, 313), Maxwell 192^3 582 -> 573
-// (573, 578), BSSN 192^3 group and Ricci kernels 5235 -> 4997 us (5082, 5033).
+// mostly resident in the same XCD's L2. Within the range the tiles go along i0, i1, i2; where the
+// planes of the state are large, along i0, then i1 through a slab of NRPY_SLAB tiles, then i2, then
+// to the next slab: the planes that an i2 stencil reads again are a few slab rows old. With whole
+// planes in between a plane's worth of every array passes through the 4 MB L2 first. MI355X,
+// whole planes -> slabs of 8 (4, 16): scalar wave 256^3 substep 320 -> 306 us (317, 313), Maxwell
+// 192^3 582 -> 573 (573, 578), BSSN 192^3 group and Ricci kernels 5235 -> 4997 us (5082, 5033).
+// Where they are not large the slabs' divisions cost more than they bring. One step, whole planes,
+// slabs: scalar wave 64^3 32.4, 33.8 us, 144^3 (330 KB a plane of the state) 176, 180, 176^3 (500 KB) 412,
+// 400, 224^3 925, 882; Maxwell 80^3 (410 KB) 166, 167, 96^3 (590 KB) 255, 246, 128^3 708, 677; BSSN 48^3 (440
+// KB) 432, 439, 64^3 (790 KB) 699, 702, 96^3 2712, 2745, 150^3 (4.3 MB) 10914, 10495; Maxwell cylindrical
+// 80x32x80 (160 KB), right-hand side, 16.0, 17.2. NRPY_SLAB_MIN_PLANE, the points of a plane up to which
+// they are whole, is the bundle's 500 KB; every plane in a bundle without stencils along i2
+// (spherical BSSN 192x128x32 right-hand side 277, 284 us) and in kernels that read no neighbours
+// (det(gammabar) enforcement at 64^3 27.3, 27.9 us).
 #define NRPY_NUM_XCD 8
 #define NRPY_SLAB 8
 #define NRPY_BLOCK_COORDS(n0, n1, n2) NRPY_BLOCK_COORDS_OF((int)gridDim.x, n0, n1, n2)
+#define NRPY_BLOCK_COORDS_POINTWISE(n0, n1, n2) NRPY_BLOCK_COORDS_AS((int)gridDim.x, true, n0, n1, n2)
 // the same for the first nblocks blocks of a launch
 #define NRPY_BLOCK_COORDS_OF(nblocks, n0, n1, n2)                                              \
+  NRPY_BLOCK_COORDS_AS(nblocks, (n0) * (n1) <= NRPY_SLAB_MIN_PLANE, n0, n1, n2)
+#define NRPY_BLOCK_COORDS_AS(nblocks, whole, n0, n1, n2)                                       \
   int nrpy_bx, nrpy_by, nrpy_bz;                                                               \
   {                                                                                            \
     const int nbx_ = ((n0) + (int)blockDim.x - 1) / (int)blockDim.x;                           \
@@ -83,12 +94,18 @@ __device__ __forceinline__ double nrpy_vjp_select(const bool inside, const doubl
     const int q_ = nb_ / NRPY_NUM_XCD, r_ = nb_ % NRPY_NUM_XCD;                                \
     const int x_ = b_ % NRPY_NUM_XCD, l_ = b_ / NRPY_NUM_XCD;                                  \
     const int t_ = (x_ < r_) ? x_ * (q_ + 1) + l_ : r_ * (q_ + 1) + (x_ - r_) * q_ + l_;      \
-    const int nbz_ = ((n2) + (int)blockDim.z - 1) / (int)blockDim.z;                           \
-    const int per_ = nbx_ * NRPY_SLAB * nbz_, slab_ = min(t_ / per_, nby_ / NRPY_SLAB);        \
-    const int h_ = min(NRPY_SLAB, nby_ - slab_ * NRPY_SLAB), u_ = t_ - slab_ * per_;           \
-    nrpy_bx = u_ % nbx_;                                                                       \
-    nrpy_by = slab_ * NRPY_SLAB + (u_ / nbx_) % h_;                                            \
-    nrpy_bz = u_ / (nbx_ * h_);                                                                \
+    if (whole) {                                                                               \
+      nrpy_bx = t_ % nbx_;                                                                     \
+      nrpy_by = (t_ / nbx_) % nby_;                                                            \
+      nrpy_bz = t_ / (nbx_ * nby_);                                                            \
+    } else {                                                                                   \
+      const int nbz_ = ((n2) + (int)blockDim.z - 1) / (int)blockDim.z;                         \
+      const int per_ = nbx_ * NRPY_SLAB * nbz_, slab_ = min(t_ / per_, nby_ / NRPY_SLAB);      \
+      const int h_ = min(NRPY_SLAB, nby_ - slab_ * NRPY_SLAB), u_ = t_ - slab_ * per_;         \
+      nrpy_bx = u_ % nbx_;                                                                     \
+      nrpy_by = slab_ * NRPY_SLAB + (u_ / nbx_) % h_;                                          \
+      nrpy_bz = u_ / (nbx_ * h_);                                                              \
+    }                                                                                          \
   }
 
 // x-neighbours of a stencil by cross-lane moves (DPP). A row is TX lanes holding

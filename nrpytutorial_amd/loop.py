@@ -162,6 +162,10 @@ def rfm_reads(body):
     return out
 
 
+# a read at another point: of a gridfunction, or of a vector-Jacobian product's slot
+_NEIGHBOUR = re.compile(r"\bi[012]\s*[+-]\s*\d|\bVJP_\w+_AT\(\w+, [^)]*[1-9]")
+
+
 def simple_loop(options, interior, batched=False):
     """Kernel body: lane -> gridpoint mapping, bounds check, coordinate/table reads, ``interior``.
 
@@ -180,7 +184,8 @@ def simple_loop(options, interior, batched=False):
     if batched:
         s = "NRPY_BATCH_TILE(%s, %s, %s);\n" % (at(n, 0), at(n, 1), at(n, 2))
     else:
-        s = "NRPY_BLOCK_COORDS(%s, %s, %s);\n" % (at(n, 0), at(n, 1), at(n, 2))
+        s = "NRPY_BLOCK_COORDS%s(%s, %s, %s);\n" % ("" if _NEIGHBOUR.search(interior) else "_POINTWISE",
+                                                   at(n, 0), at(n, 1), at(n, 2))
     for d, t in ((0, "x"), (1, "y"), (2, "z")):
         s += "const int i%d = %s + nrpy_b%s*(int)blockDim.%s + (int)threadIdx.%s;\n" % (d, at(lo, d), t, t, t)
     if o["range"] == "interior":
