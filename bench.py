@@ -20,8 +20,10 @@ python bench.py [--gpus 1] [--steps K] [--warmup W] [--n 192] [--no-cpu]
 """
 import argparse
 import ctypes
+import hashlib
 import json
 import os
+import re
 import subprocess
 import sys
 import time
@@ -122,18 +124,33 @@ def cpu_baseline(n=192, min_seconds=10.0, max_steps=8):
                       % (n, res["steps"], res["seconds"], cores, ",".join(map(str, cpus)), cpu_model())}
 
 
+def kernel_text_hash(kernel, csrc=None):
+    """Hash of a Cartesian BSSN kernel's generated text and of the order of its tiles: counters
+    collected for it hold as long as neither changes."""
+    csrc = csrc or os.path.join(ROOT, "nrpytutorial_amd", "csrc")
+    with open(os.path.join(csrc, "generated", "bssn_cartesian.hip")) as f:
+        src = f.read()
+    with open(os.path.join(csrc, "nrpy_runtime_pre.h")) as f:
+        pre = f.read()
+    m = re.search(r"__global__ [^\n]*\b%s__gpu\(" % kernel, src)
+    text = src[m.start():src.index("\n}\n", m.start())]
+    for where, name in ((src, "NRPY_SLAB_MIN_PLANE"), (pre, "NRPY_SLAB"), (pre, "NRPY_BLOCK_COORDS_AS")):
+        text += re.search(r"^#define %s\b.*?(?<!\\)\n" % name, where, re.M | re.S).group(0)
+    return hashlib.sha1(text.encode()).hexdigest()
+
+
 def measured_traffic(kernel, n, outputs):
     """HBM bytes per launch of ``kernel`` at n^3 from the committed rocprofv3 counter
     summary (FETCH_SIZE + WRITE_SIZE, scaled by the plain-copy calibration), or None when
-    there is none for this kernel and output group."""
+    there is none for this kernel, its present text and output group."""
     path = os.path.join(ROOT, "profiles", "%s_bssn%d_traffic.json" % (kernel, n))
     try:
         with open(path) as f:
             d = json.load(f)
-        if d.get("outputs") != list(outputs):
+        if d.get("outputs") != list(outputs) or d.get("kernel_text_sha1") != kernel_text_hash(kernel):
             return None
         return d["hbm_bytes_per_launch"]
-    except (OSError, KeyError, ValueError):
+    except (OSError, KeyError, ValueError, AttributeError):
         return None
 
 
