@@ -1,9 +1,10 @@
 """The path bench.py times, against the oracle: RK4 steps of the Cartesian BSSN bundle
 replayed from its captured hipGraph (MoL_graph_create / MoL_graph_launch).
 
-One step is four substeps of Ricci_eval_g0/g1 -> the fused RHS + RK4 update kernels
+One step is four substeps of Ricci_eval (one kernel) -> the fused RHS + RK4 update kernels
 rhs_eval_rk4_substep_g{0,1,2}<S> at S = 0..3 (LDS-staged stencils on 64x1x4 and
-16x4x4 tiles) -> the composed one-launch ghost fill -> det(gammabar) enforcement.
+16x4x4 tiles) -> the one-launch ghost fill (after substeps 0 to 2 the ghosts that stencils read,
+after the last all of them) -> det(gammabar) enforcement.
 The oracle runs the reference's step (MoLtimestepping/C_Code_Generation.py:266-329):
 Ricci, RHS, RK4 update loop, the layer-by-layer ghost fill, det(gammabar).
 
